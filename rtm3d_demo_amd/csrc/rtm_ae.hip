@@ -24,7 +24,11 @@ namespace rtmhip {
 namespace {
 
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
+// accesses to the caller's brick and code arrays (any 2-byte alignment)
+typedef half8_t half8_any __attribute__((aligned(2)));
+typedef half4_t half4_any __attribute__((aligned(2)));
 
 constexpr int kGemmThreads = 256;  // 4 waves; 64 x 64 tile of C, 32 x 32 per wave
 constexpr int kBrick = 32768;
@@ -203,97 +207,281 @@ __global__ void __launch_bounds__(256)
     }
 }
 
-__global__ void __launch_bounds__(256)
-    k_f32_to_f16(const float *__restrict__ a, _Float16 *__restrict__ b, long long n)
-{
-    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n;
-         i += (long long)gridDim.x * 256)
-        b[i] = (_Float16)a[i];
-}
-
-__global__ void __launch_bounds__(256)
-    k_f16_to_f32(const _Float16 *__restrict__ a, float *__restrict__ b, long long n)
-{
-    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n;
-         i += (long long)gridDim.x * 256)
-        b[i] = (float)a[i];
-}
-
-// Cell of element e of a brick (AE order).
-__device__ __forceinline__ void brick_cell(int e, int &x, int &y, int &z)
-{
-    const int l = e & 7, mi = (e >> 3) & 63, ai = e >> 9;
-    x = 8 * (ai >> 4) + 2 * (mi >> 4) + (l >> 2);
-    y = 8 * ((ai >> 2) & 3) + 2 * ((mi >> 2) & 3) + ((l >> 1) & 1);
-    z = 8 * (ai & 3) + 2 * (mi & 3) + (l & 1);
-}
-
 // One block per brick: scale = max |v| over the brick's in-grid cells, then
 // the FP16 values v * (1 / scale) (zero outside the grid, and the whole
 // brick zero with scale 0 when max |v| is zero or subnormal).
-__global__ void __launch_bounds__(256)
+//
+// Bound by memory (4 B read and 2 B written per cell).  A lane owns patches
+// of 2 x 2 x 2 cells, the 16 lanes (az, mz) of a row covering its 32 z: a
+// load instruction reads 4 whole 128-byte rows, a store 4 runs of 256 bytes
+// of the brick, and the field is read once -- the cells wait in registers
+// for the brick's scale.  VEC: the z pairs are 8-byte aligned and whole.  Salt snapshot
+// (592 x 592 x 256, 2888 bricks): 0.176 ms, 3.1 TB/s (0.374 ms in brick order,
+// two reads of the field).
+constexpr int kCutThreads = 512;
+
+// Block h of n as the position of its work in memory order: XCD h % 8 takes a
+// contiguous run, so the 128-byte lines that two z neighbours share (the
+// region starts at z = blen, in general inside a line) stay in one L2.
+__device__ __forceinline__ unsigned xcd_run(unsigned h, unsigned n)
+{
+    const unsigned q = n >> 3, r = n & 7, k = h & 7;
+    return k * q + min(k, r) + (h >> 3);
+}
+
+template <bool VEC>
+__global__ void __launch_bounds__(kCutThreads)
     k_bricks(const float *__restrict__ F, Grid g, AeRegion r, _Float16 *__restrict__ out,
              float *__restrict__ scales)
 {
-    __shared__ float red[256];
-    const int b = blockIdx.x;
+    constexpr int NW = kCutThreads / 64, NP = 64 / NW;  // waves, patches per lane
+    __shared__ float red[NW];
+    const int b = (int)xcd_run(blockIdx.x, gridDim.x);
     const int bz = b % r.nbz, by = (b / r.nbz) % r.nby, bx = b / (r.nbz * r.nby);
-    const int gx0 = r.x0 + 32 * bx, gy0 = r.y0 + 32 * by, gz0 = r.z0 + 32 * bz;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int mz = lane & 3, my = (lane >> 2) & 3, az = lane >> 4;
+    const int z0 = r.z0 + 32 * bz + 8 * az + 2 * mz;
+    float v[NP][2][2][2];
+#pragma unroll
+    for (int k = 0; k < NP; ++k) {
+        const int p = k * NW + wv;  // (ax, mx, ay) of this patch
+        const int x0 = r.x0 + 32 * bx + 2 * (p >> 2);
+        const int y0 = r.y0 + 32 * by + 8 * (p & 3) + 2 * my;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                // every lane loads (at a clamped place) and selects after: a
+                // branch around the load would wait for it
+                const int x = min(x0 + i, r.x1 - 1), y = min(y0 + j, r.y1 - 1);
+                const float *f = F + (long long)x * g.sx + (long long)y * g.sy;
+                if (VEC) {
+                    const float2 u =
+                        *reinterpret_cast<const float2 *>(f + min(z0, r.z1 - 2));
+                    v[k][i][j][0] = u.x;
+                    v[k][i][j][1] = u.y;
+                } else {
+                    v[k][i][j][0] = f[min(z0, r.z1 - 1)];
+                    v[k][i][j][1] = f[min(z0 + 1, r.z1 - 1)];
+                }
+            }
+    }
+#pragma unroll
+    for (int k = 0; k < NP; ++k) {
+        const int p = k * NW + wv;
+        const int x0 = r.x0 + 32 * bx + 2 * (p >> 2);
+        const int y0 = r.y0 + 32 * by + 8 * (p & 3) + 2 * my;
+#pragma unroll
+        for (int l = 0; l < 8; ++l)
+            if (x0 + (l >> 2) >= r.x1 || y0 + ((l >> 1) & 1) >= r.y1 || z0 + (l & 1) >= r.z1)
+                v[k][l >> 2][(l >> 1) & 1][l & 1] = 0.f;
+    }
     float mx = 0.f;
-    for (int e = threadIdx.x; e < kBrick; e += 256) {
-        int x, y, z;
-        brick_cell(e, x, y, z);
-        x += gx0;
-        y += gy0;
-        z += gz0;
-        if (x < r.x1 && y < r.y1 && z < r.z1)
-            mx = fmaxf(mx, fabsf(F[(long long)x * g.sx + (long long)y * g.sy + z]));
-    }
-    red[threadIdx.x] = mx;
+#pragma unroll
+    for (int k = 0; k < NP; ++k)
+#pragma unroll
+        for (int l = 0; l < 8; ++l) mx = fmaxf(mx, fabsf(v[k][l >> 2][(l >> 1) & 1][l & 1]));
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) mx = fmaxf(mx, __shfl_xor(mx, d, 64));
+    if (lane == 0) red[wv] = mx;
     __syncthreads();
-    for (int h = 128; h > 0; h >>= 1) {
-        if ((int)threadIdx.x < h) red[threadIdx.x] = fmaxf(red[threadIdx.x], red[threadIdx.x + h]);
-        __syncthreads();
-    }
+#pragma unroll
+    for (int k = 0; k < NW; ++k) mx = fmaxf(mx, red[k]);
     // a brick whose largest magnitude is below the smallest normal float
     // (1/s would overflow) is stored as zero
-    const float s = red[0] >= 1.17549435e-38f ? red[0] : 0.f;
+    const float s = mx >= 1.17549435e-38f ? mx : 0.f;
     if (threadIdx.x == 0) scales[b] = s;
     const float inv = s > 0.f ? 1.0f / s : 0.f;
-    _Float16 *o = out + (long long)b * kBrick;
-    for (int e = threadIdx.x; e < kBrick; e += 256) {
-        int x, y, z;
-        brick_cell(e, x, y, z);
-        x += gx0;
-        y += gy0;
-        z += gz0;
-        float v = 0.f;  // +0 outside the grid and in a zero brick
-        if (s > 0.f && x < r.x1 && y < r.y1 && z < r.z1)
-            v = F[(long long)x * g.sx + (long long)y * g.sy + z] * inv;
-        o[e] = wst<_Float16>(v);  // the FP32 product rounded, then narrowed
+    _Float16 *o = out + (long long)b * kBrick + az * 512 + my * 32 + mz * 8;
+#pragma unroll
+    for (int k = 0; k < NP; ++k) {
+        const int p = k * NW + wv;
+        const int a = (p >> 4) * 16 + (p & 3) * 4, m = (p >> 2) & 3;
+        half8_t h;
+#pragma unroll
+        for (int l = 0; l < 8; ++l) {
+            const float c = v[k][l >> 2][(l >> 1) & 1][l & 1];
+            // the FP32 product rounded, then narrowed; +0 in a zero brick
+            h[l] = wst<_Float16>(s > 0.f ? c * inv : 0.f);
+        }
+        *reinterpret_cast<half8_any *>(o + a * 512 + m * 128) = h;
     }
 }
 
-// The inverse: F(cell) = Y[brick][e] * scale for every in-grid cell of the
-// region (Y in AE order, FP32).
-__global__ void __launch_bounds__(256)
-    k_unbricks(const float *__restrict__ Y, const float *__restrict__ scales, Grid g, AeRegion r,
-               float *__restrict__ F, int b0, int nb)
+// Fused inference.  A chunk is 16 consecutive rows a of the middle layers (a
+// quarter of a brick: one ax, all ay and az), handled by one wave with
+// nothing shared between waves but the weights.  Both GEMMs of a direction
+// run transposed (weights as the A operand, rows a as the columns of B), so
+// the first product's result -- lane j + 16 g holds rows 4 g + v of column j
+// of a 16 x 16 tile -- is the second product's B operand as it stands: the
+// second product's weights take the k order {4 g + v, 16 + 4 g + v} instead of the
+// natural one, and no value crosses lanes.  The 8 x 8 layers take four
+// patches at a time as one 32 x 32 block-diagonal product (K = 32 filled).
+// Rounding is the separate layers': FP16 operands, FP32 sums, bias and tanh
+// in FP32, FP16 again for the next layer.
+//
+// Bound by the bricks' bytes (encode: 189 MB read) and the field's (decode: 357
+// MB written) with tanhf's instructions close behind; a shorter rational tanh
+// was no faster (encode 0.076, decode 0.137 ms).  Salt snapshot, 2888 bricks:
+// encode 0.083 ms, decode 0.109 ms; as separate GEMM launches with FP32
+// intermediates in memory and brick order on the field's side 1.3 and 1.8 ms.
+constexpr int kAeThreads = 512;
+constexpr int kAeFrag = 16 * 2 * 64 * 8;  // the 512 x 32 weights as MFMA fragments
+constexpr long long kOffW1 = 0, kOffB1 = 64, kOffW2 = 72, kOffB2 = kOffW2 + 512 * 32,
+                    kOffW3 = kOffB2 + 32, kOffB3 = kOffW3 + 32 * 512, kOffW4 = kOffB3 + 512,
+                    kOffB4 = kOffW4 + 64;
+
+// Lane and slot of element k (0..31) in the order {4 g + v, 16 + 4 g + v}.
+__device__ __forceinline__ int frag_pos(int i, int k)
 {
-    const long long total = (long long)nb * kBrick;
-    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < total;
-         i += (long long)gridDim.x * 256) {
-        const int bl = (int)(i / kBrick), e = (int)(i % kBrick);
-        const int b = b0 + bl;
-        const int bz = b % r.nbz, by = (b / r.nbz) % r.nby, bx = b / (r.nbz * r.nby);
-        int x, y, z;
-        brick_cell(e, x, y, z);
-        x += r.x0 + 32 * bx;
-        y += r.y0 + 32 * by;
-        z += r.z0 + 32 * bz;
-        if (x < r.x1 && y < r.y1 && z < r.z1)
-            F[(long long)x * g.sx + (long long)y * g.sy + z] = Y[i] * scales[b];
+    return (i + 16 * ((k >> 2) & 3)) * 8 + (k & 3) + 4 * (k >> 4);
+}
+
+__global__ void __launch_bounds__(kAeThreads)
+    k_ae_encode(const _Float16 *__restrict__ X, const float *__restrict__ w, long long chunks,
+                _Float16 *__restrict__ codes)
+{
+    __shared__ __align__(16) _Float16 w2[kAeFrag];  // [q][t][lane][slot]
+    const int tid = threadIdx.x, lane = tid & 63, j = lane & 15, g = lane >> 4;
+    for (int e = tid; e < 512 * 32; e += kAeThreads) {
+        const int k = e >> 5, n = e & 31;
+        w2[((k >> 5) * 2 + (n >> 4)) * 512 + frag_pos(n & 15, k & 31)] =
+            (_Float16)w[kOffW2 + e];
     }
+    half8_t w1[2];  // row o = 16 t + j: patch o / 8, channel o % 8; k = 8 g + s: patch g
+    float b1[4], b2[2][4];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const int o = 16 * t + j;
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+            w1[t][s] = (o >> 3) == g ? (_Float16)w[kOffW1 + s * 8 + (o & 7)] : (_Float16)0.f;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) b2[t][v] = w[kOffB2 + 16 * t + 4 * g + v];
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) b1[v] = w[kOffB1 + ((4 * g + v) & 7)];
+    __syncthreads();
+    const float4_t zero = {0.f, 0.f, 0.f, 0.f};
+    const long long c = (long long)xcd_run(blockIdx.x, gridDim.x) * (kAeThreads / 64) + (tid >> 6);
+    if (c >= chunks) return;
+    {
+        const _Float16 *x = X + (c * 16 + j) * 512 + g * 8;
+        float4_t acc[2] = {zero, zero};
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            const half8_t xb = *reinterpret_cast<const half8_any *>(x + q * 32);
+            half8_t h;
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const float4_t d = __builtin_amdgcn_mfma_f32_16x16x32_f16(w1[t], xb, zero, 0, 0, 0);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) h[4 * t + v] = wst<_Float16>(tanhf(d[v] + b1[v]));
+            }
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+                acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                    *reinterpret_cast<const half8_t *>(&w2[((q * 2 + t) * 64 + lane) * 8]), h,
+                    acc[t], 0, 0, 0);
+        }
+        _Float16 *z = codes + (c * 16 + j) * 32 + 4 * g;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            half4_t o;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) o[v] = wst<_Float16>(acc[t][v] + b2[t][v]);
+            *reinterpret_cast<half4_any *>(z + 16 * t) = o;
+        }
+    }
+}
+
+// Codes -> the region's cells of F (value times its brick's scale).  The
+// last layer's 32 outputs of four patches (2 x 2 x 8 cells) are assigned to
+// the rows of its two tiles so that lane (j, g) holds the run z = 4 h .. 4 h
+// + 3 with (lx, h) = (g / 2, g % 2), ly = t: one 16-byte store per tile
+// (VEC: the runs are 16-byte aligned), (az, h) filling 128-byte rows.
+template <bool VEC>
+__global__ void __launch_bounds__(kAeThreads)
+    k_ae_decode(const _Float16 *__restrict__ codes, const float *__restrict__ w, long long chunks,
+                const float *__restrict__ scales, Grid gr, AeRegion r, float *__restrict__ F)
+{
+    __shared__ __align__(16) _Float16 w3[kAeFrag];  // [q][t][lane][slot]
+    __shared__ __align__(16) float b3[512];
+    const int tid = threadIdx.x, lane = tid & 63, j = lane & 15, g = lane >> 4;
+    for (int e = tid; e < 32 * 512; e += kAeThreads) {
+        const int k = e >> 9, n = e & 511;
+        w3[((n >> 4) * 64 + (n & 15) + 16 * (k >> 3)) * 8 + (k & 7)] = (_Float16)w[kOffW3 + e];
+    }
+    for (int e = tid; e < 512; e += kAeThreads) b3[e] = w[kOffB3 + e];
+    half8_t w4[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        // row j of tile t: lx = j / 8, z = j % 8 (patch z / 2), ly = t
+        const int z = j & 7, l = (j >> 3) * 4 + t * 2 + (z & 1);
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            const int k = (s & 3) + 4 * g + 16 * (s >> 2);  // patch k / 8, channel k % 8
+            w4[t][s] = (k >> 3) == (z >> 1) ? (_Float16)w[kOffW4 + (k & 7) * 8 + l]
+                                            : (_Float16)0.f;
+        }
+    }
+    float b4[2][2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int v = 0; v < 2; ++v) b4[t][v] = w[kOffB4 + (g >> 1) * 4 + t * 2 + v];
+    __syncthreads();
+    const float4_t zero = {0.f, 0.f, 0.f, 0.f};
+    const long long c = (long long)xcd_run(blockIdx.x, gridDim.x) * (kAeThreads / 64) + (tid >> 6);
+    if (c >= chunks) return;
+    {
+        const half8_t zb = *reinterpret_cast<const half8_any *>(codes + (c * 16 + j) * 32 + g * 8);
+        const int b = (int)(c >> 2), ax = (int)(c & 3);
+        const float scale = scales[b];
+        const int bz = b % r.nbz, by = (b / r.nbz) % r.nby, bx = b / (r.nbz * r.nby);
+        const int x0 = r.x0 + 32 * bx + 8 * ax + (g >> 1);
+        const int y0 = r.y0 + 32 * by + 8 * (j >> 2);
+        const int z0 = r.z0 + 32 * bz + 8 * (j & 3) + 4 * (g & 1);
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            half8_t h;
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const float4_t d = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                    *reinterpret_cast<const half8_t *>(&w3[((q * 2 + t) * 64 + lane) * 8]), zb,
+                    zero, 0, 0, 0);
+                const float4_t bb =
+                    *reinterpret_cast<const float4_t *>(&b3[q * 32 + 16 * t + 4 * g]);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) h[4 * t + v] = wst<_Float16>(tanhf(d[v] + bb[v]));
+            }
+            const int x = x0 + 2 * (q >> 2), y = y0 + 2 * (q & 3);
+            float *p = F + (long long)x * gr.sx + (long long)y * gr.sy + z0;
+#pragma unroll
+            for (int t = 0; t < 2; ++t, p += gr.sy) {
+                const float4_t d = __builtin_amdgcn_mfma_f32_16x16x32_f16(w4[t], h, zero, 0, 0, 0);
+                float4_t o;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) o[v] = (d[v] + b4[t][v & 1]) * scale;
+                if (x < r.x1 && y + t < r.y1) {
+                    if (VEC && z0 + 4 <= r.z1) {
+                        *reinterpret_cast<float4_t *>(p) = o;
+                    } else {
+#pragma unroll
+                        for (int v = 0; v < 4; ++v)
+                            if (z0 + v < r.z1) p[v] = o[v];
+                    }
+                }
+            }
+        }
+    }
+}
+
+// The region's z runs of n cells (n a power of two) are aligned in F.
+inline bool runs_aligned(const float *F, const Grid &g, const AeRegion &r, int n)
+{
+    return ((uintptr_t)F & (4 * n - 1)) == 0 && (g.sx & (n - 1)) == 0 && (g.sy & (n - 1)) == 0 &&
+           (r.z0 & (n - 1)) == 0;
 }
 
 inline unsigned grid_for(long long n)
@@ -370,37 +558,42 @@ hipError_t launch_gather_bricks(const void *src, const int *idx, void *dst, int 
     return hipGetLastError();
 }
 
-hipError_t launch_f32_to_f16(const float *a, void *b, long long n, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_f32_to_f16, dim3(grid_for(n)), dim3(256), 0, s, a,
-                       static_cast<_Float16 *>(b), n);
-    return hipGetLastError();
-}
-
-hipError_t launch_f16_to_f32(const void *a, float *b, long long n, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_f16_to_f32, dim3(grid_for(n)), dim3(256), 0, s,
-                       static_cast<const _Float16 *>(a), b, n);
-    return hipGetLastError();
-}
-
 hipError_t launch_bricks(const float *F, const Grid &g, const AeRegion &r, void *out,
                          float *scales, hipStream_t s)
 {
     const long long nb = (long long)r.nbx * r.nby * r.nbz;
     if (nb <= 0) return hipSuccess;
     if (nb > 0x7fffffffLL) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_bricks, dim3((unsigned)nb), dim3(256), 0, s, F, g, r,
+    const bool pairs = runs_aligned(F, g, r, 2) && (r.z1 & 1) == 0;
+    hipLaunchKernelGGL(pairs ? k_bricks<true> : k_bricks<false>, dim3((unsigned)nb), dim3(kCutThreads), 0, s, F, g, r,
                        static_cast<_Float16 *>(out), scales);
     return hipGetLastError();
 }
 
-hipError_t launch_unbricks(const float *Y, const float *scales, const Grid &g, const AeRegion &r,
-                           float *F, int b0, int nb, hipStream_t s)
+// One chunk per wave, four chunks per brick.
+inline unsigned ae_blocks(long long n)
 {
-    if (nb <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_unbricks, dim3(grid_for((long long)nb * kBrick)), dim3(256), 0, s, Y,
-                       scales, g, r, F, b0, nb);
+    constexpr int waves = kAeThreads / 64;
+    return (unsigned)((4 * n + waves - 1) / waves);
+}
+
+hipError_t launch_ae_encode(const void *bricks, const float *w, long long n, void *codes,
+                            hipStream_t s)
+{
+    if (n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_ae_encode, dim3(ae_blocks(n)), dim3(kAeThreads), 0, s,
+                       static_cast<const _Float16 *>(bricks), w, 4 * n,
+                       static_cast<_Float16 *>(codes));
+    return hipGetLastError();
+}
+
+hipError_t launch_ae_decode(const void *codes, const float *w, long long n, const float *scales,
+                            const Grid &g, const AeRegion &r, float *F, hipStream_t s)
+{
+    if (n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(runs_aligned(F, g, r, 4) ? k_ae_decode<true> : k_ae_decode<false>,
+                       dim3(ae_blocks(n)), dim3(kAeThreads), 0, s,
+                       static_cast<const _Float16 *>(codes), w, 4 * n, scales, g, r, F);
     return hipGetLastError();
 }
 

@@ -2190,38 +2190,6 @@ int ae_check_region(int nxe, int nye, int nze, int x0, int y0, int z0, int x1, i
     return RTMHIP_OK;
 }
 
-// n FP16 bricks -> n x 2048 FP16 codes, in passes of at most maxb bricks.
-hipError_t ae_encode(const rtmhip_ae *a, const void *bricks, int n, void *codes)
-{
-    hipError_t e = hipSuccess;
-    for (int b0 = 0; b0 < n && e == hipSuccess; b0 += a->maxb) {
-        const int nb = std::min(a->maxb, n - b0);
-        const char *in = static_cast<const char *>(bricks) + (size_t)b0 * kBrickCells * 2;
-        e = ae_layer(a, 0, in, 1, a->h1, nb);
-        if (e == hipSuccess) e = ae_layer(a, 1, a->h1, 0, a->z, nb);
-        if (e == hipSuccess)
-            e = launch_f32_to_f16(a->z, static_cast<char *>(codes) + (size_t)b0 * kCodes * 2,
-                                  kCodes * nb, g_state.stream);
-    }
-    return e;
-}
-
-// Codes + scales of the n bricks of region r -> the region's cells of field.
-hipError_t ae_decode(const rtmhip_ae *a, const void *codes, const float *scales, int n,
-                     const Grid &g, const AeRegion &r, float *field)
-{
-    hipError_t e = hipSuccess;
-    for (int b0 = 0; b0 < n && e == hipSuccess; b0 += a->maxb) {
-        const int nb = std::min(a->maxb, n - b0);
-        e = launch_f16_to_f32(static_cast<const char *>(codes) + (size_t)b0 * kCodes * 2, a->z,
-                              kCodes * nb, g_state.stream);
-        if (e == hipSuccess) e = ae_layer(a, 2, a->z, 0, a->h3, nb);
-        if (e == hipSuccess) e = ae_layer(a, 3, a->h3, 0, a->y, nb);
-        if (e == hipSuccess) e = launch_unbricks(a->y, scales, g, r, field, b0, nb, g_state.stream);
-    }
-    return e;
-}
-
 // The imaging region of a shot's snapshots (all x, y; z in [z0, z0 + lz))
 // as bricks: on the extended grid (z0 = blen) or on a compact
 // [nxe][nye][nze-2*blen] field (z0 = 0).
@@ -2446,7 +2414,7 @@ int rtmhip_ae_encode(rtmhip_ae *a, const void *bricks, int n, void *codes)
 {
     NEED_INIT();
     if (!a || !bricks || !codes) return fail(RTMHIP_ERR_INVALID, "NULL pointer");
-    HIPCHK(ae_encode(a, bricks, n, codes), "encode");
+    HIPCHK(launch_ae_encode(bricks, a->w, n, codes, g_state.stream), "encode");
     return RTMHIP_OK;
 }
 
@@ -2462,7 +2430,7 @@ int rtmhip_ae_decode(rtmhip_ae *a, const void *codes, const float *scales, int n
     if ((long long)n != (long long)r.nbx * r.nby * r.nbz)
         return fail(RTMHIP_ERR_INVALID, "%d codes for a region of %d bricks", n,
                     r.nbx * r.nby * r.nbz);
-    HIPCHK(ae_decode(a, codes, scales, n, g, r, field), "decode");
+    HIPCHK(launch_ae_decode(codes, a->w, n, scales, g, r, field, g_state.stream), "decode");
     return RTMHIP_OK;
 }
 
@@ -2506,9 +2474,10 @@ int rtmhip_snap_ae_forward_steps(const rtmhip_shot *shot, const float *V2DT2, co
                                 HIPCHK(launch_bricks(f, c.g, r, work, scales + (size_t)j * nb,
                                                      g_state.stream),
                                        "snapshot bricks");
-                                HIPCHK(ae_encode(ae, work, (int)nb,
-                                                 static_cast<char *>(codes) +
-                                                     (size_t)j * nb * kCodes * 2),
+                                HIPCHK(launch_ae_encode(work, ae->w, nb,
+                                                        static_cast<char *>(codes) +
+                                                            (size_t)j * nb * kCodes * 2,
+                                                        g_state.stream),
                                        "snapshot encode");
                                 return RTMHIP_OK;
                             });
@@ -2537,10 +2506,10 @@ int rtmhip_snap_ae_backward_steps(const rtmhip_shot *shot, const float *V2DT2,
     float *snap = static_cast<float *>(work);
     return snap_backward_run(shot, c, V2DT2, taper, Pr, PPr, k, rcv_chunk, it_hi, nsteps,
                              [&](const float *pr, int j) {
-                                 HIPCHK(ae_decode(ae,
-                                                  static_cast<const char *>(codes) +
-                                                      (size_t)j * nb * kCodes * 2,
-                                                  scales + (size_t)j * nb, (int)nb, cg, r, snap),
+                                 HIPCHK(launch_ae_decode(static_cast<const char *>(codes) +
+                                                             (size_t)j * nb * kCodes * 2,
+                                                         ae->w, nb, scales + (size_t)j * nb, cg,
+                                                         r, snap, g_state.stream),
                                         "snapshot decode");
                                  HIPCHK(launch_snap_image(img, (const float *)snap, pr, c.g,
                                                           shot->blen, (float)k, g_state.stream),

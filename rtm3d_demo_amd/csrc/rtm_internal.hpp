@@ -306,11 +306,13 @@ hipError_t launch_colsum(const float *D, long long rows, int cols, float *db, hi
 hipError_t launch_adam(float *w, const float *g, float *m, float *v, int n, float lr_t, float b1,
                        float b2, float eps, hipStream_t s);
 hipError_t launch_gather_bricks(const void *src, const int *idx, void *dst, int n, hipStream_t s);
-hipError_t launch_f32_to_f16(const float *a, void *b, long long n, hipStream_t s);
-hipError_t launch_f16_to_f32(const void *a, float *b, long long n, hipStream_t s);
 hipError_t launch_bricks(const float *F, const Grid &g, const AeRegion &r, void *out,
                          float *scales, hipStream_t s);
-hipError_t launch_unbricks(const float *Y, const float *scales, const Grid &g, const AeRegion &r,
-                           float *F, int b0, int nb, hipStream_t s);
+// Inference over n bricks in one launch (w: the flat parameters): FP16 bricks
+// -> FP16 codes, and codes + scales -> the region's cells of F.
+hipError_t launch_ae_encode(const void *bricks, const float *w, long long n, void *codes,
+                            hipStream_t s);
+hipError_t launch_ae_decode(const void *codes, const float *w, long long n, const float *scales,
+                            const Grid &g, const AeRegion &r, float *F, hipStream_t s);
 
 }  // namespace rtmhip

@@ -107,6 +107,51 @@ def test_bricks_match_oracle(gpu):
         d.free()
 
 
+@pytest.mark.parametrize("shape,region", [
+    ((64, 64, 64), (0, 0, 0, 64, 64, 64)),    # whole bricks, aligned z runs
+    ((40, 37, 52), (0, 0, 4, 40, 37, 52)),    # aligned runs, ragged bricks
+    ((40, 37, 52), (1, 2, 4, 39, 36, 47)),    # odd end: no whole pairs or runs
+    ((33, 34, 51), (0, 0, 3, 33, 34, 50)),    # odd rows and origin: scalar access
+    ((32, 32, 35), (5, 0, 2, 6, 1, 3)),       # a single cell
+])
+def test_fused_codes_on_ragged_regions(gpu, shape, region):
+    """Cutting, encoding and decoding at the edges of bricks and of the
+    vector accesses.  Bricks and scales are exact.  Codes: the operands'
+    FP16 rounding (2^-11 each) over three products, in quadrature with random
+    signs and doubled for the output's own rounding, stays below 5e-3 of the
+    norm; cells outside the region keep their value."""
+    from rtm3d_demo_amd import ae
+    rng = np.random.default_rng(21)
+    f = _smooth_field(rng, shape)
+    B, S = ao.bricks(f, region)
+    n = B.shape[0]
+    codec = ae.Codec(max_bricks=1, seed=3)
+    p = codec.params().astype(np.float64)
+    dF = gpu.DeviceArray.from_host(f)
+    dB, dS = gpu.DeviceArray((n, ao.BRICK), np.uint16), gpu.DeviceArray((n,))
+    dC = gpu.DeviceArray((n, ao.CODES), np.uint16)
+    ae.cut_bricks(dF, region, dB, dS)
+    assert np.array_equal(dS.download(), S)
+    assert np.array_equal(dB.download(), B.view(np.uint16))
+    codec.encode(dB, n, dC)
+    want = ao.encode(p, B)
+    codes = dC.download().view(np.float16)
+    assert _rel(codes, want) < 5e-3
+    out = np.full(shape, np.float32(7.0))
+    dF.upload(out)
+    codec.decode(dC, dS, n, dF, region)
+    ao.unbricks(ao.decode(p, codes.astype(np.float64)), S, out, region)
+    got = dF.download()
+    x0, y0, z0, x1, y1, z1 = region
+    inside = np.zeros(shape, bool)
+    inside[x0:x1, y0:y1, z0:z1] = True
+    assert np.all(got[~inside] == 7.0)
+    assert _rel(got[inside], out[inside]) < 5e-3
+    for d in (dF, dB, dS, dC):
+        d.free()
+    codec.destroy()
+
+
 def test_gradient_codes_and_decode_match_oracle(gpu):
     from rtm3d_demo_amd import ae
     rng = np.random.default_rng(5)
