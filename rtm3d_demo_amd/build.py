@@ -24,7 +24,8 @@ LIBNAME = os.path.join(LIBDIR, "librtm3d_hip.so")
 DRIVER = os.path.join(BINDIR, "rtm3d")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
-HIP_SOURCES = ["rtm_stencil.hip", "rtm_ops.hip", "rtm_ae.hip", "rtm_dct.hip", "rtm_capi.hip"]
+HIP_SOURCES = ["rtm_stencil.hip", "rtm_slab.hip", "rtm_slab_even.hip", "rtm_slab_odd.hip",
+               "rtm_ops.hip", "rtm_ae.hip", "rtm_dct.hip", "rtm_capi.hip"]
 HIP_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++20", "-fPIC", "-ffp-contract=off",
     "-fno-gpu-flush-denormals-to-zero", "-Xclang", "-target-feature", "-Xclang",
@@ -60,7 +61,9 @@ def build_library(jobs=4, incremental=False):
     is older than the source or a shared header) and links the library."""
     os.makedirs(LIBDIR, exist_ok=True)
     os.makedirs(OBJDIR, exist_ok=True)
-    headers = [os.path.join(CSRC, "rtm_internal.hpp"), os.path.join(REPO, "include", "rtm_hip.h")]
+    headers = [os.path.join(CSRC, h) for h in ("rtm_internal.hpp", "rtm_slab.hpp",
+                                               "rtm_slab_launch.hpp")]
+    headers.append(os.path.join(REPO, "include", "rtm_hip.h"))
     objs = []
     cmds = []
     for src in HIP_SOURCES:

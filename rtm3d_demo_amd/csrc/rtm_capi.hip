@@ -5,6 +5,7 @@
 // and returns.  The time-loop entry points chain the operators of the
 // reference's per-step loops with no host synchronisation in between.
 #include "rtm_internal.hpp"
+#include "rtm_slab_launch.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -170,16 +171,42 @@ const StencilTiling *class_tiling(int cls)
     return g_state.tiling[cls].tz ? &g_state.tiling[cls] : nullptr;
 }
 
+// One step of kernel class cls.  FP32 steps without a requested tile shape run
+// on full-row blocks where those fit (order 8, rows of 129..512 cells, tapers
+// on the output); everything else on the shapes of launch_stencil.
+// slab_fits holds the line between them and its measurements.
+template <typename T>
+hipError_t step_launch(int cls, int radius, const T *P, T *PP, const float *V, const Coefs &cf,
+                       const Grid &g, const ImageFuse *fuse, const TaperFuse *taper)
+{
+    if constexpr (std::is_same<T, float>::value) {
+        if (!class_tiling(cls) && slab_fits(radius, g, fuse, taper))
+            return launch_slab(P, PP, V, cf, g, fuse, taper, g_state.flag, g_state.stream);
+    }
+    return launch_stencil(radius, P, PP, V, cf, g, fuse, taper, g_state.flag, g_state.stream,
+                          class_tiling(cls));
+}
+
+// The receiver step with imaging takes the upper taper on its output (and the
+// loops order their in-place tapers accordingly) where the full-row kernel
+// runs it.
+template <typename T>
+bool image_outu(int wave_format, int radius, const Grid &g, const float *taper, int b)
+{
+    if (!std::is_same<T, float>::value || !g_state.taper_outu[wave_format] || class_tiling(1))
+        return false;
+    const ImageFuse fz{};
+    const TaperFuse tf{taper, b, 1, 3, 0};
+    return b > 0 && slab_fits(radius, g, &fz, &tf);
+}
+
 template <typename T>
 hipError_t stencil(int radius, const T *P, T *PP, const float *V, const Coefs &cf, const Grid &g,
                    const ImageFuse *fuse, const TaperFuse *taper = nullptr)
 {
     // kernel class: 0 plain step, 1 fused receiver step, 2 tapered HBC step
     const int cls = fuse ? 1 : (taper ? 2 : 0);
-    return timed(cls, [&] {
-        return launch_stencil(radius, P, PP, V, cf, g, fuse, taper, g_state.flag,
-                              g_state.stream, class_tiling(cls));
-    });
+    return timed(cls, [&] { return step_launch(cls, radius, P, PP, V, cf, g, fuse, taper); });
 }
 
 
@@ -771,6 +798,10 @@ int backward_loop(const rtmhip_shot *shot, const ShotCtx &c, int hbc, const floa
     // separate in-place receiver tapers before an untapered fused step (not
     // with the dual kernel, which fuses them)
     const bool sep = hbc && fused && !dual && g_state.taper_sep[shot->wave_format];
+    // the receiver field's upper tapers on the step's output, ordered as in
+    // snap_backward_run (receivers and imaged range lie at z >= blen)
+    const bool outr = hbc && fused && !dual && !sep &&
+                      image_outu<T>(shot->wave_format, c.radius, c.g, taper, b);
     for (int it = it_hi; it > it_hi - nsteps; --it) {
         const int lt = it % shot->ntstep;
         const int ul = hbc == 2 ? lt : it;  // history layer, as in forward_loop
@@ -839,8 +870,14 @@ int backward_loop(const rtmhip_shot *shot, const ShotCtx &c, int hbc, const floa
         if (fused) {
             // tapers fused as in the forward loop (finishing taper below), or
             // applied in place first
-            if (sep) HIPCHK(launch_taper_upper2(*Pr, *PPr, taper, c.g, b, s), "taper");
-            const TaperFuse tf{taper, b, it == it_hi ? 1 : 2};
+            const bool first = it == it_hi, last = it == it_hi - nsteps + 1;
+            if (sep || (outr && first && last))
+                HIPCHK(launch_taper_upper2(*Pr, *PPr, taper, c.g, b, s), "taper");
+            else if (outr && (first || last))
+                HIPCHK(launch_taper(first ? *Pr : *PPr, taper, c.g, b, true, s), "taper");
+            const TaperFuse tf = outr ? TaperFuse{taper, b, 1, 3, 0}
+                                      : TaperFuse{taper, b, first ? 1 : 2};
+            const bool tapered = hbc && !sep && !(outr && last);
             ImageFuse fz;
             fz.img = img;
             fz.ps = S;
@@ -853,11 +890,11 @@ int backward_loop(const rtmhip_shot *shot, const ShotCtx &c, int hbc, const floa
             fz.ry0 = c.ry0;
             fz.rdy = std::max(1, shot->rcv.dist_y);
             fz.rny = shot->rcv.count_y;
-            HIPCHK(stencil(c.radius, *Pr, *PPr, V2DT2, c.cf, c.g, &fz,
-                           hbc && !sep ? &tf : nullptr),
+            HIPCHK(stencil(c.radius, *Pr, *PPr, V2DT2, c.cf, c.g, &fz, tapered ? &tf : nullptr),
                    "fused stencil");
-            if (hbc && !sep)
-                HIPCHK(launch_taper_frame(*PPr, taper, c.g, b, c.radius, tf.pp_taps, s),
+            if (tapered)
+                HIPCHK(launch_taper_frame(*PPr, taper, c.g, b, c.radius, outr ? 2 : tf.pp_taps,
+                                          s),
                        "frame taper");
             HIPCHK(launch_receivers_image(*PPr, rcv_chunk, c.g, c.rx0, c.ry0, c.rz,
                                           shot->rcv.dist_x, shot->rcv.dist_y, shot->rcv.count_x,
@@ -876,8 +913,8 @@ int backward_loop(const rtmhip_shot *shot, const ShotCtx &c, int hbc, const floa
         *Pr = *PPr;
         *PPr = t;
     }
-    // pending in-place taper of the older receiver field (fused HBC path)
-    if (hbc && fused && !sep) HIPCHK(launch_taper(*PPr, taper, c.g, b, true, s), "taper");
+    // pending in-place taper of the older receiver field (fused on load)
+    if (hbc && fused && !sep && !outr) HIPCHK(launch_taper(*PPr, taper, c.g, b, true, s), "taper");
     return RTMHIP_OK;
 }
 
@@ -1492,6 +1529,7 @@ struct rtmhip_batch {
     int mode[3] = {0, 0, 0};        // per stencil class: 0 per-shot launches, 6/8 batched
     int graph_steps = 8;            // steps per captured graph (0: no graphs)
     bool fout = false;              // forward steps: upper taper on the output (this call)
+    bool bout = false;              // backward steps: the receiver field's
     std::map<int, hipGraphExec_t> graphs;
     int tiling_gen = 0;             // g_state.tiling_gen when the graphs were captured
 };
@@ -1540,9 +1578,9 @@ int batch_fwd_step(rtmhip_batch *b, int taps, const int *itp, int itoff, int for
         const TaperFuse to{b->taper, b->blen, 1, 3, b->hf};
         for (int i = 0; i < b->n; ++i) {
             const BatchShot &h = b->hs[0][i];
-            HIPCHK(launch_stencil<T>(b->radius, (const T *)h.fs[b->cs], (T *)h.fs[b->cs ^ 1], h.V,
-                                     b->cf, h.g, nullptr, form == 1 ? &to : nullptr,
-                                     g_state.flag, s, class_tiling(form == 1 ? cls : 0)),
+            HIPCHK(step_launch<T>(form == 1 ? cls : 0, b->radius, (const T *)h.fs[b->cs],
+                                  (T *)h.fs[b->cs ^ 1], h.V, b->cf, h.g, nullptr,
+                                  form == 1 ? &to : nullptr),
                    "stencil");
         }
         HIPCHK(launch_tail_fwd<T>(b->ds[0], b->n, b->fwd_blocks, b->cs, b->taper, b->blen,
@@ -1559,9 +1597,8 @@ int batch_fwd_step(rtmhip_batch *b, int taps, const int *itp, int itoff, int for
     } else {
         for (int i = 0; i < b->n; ++i) {
             const BatchShot &h = b->hs[0][i];
-            HIPCHK(launch_stencil<T>(b->radius, (const T *)h.fs[b->cs], (T *)h.fs[b->cs ^ 1], h.V,
-                                     b->cf, h.g, nullptr, &tf, g_state.flag, s,
-                                     class_tiling(cls)),
+            HIPCHK(step_launch<T>(cls, b->radius, (const T *)h.fs[b->cs], (T *)h.fs[b->cs ^ 1],
+                                  h.V, b->cf, h.g, nullptr, &tf),
                    "stencil");
         }
     }
@@ -1571,13 +1608,40 @@ int batch_fwd_step(rtmhip_batch *b, int taps, const int *itp, int itoff, int for
     return RTMHIP_OK;
 }
 
-// One backward step (HBC, it < nt-2) of every shot: source reconstruction,
-// receiver step fused with imaging, then the small operators.
+// The backward steps of a batch store the upper taper of the receiver steps'
+// output (as backward_loop) when every shot's receiver step runs that way.
 template <typename T>
-int batch_bwd_step(rtmhip_batch *b, int taps, const int *itp, int itoff)
+bool batch_bwd_out(const rtmhip_batch *b)
+{
+    if (b->mode[1]) return false;
+    for (int i = 0; i < b->n; ++i)
+        if (!image_outu<T>(b->wave_format, b->radius, b->hs[0][i].g, b->taper, b->blen))
+            return false;
+    return true;
+}
+
+// One backward step (HBC, it < nt-2) of every shot: source reconstruction,
+// receiver step fused with imaging, then the small operators.  form and first
+// as in batch_fwd_step (form 0: the receiver tapers on load, or in place
+// before this call's steps).
+template <typename T>
+int batch_bwd_step(rtmhip_batch *b, int taps, const int *itp, int itoff, int form = 0,
+                   bool first = false)
 {
     hipStream_t s = g_state.stream;
-    const TaperFuse tf{b->taper, b->blen, taps};
+    const TaperFuse tf = form ? TaperFuse{b->taper, b->blen, 1, 3, 0}
+                              : TaperFuse{b->taper, b->blen, taps};
+    if (form) taps = form == 1 ? 2 : 0;
+    if (form == 2 || first) {
+        for (int i = 0; i < b->n && form; ++i) {
+            const BatchShot &h = b->hs[0][i];
+            T *P = (T *)h.fr[b->cr], *PP = (T *)h.fr[b->cr ^ 1];
+            if (first && form == 2)
+                HIPCHK(launch_taper_upper2<T>(P, PP, b->taper, h.g, b->blen, s), "taper");
+            else
+                HIPCHK(launch_taper<T>(first ? P : PP, b->taper, h.g, b->blen, true, s), "taper");
+        }
+    }
     if (b->mode[0]) {
         const int k = batch_tab(b, 0);
         HIPCHK(launch_stencil_batch<T>(b->mode[0], b->ds[k], b->hs[k], b->n, b->nblk[k],
@@ -1586,9 +1650,8 @@ int batch_bwd_step(rtmhip_batch *b, int taps, const int *itp, int itoff)
     } else {
         for (int i = 0; i < b->n; ++i) {
             const BatchShot &h = b->hs[0][i];
-            HIPCHK(launch_stencil<T>(b->radius, (const T *)h.fs[b->cs], (T *)h.fs[b->cs ^ 1], h.V,
-                                     b->cf, h.g, nullptr, nullptr, g_state.flag, s,
-                                     class_tiling(0)),
+            HIPCHK(step_launch<T>(0, b->radius, (const T *)h.fs[b->cs], (T *)h.fs[b->cs ^ 1], h.V,
+                                  b->cf, h.g, nullptr, nullptr),
                    "stencil");
         }
     }
@@ -1612,8 +1675,8 @@ int batch_bwd_step(rtmhip_batch *b, int taps, const int *itp, int itoff)
             fz.ry0 = h.ry0;
             fz.rdy = h.rdy;
             fz.rny = h.rny;
-            HIPCHK(launch_stencil<T>(b->radius, (const T *)h.fr[b->cr], (T *)h.fr[b->cr ^ 1], h.V,
-                                     b->cf, h.g, &fz, &tf, g_state.flag, s, class_tiling(1)),
+            HIPCHK(step_launch<T>(1, b->radius, (const T *)h.fr[b->cr], (T *)h.fr[b->cr ^ 1], h.V,
+                                  b->cf, h.g, &fz, form == 2 ? nullptr : &tf),
                    "stencil");
         }
     }
@@ -1639,7 +1702,8 @@ int batch_graph(rtmhip_batch *b, int dir, hipGraphExec_t *out)
         b->graphs.clear();
         b->tiling_gen = g_state.tiling_gen;
     }
-    const int key = (dir > 0 ? 0 : 4) | (b->cs << 1) | b->cr | (dir > 0 && b->fout ? 8 : 0);
+    const int key = (dir > 0 ? 0 : 4) | (b->cs << 1) | b->cr |
+                    ((dir > 0 ? b->fout : b->bout) ? 8 : 0);
     auto f = b->graphs.find(key);
     if (f != b->graphs.end()) {
         *out = f->second;
@@ -1656,7 +1720,7 @@ int batch_graph(rtmhip_batch *b, int dir, hipGraphExec_t *out)
     int rc = RTMHIP_OK;
     for (int k = 0; k < b->graph_steps && rc == RTMHIP_OK; ++k)
         rc = dir > 0 ? batch_fwd_step<T>(b, 2, b->ctr, k, b->fout ? 1 : 0)
-                     : batch_bwd_step<T>(b, 2, b->ctr, -k);
+                     : batch_bwd_step<T>(b, 2, b->ctr, -k, b->bout ? 1 : 0);
     hipError_t e = rc == RTMHIP_OK ? launch_tick(b->ctr, dir * b->graph_steps, false, s)
                                    : hipSuccess;
     capture_guard(false);
@@ -1691,18 +1755,20 @@ int batch_run(rtmhip_batch *b, int dir, int it0, int nsteps)
     hipStream_t s = g_state.stream;
     // forward steps with the upper taper on the output: the first tapers P
     // in place, the last (never inside a graph) runs the reference's order
+    // (backward: the same for the receiver field's P and PP)
     b->fout = dir > 0 && batch_fwd_out(b);
+    b->bout = dir < 0 && batch_bwd_out<T>(b);
+    const bool out = dir > 0 ? b->fout : b->bout;
     auto step = [&](int taps, int it, int k) {
-        if (dir > 0 && b->fout)
-            return batch_fwd_step<T>(b, taps, nullptr, it, k == nsteps - 1 ? 2 : 1, k == 0);
-        return dir > 0 ? batch_fwd_step<T>(b, taps, nullptr, it)
-                       : batch_bwd_step<T>(b, taps, nullptr, it);
+        const int form = !out ? 0 : (k == nsteps - 1 ? 2 : 1);
+        return dir > 0 ? batch_fwd_step<T>(b, taps, nullptr, it, form, k == 0)
+                       : batch_bwd_step<T>(b, taps, nullptr, it, form, k == 0);
     };
     int rc = step(1, it0, 0);
     if (rc) return rc;
     int done = 1;
     const int G = b->graph_steps;
-    const int keep = b->fout ? 1 : 0;
+    const int keep = out ? 1 : 0;
     if (G > 0 && nsteps - keep - done >= G) {
         hipGraphExec_t exec;
         if ((rc = batch_graph<T>(b, dir, &exec))) return rc;
@@ -1714,7 +1780,7 @@ int batch_run(rtmhip_batch *b, int dir, int it0, int nsteps)
     }
     for (; done < nsteps; ++done)
         if ((rc = step(2, it0 + dir * done, done))) return rc;
-    if (dir > 0 && b->fout) return RTMHIP_OK;
+    if (out) return RTMHIP_OK;
     // the pending in-place taper: P of the source field (forward) or the
     // older receiver field (backward), as the per-shot loops leave them
     for (int i = 0; i < b->n; ++i) {
