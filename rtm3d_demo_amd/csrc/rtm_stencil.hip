@@ -2333,6 +2333,12 @@ bool wave2_fits(const T *P, const T *PP, const float *V, const ImageFuse *fuse, 
     return true;
 }
 
+// One z cell per lane keeps fewer lanes idle: the row ends in the first half
+// of a 128-cell tile.  FP32 plain step, us, 128 x 1 x 4 against 64 x 1 x 8:
+// 192^3 25.3 / 23.6, 300 x 300 x 272 88 / 85, 640 x 300 x 140 118 / 100,
+// 600 x 600 x 260 409 / 364; where both fill alike 592 x 592 x 336 403 / 412.
+inline bool narrow_tiles(int nz) { return ((nz + 63) / 64) & 1; }
+
 template <typename T, int R, int RY, int WPB>
 hipError_t launch_wave2(const T *P, T *PP, const float *V, const Coefs &cf, const Grid &g,
                         const ImageFuse *fuse, const TaperFuse *taper, int *flag, hipStream_t s,
@@ -2357,8 +2363,9 @@ hipError_t launch_wave2(const T *P, T *PP, const float *V, const Coefs &cf, cons
 }
 
 // The step with taper3D applied to its output (TAPER 3, no imaging): two-z
-// 128 x 1 x 4 waves where cell pairs fit (even nz and strides), else one-z
-// 64 x 1 x RY waves, over every z tile.
+// 128 x 1 x 4 waves where cell pairs fit (even nz and strides) and, for FP32,
+// fill their tiles (narrow_tiles), else one-z 64 x 1 x RY waves, over every z
+// tile.
 template <typename T, int R, int RY, int WPB>
 hipError_t launch_wave_out(const T *P, T *PP, const float *V, const Coefs &cf, const Grid &g,
                            const ImageFuse *fuse, const TaperFuse *taper, int *flag,
@@ -2370,7 +2377,8 @@ hipError_t launch_wave_out(const T *P, T *PP, const float *V, const Coefs &cf, c
     ImageFuse fz;
     TaperFuse tf;
     fuse_args(nullptr, taper, fz, tf);
-    if (wave2_fits(P, PP, V, nullptr, g))
+    if (wave2_fits(P, PP, V, nullptr, g) &&
+        !(std::is_same<T, float>::value && narrow_tiles(g.nz)))
         return launch_wave2_cfg<T, R, 4, WPB, false, 3>(P, PP, V, cf, g, fz, tf, flag, s, xchunk,
                                                         0, 0, (g.nz + 127) / 128);
     return launch_wave_cfg<T, R, RY, WPB, false, 3>(P, PP, V, cf, g, fz, tf, flag, s, xchunk, 0,
@@ -2393,7 +2401,8 @@ hipError_t launch_wave_outu(const T *P, T *PP, const float *V, const Coefs &cf, 
     fuse_args(fuse, taper, fz, tf);
     const int xchunk = t ? t->xchunk : 0;
     const bool one = t && t->tz == 64 && t->by == 1 && (t->ry == 6 || t->ry == 8);
-    const bool two = !one && wave2_fits(P, PP, V, fuse, g);
+    const bool two = !one && wave2_fits(P, PP, V, fuse, g) &&
+                     !(!t && !fuse && std::is_same<T, float>::value && narrow_tiles(g.nz));
     const int ry = one ? t->ry : (fuse ? 6 : 8);
     if (fuse) {
         if (two)
@@ -2545,13 +2554,21 @@ hipError_t launch_radius(const T *P, T *PP, const float *V, const Coefs &cf, con
     }
     if constexpr (R == 4 && std::is_same<T, float>::value) {
         // FP32 without a requested shape: the plain step on two-z 128 x 1 x 4
-        // waves (64 x 1 x 8 waves where pairs do not fit), the tapered step
-        // on 64 x 1 x 8 waves (salt grid: 0.412 and 0.463 ms against 0.447
-        // and 0.498 for full rows 2 x 6); the fused receiver step keeps the
-        // full rows below (0.699 ms against 0.79 or more on every wave shape).
+        // waves (64 x 1 x 8 waves where pairs do not fit or fill), the tapered
+        // step on 64 x 1 x 8 waves (salt grid: 0.412 and 0.463 ms against
+        // 0.447 and 0.498 for full rows 2 x 6).  The imaging step keeps the
+        // full rows below on large grids (salt grid 0.699 ms against 0.79 or
+        // more on every wave shape) and runs 64 x 1 x 8 waves on short rows
+        // and on grids that its blocks of 12 rows would not fill (us, waves
+        // against rows: 192^3 41 / 63, 256^3 105 / 122, 500 x 500 x 130 245 /
+        // 334, 200 x 180 x 300 72 / 78, 301 x 277 x 259 164 / 178; 336^3
+        // 260 / 249).
+        const bool small = g.nz <= 256 || (long long)(g.ny / 12) * (g.nx / 16) < 500;
+        if (!t && fuse && small && (!taper || taper->b <= 8192))
+            return launch_wave<T, R, 8, 4>(P, PP, V, cf, g, fuse, taper, flag, s, xchunk);
         if (!t && !fuse && (!taper || taper->b <= 8192)) {
             const bool tapered = taper && taper->b > 0;
-            if (!tapered && wave2_fits(P, PP, V, fuse, g))
+            if (!tapered && wave2_fits(P, PP, V, fuse, g) && !narrow_tiles(g.nz))
                 return launch_wave2<T, R, 4, 4>(P, PP, V, cf, g, fuse, taper, flag, s, xchunk);
             return launch_wave<T, R, 8, 4>(P, PP, V, cf, g, fuse, taper, flag, s, xchunk);
         }
