@@ -115,6 +115,29 @@ def test_coder_matches_restatement(gpu, shape, b, keep_div):
         assert err < 2e-3
 
 
+@pytest.mark.parametrize("keep_div", [1, 16])
+@pytest.mark.parametrize("shape, b", [((8, 8, 64), 16), ((50, 8, 64), 16), ((24, 24, 64), 16),
+                                      ((17, 31, 75), 5)])
+def test_coder_groups_of_bricks(gpu, shape, b, keep_div):
+    """2, 14, 18 and 36 bricks (they are packed in groups of 8): some all zero,
+    some far below the others (every coefficient under the threshold at 1/16).
+    Same bounds as above, from FP16 quantisation and the threshold's rounding."""
+    f = np.ascontiguousarray(_wavefield((56, 40, 80), 5)[:shape[0], :shape[1], :shape[2]])
+    if shape[0] > 8:
+        f[:8, :8] = 0.0
+        f[16:, :8] *= np.float32(1e-20)
+    d = gpu.DeviceArray.from_host(f)
+    try:
+        got, kept = gpu.dct_roundtrip(d, "f32", b, keep_div)
+    finally:
+        d.free()
+    want, kept_np = coder(f, b, keep_div)
+    inside = np.s_[:, :, b:shape[2] - b]
+    assert np.isfinite(got).all()
+    assert abs(kept - kept_np) <= max(2, kept_np // 10000), (kept, kept_np)
+    assert _rel(got[inside], want[inside]) < 2e-4
+
+
 def _random_basis(seed):
     """A random orthonormal separable basis, packed (z, x, y rows)."""
     rng = np.random.default_rng(seed)
