@@ -62,7 +62,7 @@ def build_library(jobs=4, incremental=False):
     os.makedirs(LIBDIR, exist_ok=True)
     os.makedirs(OBJDIR, exist_ok=True)
     headers = [os.path.join(CSRC, h) for h in ("rtm_internal.hpp", "rtm_slab.hpp",
-                                               "rtm_slab_launch.hpp")]
+                                               "rtm_slab_launch.hpp", "rtm_tail.hpp")]
     headers.append(os.path.join(REPO, "include", "rtm_hip.h"))
     objs = []
     cmds = []

@@ -6,6 +6,7 @@
 // reference's per-step loops with no host synchronisation in between.
 #include "rtm_internal.hpp"
 #include "rtm_slab_launch.hpp"
+#include "rtm_tail.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -272,6 +273,15 @@ bool off_borders(const rtmhip_shot *shot, const ShotCtx &c)
     return in(c.rz, c.g.nz) && in(c.rx0, c.g.nx) && in(c.ry0, c.g.ny) &&
            in(c.rx0 + (long long)(r.count_x - 1) * r.dist_x, c.g.nx) &&
            in(c.ry0 + (long long)(r.count_y - 1) * r.dist_y, c.g.ny);
+}
+
+// The shot's receivers of one record chunk at time lt (mode as TailReceivers).
+TailReceivers tail_receivers(const rtmhip_shot *shot, const ShotCtx &c, const float *rec, int lt,
+                             int mode)
+{
+    const rtmhip_rcv_geom &r = shot->rcv;
+    return TailReceivers{const_cast<float *>(rec), c.rx0, c.ry0, c.rz, r.dist_x, r.dist_y,
+                         r.count_x, r.count_y, shot->ntstep, lt, mode};
 }
 
 int check_format(const rtmhip_shot *s)
@@ -595,14 +605,10 @@ int rtmhip_freq_steps(const rtmhip_shot *shot, const float *V2DT2, const float *
         if (out) {
             const TaperFuse tf{taper, b, k == 0 ? 0 : 1, 2};
             float **fields[2][2] = {{Ps, PPs}, {Pr, PPr}};
-            for (auto &f : fields) {
-                HIPCHK(launch_taper_frame_xy(*f[1], taper, c.g, b, c.radius, k == 0 ? 1 : 2, s),
-                       "frame taper");
+            for (auto &f : fields)
                 HIPCHK(stencil(c.radius, (const float *)*f[0], *f[1], V2DT2, c.cf, c.g, nullptr,
                                &tf),
                        "stencil");
-                HIPCHK(launch_taper_quirk_out(*f[1], taper, c.g, b, s), "front-right taper");
-            }
         } else {
             HIPCHK(stencil(c.radius, (const float *)*Ps, *PPs, V2DT2, c.cf, c.g, nullptr),
                    "source stencil");
@@ -611,11 +617,13 @@ int rtmhip_freq_steps(const rtmhip_shot *shot, const float *V2DT2, const float *
             HIPCHK(launch_taper_all2(*Ps, *PPs, taper, c.g, b, s), "taper");
             HIPCHK(launch_taper_all2(*Pr, *PPr, taper, c.g, b, s), "taper");
         }
-        HIPCHK(launch_source(*PPs, c.src_off, ricker, st, 0.f, s), "source");
-        HIPCHK(launch_receivers(*PPr, const_cast<float *>(rcv_chunk), c.g, c.rx0, c.ry0, c.rz,
-                                shot->rcv.dist_x, shot->rcv.dist_y, shot->rcv.count_x,
-                                shot->rcv.count_y, shot->ntstep, lt, true, s),
-               "receivers");
+        const TailReceivers rcv = tail_receivers(shot, c, rcv_chunk, lt, 2);
+        const TailSource src{ricker, c.src_off, st};
+        const int taps = !out ? 0 : (k == 0 ? 1 : 2);
+        HIPCHK(launch_tail_all(*PPs, taper, c.g, b, c.radius, taps, nullptr, &src, s),
+               "tapers and source");
+        HIPCHK(launch_tail_all(*PPr, taper, c.g, b, c.radius, taps, &rcv, nullptr, s),
+               "tapers and receivers");
         HIPCHK(launch_freq_image(img, *PPs, *PPr, sre, sim, rre, rim, kre, kim, w2, c.g, b, nwstep,
                                  iw0, nw, nt, st, s),
                "frequency contributions");
@@ -664,9 +672,10 @@ int model_loop(const rtmhip_shot *shot, const ShotCtx &c, const float *V2DT2, co
     // rtmhip_set_taper_fusion mode 3) it is applied to each step's output:
     // the step stores taper3D of its new value (the next step's P, so P is
     // read as stored) and tapers the centre PP once; PP's x-y frame is
-    // tapered twice before the step (it is this step's PP and the next
+    // tapered twice (it is this step's PP and the next
     // step's P), the z frame by the stencil, and the front-right edge is
-    // written after the step from the stored (b, y, z).  The first step of a
+    // written after the step from the stored (b, y, z), with the frame, the
+    // source and the receivers (k_tail_all).  The first step of a
     // call tapers P in place, the last tapers PP in place and runs the plain
     // step, so the state between calls is the reference's.  The source and
     // the receivers must lie off the borders, where taper3D leaves values
@@ -689,9 +698,7 @@ int model_loop(const rtmhip_shot *shot, const ShotCtx &c, const float *V2DT2, co
         if (out && !last) {
             if (it == it0) HIPCHK(launch_taper(*P, taper, c.g, b, false, s), "taper");
             const TaperFuse tf{taper, b, 1, 2};
-            HIPCHK(launch_taper_frame_xy(*PP, taper, c.g, b, c.radius, 2, s), "frame taper");
             HIPCHK(stencil(c.radius, *P, *PP, V2DT2, c.cf, c.g, nullptr, &tf), "stencil");
-            HIPCHK(launch_taper_quirk_out(*PP, taper, c.g, b, s), "front-right taper");
         } else if (out) {
             if (it == it0)
                 HIPCHK(launch_taper_all2(*P, *PP, taper, c.g, b, s), "taper");
@@ -708,11 +715,12 @@ int model_loop(const rtmhip_shot *shot, const ShotCtx &c, const float *V2DT2, co
             HIPCHK(launch_taper_all2(*P, *PP, taper, c.g, b, s), "taper");
             HIPCHK(stencil(c.radius, *P, *PP, V2DT2, c.cf, c.g, nullptr), "stencil");
         }
-        HIPCHK(launch_source(*PP, c.src_off, ricker, it, 0.f, s), "source");
-        HIPCHK(launch_receivers(*PP, rcv_chunk, c.g, c.rx0, c.ry0, c.rz, shot->rcv.dist_x,
-                                shot->rcv.dist_y, shot->rcv.count_x, shot->rcv.count_y,
-                                shot->ntstep, it % shot->ntstep, false, s),
-               "receivers");
+        // the frame and the front-right edge of an output-tapered step, the
+        // source and the receivers
+        const TailReceivers rcv = tail_receivers(shot, c, rcv_chunk, it % shot->ntstep, 1);
+        const TailSource src{ricker, c.src_off, it};
+        HIPCHK(launch_tail_all(*PP, taper, c.g, b, c.radius, out && !last ? 2 : 0, &rcv, &src, s),
+               "tapers, source and receivers");
     }
     if (fused && nsteps > 0) HIPCHK(launch_taper(*P, taper, c.g, b, false, s), "taper");
     return RTMHIP_OK;
@@ -743,8 +751,10 @@ int forward_loop(const rtmhip_shot *shot, const ShotCtx &c, int hbc, const float
     //   orders them.
     const bool sep = g_state.taper_sep[shot->wave_format];
     const int b = shot->blen;
+    // (b >= 2R keeps the layer off the z frame)
     const bool outu = hbc && g_state.taper_outu[shot->wave_format] && c.radius == 4 &&
-                      shot->sze >= b;
+                      shot->sze >= b && b >= 2 * c.radius;
+    const size_t layer = (size_t)c.g.nx * c.g.ny * c.hf;
     for (int it = it0; it < it0 + nsteps; ++it) {
         // history layer: every step held (hbc 1) or one receiver chunk (hbc 2)
         const int ul = hbc == 2 ? it % shot->ntstep : it;
@@ -756,10 +766,11 @@ int forward_loop(const rtmhip_shot *shot, const ShotCtx &c, int hbc, const float
                 if (it == it0) HIPCHK(launch_taper(*P, taper, c.g, b, true, s), "taper");
                 const TaperFuse tf{taper, b, 1, 3, c.hf};
                 HIPCHK(stencil(c.radius, *P, *PP, V2DT2, c.cf, c.g, nullptr, &tf), "stencil");
-                HIPCHK(launch_taper_frame(*PP, taper, c.g, b, c.radius, 2, s, c.hf),
-                       "frame taper");
-                HIPCHK(launch_source(*PP, c.src_off, ricker, it, 0.f, s), "source");
-                HIPCHK(launch_upb_save_taper(*PP, upb, taper, c.g, b, c.hf, ul, s), "upb save");
+                const TailLayer<T> w{2, 1, upb + (size_t)ul * layer, nullptr, nullptr};
+                const TailSource src{ricker, c.src_off, it};
+                HIPCHK(launch_tail_upper<T>(*PP, taper, c.g, b, c.radius, w, nullptr, &src,
+                                            nullptr, nullptr, s),
+                       "frame, history and source");
                 continue;
             }
             if (it == it0)
@@ -777,6 +788,16 @@ int forward_loop(const rtmhip_shot *shot, const ShotCtx &c, int hbc, const float
                    "frame taper");
         } else {
             HIPCHK(stencil(c.radius, *P, *PP, V2DT2, c.cf, c.g, nullptr), "stencil");
+        }
+        // the source lies off the layer or is saved with it
+        const long long sz = c.src_off % c.g.sy;
+        if (hbc && (sz < b - c.hf || sz >= b)) {
+            const TailLayer<T> w{0, 0, upb + (size_t)ul * layer, nullptr, nullptr};
+            const TailSource src{ricker, c.src_off, it};
+            HIPCHK(launch_tail_upper<T>(*PP, taper, c.g, b, c.radius, w, nullptr, &src,
+                                        nullptr, nullptr, s),
+                   "history and source");
+            continue;
         }
         HIPCHK(launch_source(*PP, c.src_off, ricker, it, 0.f, s), "source");
         if (hbc) HIPCHK(launch_upb(*PP, upb, c.g, shot->blen, c.hf, ul, false, s), "upb save");
@@ -802,9 +823,11 @@ int backward_loop(const rtmhip_shot *shot, const ShotCtx &c, int hbc, const floa
     // snap_backward_run (receivers and imaged range lie at z >= blen)
     const bool outr = hbc && fused && !dual && !sep &&
                       image_outu<T>(shot->wave_format, c.radius, c.g, taper, b);
+    const size_t layer = (size_t)c.g.nx * c.g.ny * c.hf;
     for (int it = it_hi; it > it_hi - nsteps; --it) {
         const int lt = it % shot->ntstep;
         const int ul = hbc == 2 ? lt : it;  // history layer, as in forward_loop
+        const T *restore = nullptr;  // the layer to restore after the receiver step
         if constexpr (std::is_same<T, float>::value) {
             if (dual && it < nt - 2) {
                 // both backward steps in one pass (class 3), then the UPB
@@ -856,8 +879,9 @@ int backward_loop(const rtmhip_shot *shot, const ShotCtx &c, int hbc, const floa
         } else if (it == nt - 2) {
             S = *Ps;   // snap0 (entry state: Ps = snap0, PPs = snap1)
         } else {
+            if (hbc) restore = upb + (size_t)ul * layer;
             HIPCHK(stencil(c.radius, *Ps, *PPs, V2DT2, c.cf, c.g, nullptr), "stencil");
-            if (hbc)
+            if (hbc && !fused)
                 HIPCHK(launch_upb(*PPs, const_cast<T *>(upb), c.g, b, c.hf, ul, true, s),
                        "upb restore");
             T *t = *Ps;
@@ -892,15 +916,12 @@ int backward_loop(const rtmhip_shot *shot, const ShotCtx &c, int hbc, const floa
             fz.rny = shot->rcv.count_y;
             HIPCHK(stencil(c.radius, *Pr, *PPr, V2DT2, c.cf, c.g, &fz, tapered ? &tf : nullptr),
                    "fused stencil");
-            if (tapered)
-                HIPCHK(launch_taper_frame(*PPr, taper, c.g, b, c.radius, outr ? 2 : tf.pp_taps,
-                                          s),
-                       "frame taper");
-            HIPCHK(launch_receivers_image(*PPr, rcv_chunk, c.g, c.rx0, c.ry0, c.rz,
-                                          shot->rcv.dist_x, shot->rcv.dist_y, shot->rcv.count_x,
-                                          shot->rcv.count_y, shot->ntstep, lt, img, S, z0, z1,
-                                          c.radius, s),
-                   "receivers+image");
+            // (the layer lies above the imaged range, so its restore may wait)
+            const TailLayer<T> w{!tapered ? 0 : (outr ? 2 : tf.pp_taps), 0, nullptr, *Ps, restore};
+            const TailReceivers rcv = tail_receivers(shot, c, rcv_chunk, lt, 3);
+            HIPCHK(launch_tail_upper<T>(*PPr, taper, c.g, b, c.radius, w, &rcv, nullptr, img,
+                                        S, s),
+                   "frame, history, receivers and image");
         } else {
             HIPCHK(stencil(c.radius, *Pr, *PPr, V2DT2, c.cf, c.g, nullptr), "stencil");
             HIPCHK(launch_receivers(*PPr, const_cast<float *>(rcv_chunk), c.g, c.rx0, c.ry0,
@@ -950,11 +971,12 @@ int snap_forward_run(const rtmhip_shot *shot, const ShotCtx &c, const float *V2D
         T *t = *P;
         *P = *PP;
         *PP = t;
+        TailLayer<T> w{0, 0, nullptr, nullptr, nullptr};  // the frame after the step
         if (outu && it < it0 + nsteps - 1) {
             if (it == it0) HIPCHK(launch_taper(*P, taper, c.g, b, true, s), "taper");
             const TaperFuse tf{taper, b, 1, 3, 0};
             HIPCHK(stencil(c.radius, *P, *PP, V2DT2, c.cf, c.g, nullptr, &tf), "stencil");
-            HIPCHK(launch_taper_frame(*PP, taper, c.g, b, c.radius, 2, s), "frame taper");
+            w.taps = 2;
         } else if (outu) {
             if (it == it0)
                 HIPCHK(launch_taper_upper2(*P, *PP, taper, c.g, b, s), "taper");
@@ -970,7 +992,10 @@ int snap_forward_run(const rtmhip_shot *shot, const ShotCtx &c, const float *V2D
             HIPCHK(launch_taper_frame(*PP, taper, c.g, b, c.radius, tf.pp_taps, s),
                    "frame taper");
         }
-        HIPCHK(launch_source(*PP, c.src_off, ricker, it, 0.f, s), "source");
+        const TailSource src{ricker, c.src_off, it};
+        HIPCHK(launch_tail_upper<T>(*PP, taper, c.g, b, c.radius, w, nullptr, &src, nullptr,
+                                    nullptr, s),
+               "frame and source");
         const int j = snap_slot(it, shot->nt, k);
         if (j >= 0) {
             const int rc = store((const T *)*PP, j);
@@ -1011,11 +1036,12 @@ int snap_backward_run(const rtmhip_shot *shot, const ShotCtx &c, const float *V2
     // forward loops (the receivers and the imaged range lie at z >= blen)
     const bool outu = g_state.taper_outu[shot->wave_format] && c.radius == 4 && c.rz >= b;
     for (int it = it_hi; it > it_hi - nsteps; --it) {
+        TailLayer<T> w{0, 0, nullptr, nullptr, nullptr};  // the frame after the step
         if (outu && it > it_hi - nsteps + 1) {
             if (it == it_hi) HIPCHK(launch_taper(*Pr, taper, c.g, b, true, s), "taper");
             const TaperFuse tf{taper, b, 1, 3, 0};
             HIPCHK(stencil(c.radius, *Pr, *PPr, V2DT2, c.cf, c.g, nullptr, &tf), "stencil");
-            HIPCHK(launch_taper_frame(*PPr, taper, c.g, b, c.radius, 2, s), "frame taper");
+            w.taps = 2;
         } else if (outu) {
             if (it == it_hi)
                 HIPCHK(launch_taper_upper2(*Pr, *PPr, taper, c.g, b, s), "taper");
@@ -1031,10 +1057,10 @@ int snap_backward_run(const rtmhip_shot *shot, const ShotCtx &c, const float *V2
             HIPCHK(launch_taper_frame(*PPr, taper, c.g, b, c.radius, tf.pp_taps, s),
                    "frame taper");
         }
-        HIPCHK(launch_receivers(*PPr, const_cast<float *>(rcv_chunk), c.g, c.rx0, c.ry0, c.rz,
-                                shot->rcv.dist_x, shot->rcv.dist_y, shot->rcv.count_x,
-                                shot->rcv.count_y, shot->ntstep, it % shot->ntstep, true, s),
-               "receivers");
+        const TailReceivers rcv = tail_receivers(shot, c, rcv_chunk, it % shot->ntstep, 2);
+        HIPCHK(launch_tail_upper<T>(*PPr, taper, c.g, b, c.radius, w, &rcv, nullptr,
+                                    nullptr, nullptr, s),
+               "frame and receivers");
         const int j = snap_slot(it, shot->nt, k);
         if (j >= 0) {
             const int rc = image((const T *)*PPr, j);

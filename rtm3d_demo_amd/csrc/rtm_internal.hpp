@@ -188,15 +188,6 @@ hipError_t launch_taper_frame(T *P, const float *taper, const Grid &g, int b, in
 template <typename T>
 hipError_t launch_taper_frame_all(T *P, const float *taper, const Grid &g, int b, int R, int taps,
                                   hipStream_t s);
-// taper3D on a step's output (TaperFuse all 2): the cells with x or y within
-// R of a face, `taps` times in place, front-right edge cells excepted
-// (launch_taper_frame_xy, before the step); then the front-right edge cells
-// from the stored (b, y, z) (launch_taper_quirk_out, after the step).
-template <typename T>
-hipError_t launch_taper_frame_xy(T *P, const float *taper, const Grid &g, int b, int R, int taps,
-                                 hipStream_t s);
-template <typename T>
-hipError_t launch_taper_quirk_out(T *P, const float *taper, const Grid &g, int b, hipStream_t s);
 template <typename T>
 hipError_t launch_source(T *PP, long long offset, const float *table, int it, float value,
                          hipStream_t s);
@@ -211,12 +202,6 @@ hipError_t launch_receivers_image(T *PP, const float *rcv, const Grid &g, int rx
 template <typename T>
 hipError_t launch_upb(T *PP, T *upb, const Grid &g, int blen, int hf, long long lt, bool restore,
                       hipStream_t s);
-// The upper-border history saved from PP's planes [blen-hf, blen), then the
-// upper taper applied to those planes in place (a step that stores the upper
-// taper of its output left them untapered).
-template <typename T>
-hipError_t launch_upb_save_taper(T *PP, T *upb, const float *taper, const Grid &g, int blen,
-                                 int hf, long long lt, hipStream_t s);
 template <typename T>
 hipError_t launch_image(float *img, const T *PS, const T *PR, const Grid &g, int z0, int z1,
                         hipStream_t s);

@@ -7,6 +7,7 @@
 // float and rounded once per stored value, as the reference's in-place
 // operators would with grids of that type.
 #include "rtm_internal.hpp"
+#include "rtm_tail.hpp"
 
 #include <algorithm>
 
@@ -425,31 +426,6 @@ __global__ void __launch_bounds__(kThreads)
     P[o] = wst<T>(all_taper<T>(wld(P[o]), t, g, b, x, y, z, taps));
 }
 
-// The front-right edge of taper3D applied to a step's output (the step
-// fused with TAPER 3 stored every other cell tapered): cells x < b, y >=
-// ny-b, z in [b, nz-b) take the face-tapered value of (b, y, z), which the
-// step stored as (v*gy) rounded, then ((.)*gx)*gy.  Runs after the step and
-// after the frame pass.
-template <typename T>
-__global__ void __launch_bounds__(kThreads)
-    k_taper_quirk_out(T *__restrict__ P, const float *__restrict__ t, Grid g, int b, FastDiv dlz,
-                      FastDiv db, int n)
-{
-    const int i = (int)(blockIdx.x * kThreads + threadIdx.x);  // n < 2^31 (launcher)
-    if (i >= n) return;
-    const int lz = g.nz - 2 * b;
-    const int r = fdiv(i, dlz);
-    const int z = b + (i - r * lz);
-    const int x = fdiv(r, db);
-    const int iy = r - x * b;
-    const int y = g.ny - b + iy;
-    const float gy = t[iy];
-    float v = wld(P[goff(g, b, y, z)]);
-    v *= t[b - 1 - x];
-    v *= gy;
-    P[goff(g, x, y, z)] = wst<T>(v);
-}
-
 // The front-right edge cells of that frame (x < R, or y >= ny-R), from the
 // cell (b, y, z) before this step's tapers: the face pass's (v*gy) rounded,
 // `taps` times, then (v*gx)*gy.  Runs before k_taper_frame_all, which
@@ -787,14 +763,12 @@ __global__ void __launch_bounds__(kThreads)
 
 // rtmSaveUpperBorder / rtmRestoreUpperBorder (RTMCPUPlatform.cpp:153-189):
 // upb[lt][x][y][k] <-> PP[x][y][blen-hf+k], 64-bit offsets.
-// mode 0 save, 1 restore, 2 save and then apply the upper taper (table t)
-// to the saved cell in place.
 // 32-bit cell index (n = nx * ny * hf < 2^31, launcher) with divisions by
 // launch constants through a multiply-high; the history offset is 64-bit.
 template <typename T>
 __global__ void __launch_bounds__(kThreads)
-    k_upb(T *__restrict__ PP, T *__restrict__ upb, Grid g, int b, int hf, long long lt, int mode,
-          const float *__restrict__ t, int n, FastDiv dhf, FastDiv dny)
+    k_upb(T *__restrict__ PP, T *__restrict__ upb, Grid g, int b, int hf, long long lt,
+          int restore, int n, FastDiv dhf, FastDiv dny)
 {
     const int i = (int)(blockIdx.x * kThreads + threadIdx.x);
     if (i >= n) return;
@@ -805,13 +779,8 @@ __global__ void __launch_bounds__(kThreads)
     const long long u = lt * (long long)n + i;
     const int z = b - hf + k;
     const long long o = goff(g, x, y, z);
-    if (mode == 1) {
-        PP[o] = upb[u];
-    } else {
-        const T v = PP[o];
-        upb[u] = v;
-        if (mode == 2) PP[o] = wst<T>(frame_taper<T>(wld(v), t, g, b, x, y, z, 1));
-    }
+    if (restore) PP[o] = upb[u];
+    else upb[u] = PP[o];
 }
 
 // rtmImageCondition (RTMCPUPlatform.cpp:513-540): z in [z0, z1), all x, y.
@@ -1047,6 +1016,250 @@ __global__ void __launch_bounds__(kThreads)
     sh.img[o] = sh.img[o] + wld(PPs[o]) * wld(PPr[o]);
 }
 
+// ---------------------------------------------------------------------------
+// Tails: every small operator that follows a step of one grid, in one launch.
+// A launch costs 2.5-5 us from end to end, as much as any of these operators
+// on its own (salt grid: frame taper 17 us, history 17, source 5, receivers 5;
+// 192^3 and smaller: 2.3-4.8 us each against a 24-us step), so what they
+// share is the launch.  Work items are numbered through the parts in order;
+// the parts of one launch touch disjoint cells, and a part that would depend
+// on another does that cell's work itself (see k_tail_all).
+
+// One receiver: 1 sampled into the record, 2 set, 3 set and imaged.  A sampled
+// receiver on the source cell takes the source with it (src_on_rcv).
+struct TailRcv {
+    float *rec;
+    int rx0, ry0, rz, rdx, rdy, rnx, rny, ntstep, lt, mode;
+    FastDiv dny;
+};
+struct TailSrc {
+    const float *table;  // NULL: no source
+    long long off;
+    int it;
+    int on_rcv;  // the source cell is a sampled receiver's
+};
+
+// Receiver i; false where it lies off the grid.
+template <typename T>
+__device__ __forceinline__ void tail_receiver(T *__restrict__ PP, const TailRcv &r, const Grid &g,
+                                              int i, const TailSrc &src, float *__restrict__ img,
+                                              const T *__restrict__ ps, int z0, int z1)
+{
+    const int ix = fdiv(i, r.dny), iy = i - ix * r.rny;
+    const int rx = r.rx0 + ix * r.rdx, ry = r.ry0 + iy * r.rdy;
+    if (rx < 0 || rx >= g.nx || ry < 0 || ry >= g.ny) return;
+    const long long o = goff(g, rx, ry, r.rz), ro = (long long)i * r.ntstep + r.lt;
+    if (r.mode == 1) {
+        T v = PP[o];
+        if (src.on_rcv && o == src.off) {
+            v = wst<T>(wld(v) + src.table[src.it]);
+            PP[o] = v;
+        }
+        r.rec[ro] = wld(v);
+    } else if (r.mode == 2) {
+        PP[o] = wst<T>(r.rec[ro]);
+    } else {
+        inject_image(PP, img, ps, g, rx, ry, r.rz, r.rec[ro], z0, z1);
+    }
+}
+
+// After a step with taper3D on its output: the x-y frame of PP tapered `taps`
+// times and the front-right edge from the stored (b, y, z); with taps 0 only
+// the source and the receivers.  Items: frame cells (nX in the x slabs, nF in
+// all), the edge's cells with y < ny - R, the receivers, the source.  The
+// edge's cells with y >= ny - R come from frame cells of this launch, so the
+// item that tapers (b, y, z) writes them.
+template <typename T>
+__global__ void __launch_bounds__(kThreads)
+    k_tail_all(T *__restrict__ P, const float *__restrict__ t, Grid g, int b, int R, int taps,
+               int nX, int nF, int nQ, FastDiv dnz, FastDiv dny, FastDiv dr2, FastDiv dlz,
+               FastDiv dqy, TailRcv rcv, TailSrc src)
+{
+    int i = (int)(blockIdx.x * kThreads + threadIdx.x);  // count < 2^31 (launcher)
+    if (i < nF) {
+        int x, y;
+        const int r = fdiv(i < nX ? i : i - nX, dnz);
+        const int z = (i < nX ? i : i - nX) - r * g.nz;
+        if (i < nX) {
+            const int xx = fdiv(r, dny);
+            y = r - xx * g.ny;
+            x = xx < R ? xx : g.nx - 2 * R + xx;
+        } else {
+            const int xr = fdiv(r, dr2);
+            const int yy = r - xr * 2 * R;
+            x = R + xr;
+            y = yy < R ? yy : g.ny - 2 * R + yy;
+        }
+        const bool zin = z >= b && z < g.nz - b;
+        if (x < b && y >= g.ny - b && zin) return;  // the edge, below
+        const long long o = goff(g, x, y, z);
+        const T v = wst<T>(all_taper<T>(wld(P[o]), t, g, b, x, y, z, taps));
+        P[o] = v;
+        if (x == b && y >= g.ny - R && zin) {
+            const float gy = t[y - (g.ny - b)];
+            for (int ex = 0; ex < b; ++ex) {
+                float w = wld(v);
+                w *= t[b - 1 - ex];
+                w *= gy;
+                P[goff(g, ex, y, z)] = wst<T>(w);
+            }
+        }
+        return;
+    }
+    i -= nF;
+    if (i < nQ) {
+        const int lz = g.nz - 2 * b;
+        const int r = fdiv(i, dlz);
+        const int z = b + (i - r * lz);
+        const int x = fdiv(r, dqy);
+        const int iy = r - x * (b - R);
+        const int y = g.ny - b + iy;
+        float v = wld(P[goff(g, b, y, z)]);
+        v *= t[b - 1 - x];
+        v *= t[iy];
+        P[goff(g, x, y, z)] = wst<T>(v);
+        return;
+    }
+    i -= nQ;
+    const int nr = rcv.mode ? rcv.rnx * rcv.rny : 0;
+    if (i < nr) {
+        tail_receiver(P, rcv, g, i, src, (float *)nullptr, (const T *)nullptr, 0, 0);
+    } else if (i == nr && src.table && !src.on_rcv) {
+        P[src.off] = wst<T>(wld(P[src.off]) + src.table[src.it]);
+    }
+}
+
+// After an HBC step.  Parts, each of a launch's choice:
+//   layer   the upper-border layer (z in [b - R, b)): of Q from restore; or
+//           of PP into save -- its frame cells tapered taps - 1 times first --
+//           and then, with hold (a step that left the layer untapered),
+//           tapered once;
+//   frame   the cells of PP's slab frame tapered `taps` times (outside the
+//           layer with hold: the layer's items do those);
+//   rcv     the receivers of PP;  image  img += ps * PP on the imaged cells
+//           that the step does not visit;  src  the source cell of PP.
+//
+// The layer and the frame's z < R cells are 4 cells of every row: one thread
+// per row moves them as a vector (VEC: rows, border and arrays allow it), since
+// the cost is the 128-byte line each row touches.
+struct TailUpper {
+    int nl, na, nf, ni;  // items: layer rows, frame rows (z < R), frame cells, imaged cells
+    int taps, hold;
+    FrameDivs fd, id;
+    FastDiv dny;
+    int z0, z1;
+};
+
+// N consecutive cells of a row.
+template <typename T, int N, bool VEC>
+__device__ __forceinline__ void ld_run(const T *p, T (&v)[N])
+{
+    if constexpr (VEC) {
+        const SnapVec<T, N> a = *reinterpret_cast<const SnapVec<T, N> *>(p);
+#pragma unroll
+        for (int k = 0; k < N; ++k) v[k] = a.v[k];
+    } else {
+#pragma unroll
+        for (int k = 0; k < N; ++k) v[k] = p[k];
+    }
+}
+template <typename T, int N, bool VEC>
+__device__ __forceinline__ void st_run(T *p, const T (&v)[N])
+{
+    if constexpr (VEC) {
+        SnapVec<T, N> a;
+#pragma unroll
+        for (int k = 0; k < N; ++k) a.v[k] = v[k];
+        *reinterpret_cast<SnapVec<T, N> *>(p) = a;
+    } else {
+#pragma unroll
+        for (int k = 0; k < N; ++k) p[k] = v[k];
+    }
+}
+
+template <typename T, int R, bool VEC>
+__global__ void __launch_bounds__(kThreads)
+    k_tail_upper(T *__restrict__ PP, const float *__restrict__ t, Grid g, int b, TailUpper u,
+                 T *__restrict__ save, T *__restrict__ Q, const T *__restrict__ restore,
+                 TailRcv rcv, TailSrc src, float *__restrict__ img, const T *__restrict__ ps)
+{
+    int i = (int)(blockIdx.x * kThreads + threadIdx.x);  // count < 2^31 (launcher)
+    int x, y, z;
+    if (i < u.nl + u.na) {
+        const bool lay = i < u.nl;
+        const int row = lay ? i : i - u.nl;
+        x = fdiv(row, u.dny);
+        y = row - x * g.ny;
+        z = lay ? b - R : 0;
+        const long long o = goff(g, x, y, z);
+        T v[R];
+        if (lay && restore) {
+            ld_run<T, R, VEC>(restore + (long long)row * R, v);
+            st_run<T, R, VEC>(Q + o, v);
+            return;
+        }
+        ld_run<T, R, VEC>(PP + o, v);
+        if (!lay || u.hold) {
+            const bool bx = x < b || x >= g.nx - b, by = y < b || y >= g.ny - b;
+            const float fy = by ? gfac(t, y, g.ny, b) : 1.0f;
+            const float fx = bx ? gfac(t, x, g.nx, b) : 1.0f;
+            const bool rim = x < R || x >= g.nx - R || y < R || y >= g.ny - R;
+            auto taper = [&](int taps) {
+                for (int k = 0; k < taps; ++k)
+#pragma unroll
+                    for (int e = 0; e < R; ++e) {
+                        float w = wld(v[e]) * fy;
+                        w *= fx;
+                        w *= t[b - 1 - z - e];
+                        v[e] = wst<T>(w);
+                    }
+            };
+            if (!lay) {
+                taper(u.taps);
+                st_run<T, R, VEC>(PP + o, v);
+                return;
+            }
+            // a row of the frame; elsewhere the step tapers nothing here
+            // (b >= 2R, or its z < R cells would be frame cells too)
+            if (rim) taper(u.taps - 1);
+            st_run<T, R, VEC>(save + (long long)row * R, v);
+            taper(1);
+            st_run<T, R, VEC>(PP + o, v);
+            return;
+        }
+        st_run<T, R, VEC>(save + (long long)row * R, v);
+        return;
+    }
+    i -= u.nl + u.na;
+    if (i < u.nf) {
+        // past the z < R rows: the x and y frame on z in [R, b)
+        if (!frame_cell_fd(g, b, R, g.nx * g.ny * R + i, u.fd, x, y, z) ||
+            (u.hold && z >= b - R))
+            return;
+        const long long o = goff(g, x, y, z);
+        PP[o] = wst<T>(frame_taper<T>(wld(PP[o]), t, g, b, x, y, z, u.taps));
+        return;
+    }
+    i -= u.nf;
+    const int nr = rcv.mode ? rcv.rnx * rcv.rny : 0;
+    if (i < nr) {
+        tail_receiver(PP, rcv, g, i, src, img, ps, u.z0, u.z1);
+        return;
+    }
+    i -= nr;
+    if (i < u.ni) {
+        if (!image_frame_cell_fd(g, R, u.z0, u.z1, i, u.id, x, y, z)) return;
+        if (z == rcv.rz && is_receiver(x, y, z, rcv.rx0, rcv.ry0, rcv.rz, rcv.rdx, rcv.rdy,
+                                       rcv.rnx, rcv.rny))
+            return;
+        const long long o = goff(g, x, y, z);
+        img[o] = img[o] + wld(ps[o]) * wld(PP[o]);
+        return;
+    }
+    if (i == u.ni && src.table && !src.on_rcv)
+        PP[src.off] = wst<T>(wld(PP[src.off]) + src.table[src.it]);
+}
+
 __global__ void k_tick(int *p, int d, int set)
 {
     if (threadIdx.x == 0 && blockIdx.x == 0) *p = set ? d : *p + d;
@@ -1178,33 +1391,6 @@ hipError_t launch_taper_frame_all(T *P, const float *taper, const Grid &g, int b
 }
 
 template <typename T>
-hipError_t launch_taper_frame_xy(T *P, const float *taper, const Grid &g, int b, int R, int taps,
-                                 hipStream_t s)
-{
-    if (b <= 0 || taps <= 0) return hipSuccess;
-    if (b < R || 2 * b >= g.nx || 2 * b >= g.ny || 2 * b >= g.nz) return hipErrorInvalidValue;
-    const long long nX = (long long)2 * R * g.ny * g.nz;
-    const long long n = nX + (long long)(g.nx - 2 * R) * 2 * R * g.nz;
-    if (n + kThreads >= (1LL << 31)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_taper_frame_all<T>, dim3(nblocks(n)), dim3(kThreads), 0, s, P, taper, g,
-                       b, R, taps, (int)nX, (int)n);
-    return hipGetLastError();
-}
-
-template <typename T>
-hipError_t launch_taper_quirk_out(T *P, const float *taper, const Grid &g, int b, hipStream_t s)
-{
-    if (b <= 0) return hipSuccess;
-    if (2 * b >= g.nx || 2 * b >= g.ny || 2 * b >= g.nz) return hipErrorInvalidValue;
-    const long long lz = g.nz - 2 * b;
-    const long long n = (long long)b * b * lz;
-    if (n + kThreads >= (1LL << 31)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_taper_quirk_out<T>, dim3(nblocks(n)), dim3(kThreads), 0, s, P, taper, g,
-                       b, fast_div((uint32_t)lz), fast_div((uint32_t)b), (int)n);
-    return hipGetLastError();
-}
-
-template <typename T>
 hipError_t launch_source(T *PP, long long offset, const float *table, int it, float value,
                          hipStream_t s)
 {
@@ -1249,20 +1435,8 @@ hipError_t launch_upb(T *PP, T *upb, const Grid &g, int b, int hf, long long lt,
     const long long n = (long long)g.nx * g.ny * hf;
     if (hf <= 0 || n + kThreads >= (1LL << 31)) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_upb<T>, dim3(nblocks(n)), dim3(kThreads), 0, s, PP, upb, g, b, hf, lt,
-                       restore ? 1 : 0, (const float *)nullptr, (int)n, fast_div((uint32_t)hf),
+                       restore ? 1 : 0, (int)n, fast_div((uint32_t)hf),
                        fast_div((uint32_t)g.ny));
-    return hipGetLastError();
-}
-
-template <typename T>
-hipError_t launch_upb_save_taper(T *PP, T *upb, const float *taper, const Grid &g, int b, int hf,
-                                 long long lt, hipStream_t s)
-{
-    if (!taper || hf <= 0 || hf > b) return hipErrorInvalidValue;
-    const long long n = (long long)g.nx * g.ny * hf;
-    if (n + kThreads >= (1LL << 31)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_upb<T>, dim3(nblocks(n)), dim3(kThreads), 0, s, PP, upb, g, b, hf, lt, 2,
-                       taper, (int)n, fast_div((uint32_t)hf), fast_div((uint32_t)g.ny));
     return hipGetLastError();
 }
 
@@ -1390,6 +1564,128 @@ hipError_t launch_tail_bwd(const BatchShot *shots, int n, int blocks, int spar, 
     return hipGetLastError();
 }
 
+namespace {
+
+// Cells of the slab frame (frame_cell_fd's range).
+long long tail_frame_count(const Grid &g, int b, int R)
+{
+    const long long lz = b - R;
+    return (long long)g.nx * g.ny * R + (long long)2 * R * g.ny * lz +
+           (long long)(g.nx - 2 * R) * 2 * R * lz;
+}
+
+TailRcv tail_rcv(const TailReceivers *r)
+{
+    TailRcv o{};
+    o.rdx = o.rdy = 1;
+    if (!r || r->rnx <= 0 || r->rny <= 0) return o;
+    o.rec = r->rec;
+    o.rx0 = r->rx0;
+    o.ry0 = r->ry0;
+    o.rz = r->rz;
+    o.rdx = std::max(1, r->rdx);
+    o.rdy = std::max(1, r->rdy);
+    o.rnx = r->rnx;
+    o.rny = r->rny;
+    o.ntstep = r->ntstep;
+    o.lt = r->lt;
+    o.mode = r->mode;
+    o.dny = fast_div((uint32_t)r->rny);
+    return o;
+}
+
+// The source, and whether a sampled receiver sits on its cell.
+TailSrc tail_src(const TailSource *q, const TailRcv &r, const Grid &g)
+{
+    TailSrc o{};
+    if (!q) return o;
+    const auto on = [](int v, int v0, int d, int n) {
+        return v >= v0 && (v - v0) % d == 0 && (v - v0) / d < n;
+    };
+    o.table = q->table;
+    o.off = q->off;
+    o.it = q->it;
+    const int x = (int)(q->off / g.sx), y = (int)(q->off % g.sx / g.sy), z = (int)(q->off % g.sy);
+    o.on_rcv = r.mode == 1 && z == r.rz && on(x, r.rx0, r.rdx, r.rnx) && on(y, r.ry0, r.rdy, r.rny);
+    return o;
+}
+
+}  // namespace
+
+template <typename T>
+hipError_t launch_tail_all(T *PP, const float *taper, const Grid &g, int b, int R, int taps,
+                           const TailReceivers *receivers, const TailSource *source,
+                           hipStream_t s)
+{
+    const TailRcv r = tail_rcv(receivers);
+    const TailSrc q = tail_src(source, r, g);
+    long long nX = 0, nF = 0, nQ = 0;
+    if (taps > 0) {
+        if (b < R || 2 * b >= g.nx || 2 * b >= g.ny || 2 * b >= g.nz) return hipErrorInvalidValue;
+        nX = (long long)2 * R * g.ny * g.nz;
+        nF = nX + (long long)(g.nx - 2 * R) * 2 * R * g.nz;
+        nQ = (long long)b * (b - R) * (g.nz - 2 * b);
+    }
+    const long long n = nF + nQ + (r.mode ? (long long)r.rnx * r.rny : 0) + 1;
+    if (n + kThreads >= (1LL << 31)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_tail_all<T>, dim3(nblocks(n)), dim3(kThreads), 0, s, PP, taper, g, b, R,
+                       taps, (int)nX, (int)nF, (int)nQ, fast_div((uint32_t)g.nz),
+                       fast_div((uint32_t)g.ny), fast_div((uint32_t)(2 * R)),
+                       fast_div((uint32_t)std::max(1, g.nz - 2 * b)),
+                       fast_div((uint32_t)std::max(1, b - R)), r, q);
+    return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_tail_upper(T *PP, const float *taper, const Grid &g, int b, int R,
+                             const TailLayer<T> &w, const TailReceivers *receivers,
+                             const TailSource *source, float *img, const T *ps, hipStream_t s)
+{
+    const TailRcv r = tail_rcv(receivers);
+    const TailSrc q = tail_src(source, r, g);
+    const int z0 = b, z1 = g.nz - b;
+    TailUpper u{};
+    u.taps = w.taps;
+    u.hold = w.hold;
+    long long nl = 0, na = 0, nf = 0, ni = 0;
+    const long long rows = (long long)g.nx * g.ny;
+    if (w.save && w.restore) return hipErrorInvalidValue;
+    if (w.save || w.restore) nl = rows;
+    if (w.taps > 0) {
+        na = rows;
+        nf = tail_frame_count(g, b, R) - rows * R;
+    }
+    if (img) ni = (long long)2 * R * (g.ny + g.nx - 2 * R) * std::max(0, z1 - z0);
+    if (w.hold && (!w.save || w.taps < 1 || b < 2 * R)) return hipErrorInvalidValue;
+    if ((nl || nf) && b < R) return hipErrorInvalidValue;
+    const long long n = nl + na + nf + (r.mode ? (long long)r.rnx * r.rny : 0) + ni + 1;
+    if (n + kThreads >= (1LL << 31) || rows * R + n >= (1LL << 31)) return hipErrorInvalidValue;
+    u.nl = (int)nl;
+    u.na = (int)na;
+    u.nf = (int)nf;
+    u.ni = (int)ni;
+    u.fd = frame_divs(R, b - R, g.ny);
+    u.id = frame_divs(R, z1 - z0, g.ny);
+    u.dny = fast_div((uint32_t)g.ny);
+    u.z0 = z0;
+    u.z1 = z1;
+    const auto al = [](const void *p) { return ((uintptr_t)p % (4 * sizeof(T))) == 0; };
+    const bool vec = R == 4 && ((g.sy | b) & 3) == 0 && (g.sx & 3) == 0 && al(PP) && al(w.save) &&
+                     al(w.field) && al(w.restore);
+    const auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(nblocks(n)), dim3(kThreads), 0, s, PP, taper, g, b, u,
+                           w.save, w.field, w.restore, r, q, img, ps);
+        return hipGetLastError();
+    };
+    switch (R) {
+    case 4: return vec ? go(k_tail_upper<T, 4, true>) : go(k_tail_upper<T, 4, false>);
+    case 3: return go(k_tail_upper<T, 3, false>);
+    case 2: return go(k_tail_upper<T, 2, false>);
+    case 1: return go(k_tail_upper<T, 1, false>);
+    default: return hipErrorInvalidValue;
+    }
+}
+
 hipError_t launch_tick(int *p, int d, bool set, hipStream_t s)
 {
     hipLaunchKernelGGL(k_tick, dim3(1), dim3(64), 0, s, p, d, set ? 1 : 0);
@@ -1397,6 +1693,13 @@ hipError_t launch_tick(int *p, int d, bool set, hipStream_t s)
 }
 
 #define RTM_INSTANTIATE_OPS(T)                                                                \
+    template hipError_t launch_tail_all<T>(T *, const float *, const Grid &, int, int, int,     \
+                                           const TailReceivers *, const TailSource *,           \
+                                           hipStream_t);                                        \
+    template hipError_t launch_tail_upper<T>(T *, const float *, const Grid &, int, int,        \
+                                             const TailLayer<T> &, const TailReceivers *,       \
+                                             const TailSource *, float *, const T *,            \
+                                             hipStream_t);                                      \
     template hipError_t launch_taper<T>(T *, const float *, const Grid &, int, bool,            \
                                         hipStream_t);                                           \
     template hipError_t launch_taper_all2<T>(T *, T *, const float *, const Grid &, int,        \
@@ -1407,10 +1710,6 @@ hipError_t launch_tick(int *p, int d, bool set, hipStream_t s)
                                               hipStream_t, int);                                \
     template hipError_t launch_taper_frame_all<T>(T *, const float *, const Grid &, int, int,   \
                                                   int, hipStream_t);                            \
-    template hipError_t launch_taper_frame_xy<T>(T *, const float *, const Grid &, int, int,    \
-                                                 int, hipStream_t);                             \
-    template hipError_t launch_taper_quirk_out<T>(T *, const float *, const Grid &, int,        \
-                                                  hipStream_t);                                 \
     template hipError_t launch_source<T>(T *, long long, const float *, int, float, hipStream_t); \
     template hipError_t launch_receivers<T>(T *, float *, const Grid &, int, int, int, int, int, \
                                             int, int, int, int, bool, hipStream_t);             \
@@ -1419,8 +1718,6 @@ hipError_t launch_tick(int *p, int d, bool set, hipStream_t s)
                                                   const T *, int, int, int, hipStream_t);       \
     template hipError_t launch_upb<T>(T *, T *, const Grid &, int, int, long long, bool,        \
                                       hipStream_t);                                             \
-    template hipError_t launch_upb_save_taper<T>(T *, T *, const float *, const Grid &, int,    \
-                                                 int, long long, hipStream_t);                  \
     template hipError_t launch_image<T>(float *, const T *, const T *, const Grid &, int, int,  \
                                         hipStream_t);                                           \
     template hipError_t launch_tail_fwd<T>(const BatchShot *, int, int, int, const float *,    \
