@@ -117,96 +117,6 @@ __global__ void __launch_bounds__(kGemmThreads) k_gemm(AeGemm p)
             }
 }
 
-// dY = Y - X (the gradient of 0.5 * sum (Y - X)^2), loss += sum (Y - X)^2.
-__global__ void __launch_bounds__(256)
-    k_ae_residual(const float *__restrict__ Y, const _Float16 *__restrict__ X,
-                  float *__restrict__ dY, long long n, float *__restrict__ loss)
-{
-    __shared__ float red[256];
-    float s = 0.f;
-    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n;
-         i += (long long)gridDim.x * 256) {
-        const float d = Y[i] - (float)X[i];
-        dY[i] = d;
-        s += d * d;
-    }
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int h = 128; h > 0; h >>= 1) {
-        if ((int)threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) atomicAdd(loss, red[0]);
-}
-
-// dA = dH * (1 - H^2): back through tanh, in place.
-__global__ void __launch_bounds__(256)
-    k_tanh_back(float *__restrict__ dH, const float *__restrict__ H, long long n)
-{
-    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n;
-         i += (long long)gridDim.x * 256)
-        dH[i] = dH[i] * (1.0f - H[i] * H[i]);
-}
-
-// db[c] += sum over rows of D[row][c] (rows x cols, row-major; cols divides
-// 256 or is a multiple of 256).  A block walks its row range in row-major
-// order, so every load is coalesced; thread t keeps the partial sums of the
-// columns t, t + 256, ... (or of column t % cols), then one block reduction.
-__global__ void __launch_bounds__(256)
-    k_colsum(const float *__restrict__ D, long long rows, int cols, float *__restrict__ db,
-             long long rows_per_block)
-{
-    __shared__ float red[256];
-    const long long r0 = (long long)blockIdx.x * rows_per_block;
-    const long long r1 = min(rows, r0 + rows_per_block);
-    const long long e0 = r0 * cols, e1 = r1 * cols;
-    const int t = threadIdx.x;
-    if (cols <= 256) {
-        float acc = 0.f;
-        for (long long e = e0 + t; e < e1; e += 256) acc += D[e];
-        red[t] = acc;
-        __syncthreads();
-        if (t < cols) {
-            float s = 0.f;
-            for (int k = t; k < 256; k += cols) s += red[k];
-            atomicAdd(&db[t], s);
-        }
-    } else {
-        for (int c = t; c < cols; c += 256) {
-            float acc = 0.f;
-            for (long long e = e0 + c; e < e1; e += cols) acc += D[e];
-            atomicAdd(&db[c], acc);
-        }
-    }
-}
-
-// Adam (Kingma & Ba 2015) with bias correction folded into the step size.
-__global__ void __launch_bounds__(256)
-    k_adam(float *__restrict__ w, const float *__restrict__ g, float *__restrict__ m,
-           float *__restrict__ v, int n, float lr_t, float b1, float b2, float eps)
-{
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const float gi = g[i];
-    const float mi = b1 * m[i] + (1.0f - b1) * gi;
-    const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    w[i] = w[i] - lr_t * mi / (sqrtf(vi) + eps);
-}
-
-__global__ void __launch_bounds__(256)
-    k_gather_bricks(const _Float16 *__restrict__ src, const int *__restrict__ idx,
-                    _Float16 *__restrict__ dst, int n)
-{
-    const long long total = (long long)n * kBrick;
-    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < total;
-         i += (long long)gridDim.x * 256) {
-        const long long b = i / kBrick, e = i % kBrick;
-        dst[i] = src[(long long)idx[b] * kBrick + e];
-    }
-}
-
 // One block per brick: scale = max |v| over the brick's in-grid cells, then
 // the FP16 values v * (1 / scale) (zero outside the grid, and the whole
 // brick zero with scale 0 when max |v| is zero or subnormal).
@@ -477,17 +387,398 @@ __global__ void __launch_bounds__(kAeThreads)
     }
 }
 
+// Gradient of 0.5 * sum (Y - X)^2, forward and backward of one batch in one
+// launch.  A tile is 16 rows a of the middle layers, as in k_ae_encode; the
+// block's 8 waves take 64 of the 512 elements of a row each (q = 2 w, 2 w + 1),
+// so everything between the two sums over all elements (z and dz, through LDS)
+// stays in a wave: lane j + 16 g holds row j, elements 32 q + 16 t + 4 g + v.
+// The products over elements run transposed as there; the products over rows
+// (weight gradients) read their FP16 operands from LDS row-transposed, 16 rows
+// to one 16x16x16 product, and accumulate in registers over the block's tiles;
+// for the 8 x 8 layers the diagonal blocks of a 16 x 16 product are two
+// patches.  A block writes its partial gradient and squared error to a slab of
+// its own, k_ae_update adds the slabs.  Rounding as in separate GEMM launches:
+// FP16 operands, FP32 sums, FP32 between layers.
+//
+// Bound by the slabs (134 KB per block written and read back) and by latency:
+// one tile per block at 64 bricks (256 blocks).  One step on 64 bricks: 0.040 ms
+// and 0.007 of k_ae_update; as 11 GEMM launches of 0.035 ms with every layer in
+// memory, column sums and elementwise passes 0.50 ms.
+constexpr int kSlabFloats = (int)kOffB4 + 8 + 16;  // parameters, then the loss; padded
+constexpr int kLossAt = (int)kOffB4 + 8;
+constexpr int kTrainBlocks = 256;  // one per CU: slabs stay few
+constexpr int kRowPad = 20;        // LDS row of 16 row values (halves)
+
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+__global__ void __launch_bounds__(kAeThreads)
+    k_ae_gradient(const _Float16 *__restrict__ X, const int *__restrict__ idx, int tiles,
+                  const float *__restrict__ w, float *__restrict__ slabs)
+{
+    constexpr int NW = kAeThreads / 64;
+    static_assert(NW == 8);
+    __shared__ float zred[NW][8][64], dzred[NW][8][64];
+    __shared__ __align__(16) _Float16 tr[NW][32 + 64 + 64][kRowPad];
+    const int tid = threadIdx.x, lane = tid & 63, j = lane & 15, g = lane >> 4;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    _Float16(*tc)[kRowPad] = tr[wv], (*ta)[kRowPad] = tr[wv] + 32, (*tb)[kRowPad] = tr[wv] + 96;
+    const float4_t zero = {0.f, 0.f, 0.f, 0.f};
+    // element (slot s of lane group g) in the k order of a product's result
+    auto kel = [&](int s) { return (s & 3) + 4 * g + 16 * (s >> 2); };
+    auto half8 = [](const float(&v)[2][4]) {
+        half8_t h;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) h[4 * t + i] = wst<_Float16>(v[t][i]);
+        return h;
+    };
+    // 32 elements of the lane's row into LDS, element-major
+    auto put = [&](_Float16(*dst)[kRowPad], const half8_t &h) {
+#pragma unroll
+        for (int s = 0; s < 8; ++s) dst[kel(s)][j] = h[s];
+    };
+    // operand of a product over the 16 rows: elements i0 + j, rows 4 g + s
+    auto get = [&](const _Float16(*src)[kRowPad], int i0) {
+        return *reinterpret_cast<const half4_t *>(&src[i0 + j][4 * g]);
+    };
+    float4_t gw2[4][2], gw3[2][4], gw1 = zero, gw4 = zero;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) gw2[i][t] = gw3[t][i] = zero;
+    float gb1[4] = {}, gb4[4] = {}, gb2[2][4] = {}, gb3[2][2][4] = {}, loss = 0.f;
+
+    for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        // the weights are read anew for each tile (L2): the accumulators leave
+        // no registers to keep them
+        int again = 0;
+        asm volatile("" : "+s"(again));
+        const float *wt = w + again;
+        const long long brick = idx ? idx[tile >> 2] : tile >> 2;
+        const _Float16 *x = X + brick * kBrick + ((tile & 3) * 16 + j) * 512 + wv * 64;
+        // ---- forward ----
+        float h1[2][2][4], z[2][4];
+        half8_t xd[2];  // x in the products' result order
+        {
+            float4_t acc[2] = {zero, zero};
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const half8_t xb = *reinterpret_cast<const half8_any *>(x + q * 32 + g * 8);
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const half4_t u =
+                        *reinterpret_cast<const half4_any *>(x + q * 32 + 16 * t + 4 * g);
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) xd[q][4 * t + v] = u[v];
+                }
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const int o = 16 * t + j;  // row: patch o / 8, channel o % 8
+                    half8_t a;
+#pragma unroll
+                    for (int s = 0; s < 8; ++s)
+                        a[s] = (o >> 3) == g ? (_Float16)wt[kOffW1 + s * 8 + (o & 7)]
+                                             : (_Float16)0.f;
+                    const float4_t d = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, xb, zero, 0, 0, 0);
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        h1[q][t][v] = tanhf(d[v] + wt[kOffB1 + ((4 * g + v) & 7)]);
+                }
+                const half8_t h = half8(h1[q]);
+                const float *w2 = wt + kOffW2 + (wv * 64 + q * 32) * 32 + j;
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    half8_t a;
+#pragma unroll
+                    for (int s = 0; s < 8; ++s) a[s] = (_Float16)w2[kel(s) * 32 + 16 * t];
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, h, acc[t], 0, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) zred[wv][4 * t + v][lane] = acc[t][v];
+            __syncthreads();
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    float sum = 0.f;
+#pragma unroll
+                    for (int k = 0; k < NW; ++k) sum += zred[k][4 * t + v][lane];
+                    z[t][v] = sum + wt[kOffB2 + 16 * t + 4 * g + v];
+                }
+        }
+        const half8_t zh = half8(z);
+        wave_lds_fence();  // the previous tile's reads of tc, ta, tb
+        put(tc, zh);
+        float d3[2][2][4];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            float h3[2][4], dy[2][4];
+            const float *w3 = wt + kOffW3 + wv * 64 + q * 32 + j;
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                half8_t a;
+#pragma unroll
+                for (int s = 0; s < 8; ++s) a[s] = (_Float16)w3[kel(s) * 512 + 16 * t];
+                const float4_t d = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, zh, zero, 0, 0, 0);
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    h3[t][v] = tanhf(d[v] + wt[kOffB3 + wv * 64 + q * 32 + 16 * t + 4 * g + v]);
+            }
+            const half8_t h3h = half8(h3);
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const int o = 16 * t + j;
+                half8_t a;
+#pragma unroll
+                for (int s = 0; s < 8; ++s)
+                    a[s] = (o >> 3) == (kel(s) >> 3)
+                               ? (_Float16)wt[kOffW4 + (kel(s) & 7) * 8 + (o & 7)]
+                               : (_Float16)0.f;
+                const float4_t d = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, h3h, zero, 0, 0, 0);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    dy[t][v] = d[v] + wt[kOffB4 + ((4 * g + v) & 7)] - (float)xd[q][4 * t + v];
+                    loss += dy[t][v] * dy[t][v];
+                    gb4[v] += dy[t][v];
+                }
+            }
+            // ---- backward ----
+            const half8_t dyh = half8(dy);
+            put(ta + 32 * q, h3h);
+            put(tb + 32 * q, dyh);
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const int o = 16 * t + j;
+                half8_t a;
+#pragma unroll
+                for (int s = 0; s < 8; ++s)
+                    a[s] = (o >> 3) == (kel(s) >> 3)
+                               ? (_Float16)wt[kOffW4 + (o & 7) * 8 + (kel(s) & 7)]
+                               : (_Float16)0.f;
+                const float4_t d = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, dyh, zero, 0, 0, 0);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    d3[q][t][v] = d[v] * (1.0f - h3[t][v] * h3[t][v]);
+                    gb3[q][t][v] += d3[q][t][v];
+                }
+            }
+        }
+        wave_lds_fence();
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            gw4 = __builtin_amdgcn_mfma_f32_16x16x16f16(get(ta, 16 * i), get(tb, 16 * i), gw4, 0,
+                                                        0, 0);
+        wave_lds_fence();
+        float dz[2][4];
+        {
+            float4_t acc[2] = {zero, zero};
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const half8_t d3h = half8(d3[q]);
+                put(ta + 32 * q, d3h);
+                put(tb + 32 * q, half8(h1[q]));
+                const float *w3 = wt + kOffW3 + j * 512 + wv * 64 + q * 32 + 4 * g;
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    half8_t a;
+#pragma unroll
+                    for (int s = 0; s < 8; ++s)
+                        a[s] = (_Float16)w3[16 * t * 512 + 16 * (s >> 2) + (s & 3)];
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, d3h, acc[t], 0, 0, 0);
+                }
+            }
+            wave_lds_fence();
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    gw3[t][i] = __builtin_amdgcn_mfma_f32_16x16x16f16(
+                        get(tc, 16 * t), get(ta, 16 * i), gw3[t][i], 0, 0, 0);
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) dzred[wv][4 * t + v][lane] = acc[t][v];
+            __syncthreads();
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    float sum = 0.f;
+#pragma unroll
+                    for (int k = 0; k < NW; ++k) sum += dzred[k][4 * t + v][lane];
+                    dz[t][v] = sum;
+                    gb2[t][v] += sum;
+                }
+        }
+        const half8_t dzh = half8(dz);
+        put(tc, dzh);
+        wave_lds_fence();
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+                gw2[i][t] = __builtin_amdgcn_mfma_f32_16x16x16f16(
+                    get(tb, 16 * i), get(tc, 16 * t), gw2[i][t], 0, 0, 0);
+        wave_lds_fence();
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            float d1[2][4];
+            const float *w2 = wt + kOffW2 + (wv * 64 + q * 32 + j) * 32 + 4 * g;
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                half8_t a;
+#pragma unroll
+                for (int s = 0; s < 8; ++s)
+                    a[s] = (_Float16)w2[16 * t * 32 + 16 * (s >> 2) + (s & 3)];
+                const float4_t d = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, dzh, zero, 0, 0, 0);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    d1[t][v] = d[v] * (1.0f - h1[q][t][v] * h1[q][t][v]);
+                    gb1[v] += d1[t][v];
+                }
+            }
+            put(ta + 32 * q, xd[q]);
+            put(tb + 32 * q, half8(d1));
+        }
+        wave_lds_fence();
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            gw1 = __builtin_amdgcn_mfma_f32_16x16x16f16(get(ta, 16 * i), get(tb, 16 * i), gw1, 0,
+                                                        0, 0);
+    }
+
+    // ---- the block's slab ----
+    float *out = slabs + (long long)blockIdx.x * kSlabFloats;
+    // result (i, j) of a 16 x 16 product: lane j + 16 (i / 4), item i % 4
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                out[kOffW2 + (wv * 64 + 16 * i + 4 * g + v) * 32 + 16 * t + j] = gw2[i][t][v];
+                out[kOffW3 + (16 * t + 4 * g + v) * 512 + wv * 64 + 16 * i + j] = gw3[t][i][v];
+            }
+    // sums over the 16 rows (lanes j)
+    auto rows = [&](float v) {
+#pragma unroll
+        for (int d = 8; d > 0; d >>= 1) v += __shfl_xor(v, d, 64);
+        return v;
+    };
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const float b = rows(gb3[q][t][v]);
+                if (j == 0) out[kOffB3 + wv * 64 + q * 32 + 16 * t + 4 * g + v] = b;
+            }
+    if (wv == 0) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const float b = rows(gb2[t][v]);
+                if (j == 0) out[kOffB2 + 16 * t + 4 * g + v] = b;
+            }
+    }
+    // over the waves: the 8 x 8 layers (two diagonal blocks each), their
+    // biases (lane groups g and g + 2 hold the same channels) and the loss
+    __syncthreads();
+    float(*red)[8][64] = zred;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        red[wv][v][lane] = gw1[v];
+        red[wv][4 + v][lane] = gw4[v];
+    }
+    float(*redb)[8][64] = dzred;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        redb[wv][v][lane] = rows(gb1[v]);
+        redb[wv][4 + v][lane] = rows(gb4[v]);
+    }
+    __syncthreads();
+    // 64 + 64 weights, 8 + 8 biases
+    if (tid < 144) {
+        const bool second = tid >= 128 ? tid >= 136 : tid >= 64;  // layer 4
+        float sum = 0.f;
+        if (tid < 128) {
+            const int c = (tid & 63) >> 3, o = tid & 7;
+#pragma unroll
+            for (int p = 0; p < 2; ++p) {
+                const int i = 8 * p + c, l = 8 * p + o + 16 * (i >> 2);
+                for (int k = 0; k < NW; ++k) sum += red[k][(second ? 4 : 0) + (i & 3)][l];
+            }
+            out[(second ? kOffW4 : kOffW1) + c * 8 + o] = sum;
+        } else {
+            const int o = tid & 7;
+#pragma unroll
+            for (int p = 0; p < 2; ++p)
+                for (int k = 0; k < NW; ++k)
+                    sum += redb[k][(second ? 4 : 0) + (o & 3)][16 * (2 * p + (o >> 2))];
+            out[(second ? kOffB4 : kOffB1) + o] = sum;
+        }
+    }
+    loss = rows(loss);
+#pragma unroll
+    for (int d = 16; d < 64; d <<= 1) loss += __shfl_xor(loss, d, 64);
+    __syncthreads();
+    if (lane == 0) red[0][0][wv] = loss;
+    __syncthreads();
+    if (tid == 0) {
+        float sum = 0.f;
+        for (int k = 0; k < NW; ++k) sum += red[0][0][k];
+        out[kLossAt] = sum;
+    }
+}
+
+// The gradient and the loss as sums of the slabs, in their order, then with w
+// one step of Adam (Kingma & Ba 2015), bias correction folded into the step
+// size.  A block takes 64 parameters, 4 threads each.
+__global__ void __launch_bounds__(256)
+    k_ae_update(const float *__restrict__ slabs, int nslabs, float *__restrict__ grad,
+                float *__restrict__ loss, float *__restrict__ w, float *__restrict__ m,
+                float *__restrict__ v, float lr_t, float b1, float b2, float eps)
+{
+    __shared__ float red[4][64];
+    const int lane = threadIdx.x & 63, part = threadIdx.x >> 6;
+    const int i = blockIdx.x * 64 + lane;
+    float sum = 0.f;
+    if (i <= kLossAt) {
+#pragma unroll 8
+        for (int k = part; k < nslabs; k += 4) sum += slabs[(long long)k * kSlabFloats + i];
+    }
+    red[part][lane] = sum;
+    __syncthreads();
+    if (part != 0 || i > kLossAt) return;
+    const float gi = red[0][lane] + red[1][lane] + red[2][lane] + red[3][lane];
+    if (i == kLossAt) {
+        *loss = gi;
+        return;
+    }
+    grad[i] = gi;
+    if (!w) return;
+    const float mi = b1 * m[i] + (1.0f - b1) * gi;
+    const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
+    m[i] = mi;
+    v[i] = vi;
+    w[i] = w[i] - lr_t * mi / (sqrtf(vi) + eps);
+}
+
 // The region's z runs of n cells (n a power of two) are aligned in F.
 inline bool runs_aligned(const float *F, const Grid &g, const AeRegion &r, int n)
 {
     return ((uintptr_t)F & (4 * n - 1)) == 0 && (g.sx & (n - 1)) == 0 && (g.sy & (n - 1)) == 0 &&
            (r.z0 & (n - 1)) == 0;
-}
-
-inline unsigned grid_for(long long n)
-{
-    long long b = (n + 255) / 256;
-    return (unsigned)(b > 16384 ? 16384 : (b ? b : 1));
 }
 
 }  // namespace
@@ -516,45 +807,28 @@ hipError_t launch_ae_gemm(const AeGemm &p, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t launch_ae_residual(const float *Y, const void *X, float *dY, long long n, float *loss,
-                              hipStream_t s)
+size_t ae_gradient_floats(int n)
 {
-    // at most 1024 blocks: one atomic per block on the single loss word
-    hipLaunchKernelGGL(k_ae_residual, dim3(std::min(1024u, grid_for(n))), dim3(256), 0, s, Y,
-                       static_cast<const _Float16 *>(X), dY, n, loss);
+    return (size_t)std::min(4 * n, kTrainBlocks) * kSlabFloats;
+}
+
+hipError_t launch_ae_gradient(const void *bricks, const int *idx, int n, const float *w,
+                              float *slabs, hipStream_t s)
+{
+    if (n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_ae_gradient, dim3((unsigned)std::min(4 * n, kTrainBlocks)),
+                       dim3(kAeThreads), 0, s, static_cast<const _Float16 *>(bricks), idx, 4 * n,
+                       w, slabs);
     return hipGetLastError();
 }
 
-hipError_t launch_tanh_back(float *dH, const float *H, long long n, hipStream_t s)
+hipError_t launch_ae_update(const float *slabs, int n, float *grad, float *loss, float *w,
+                            float *m, float *v, float lr_t, float b1, float b2, float eps,
+                            hipStream_t s)
 {
-    hipLaunchKernelGGL(k_tanh_back, dim3(grid_for(n)), dim3(256), 0, s, dH, H, n);
-    return hipGetLastError();
-}
-
-hipError_t launch_colsum(const float *D, long long rows, int cols, float *db, hipStream_t s)
-{
-    if (cols <= 0 || rows <= 0) return hipSuccess;
-    if (!(cols <= 256 ? 256 % cols == 0 : cols % 256 == 0)) return hipErrorInvalidValue;
-    // about 16K elements per block
-    const long long rpb = std::max(1LL, 16384LL / cols);
-    const long long nb = (rows + rpb - 1) / rpb;
-    if (nb > 0x7fffffffLL) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_colsum, dim3((unsigned)nb), dim3(256), 0, s, D, rows, cols, db, rpb);
-    return hipGetLastError();
-}
-
-hipError_t launch_adam(float *w, const float *g, float *m, float *v, int n, float lr_t, float b1,
-                       float b2, float eps, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_adam, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, w, g, m, v, n,
-                       lr_t, b1, b2, eps);
-    return hipGetLastError();
-}
-
-hipError_t launch_gather_bricks(const void *src, const int *idx, void *dst, int n, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_gather_bricks, dim3(grid_for((long long)n * kBrick)), dim3(256), 0, s,
-                       static_cast<const _Float16 *>(src), idx, static_cast<_Float16 *>(dst), n);
+    if (n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_ae_update, dim3((unsigned)(kLossAt / 64 + 1)), dim3(256), 0, s, slabs,
+                       std::min(4 * n, kTrainBlocks), grad, loss, w, m, v, lr_t, b1, b2, eps);
     return hipGetLastError();
 }
 
@@ -565,8 +839,8 @@ hipError_t launch_bricks(const float *F, const Grid &g, const AeRegion &r, void 
     if (nb <= 0) return hipSuccess;
     if (nb > 0x7fffffffLL) return hipErrorInvalidValue;
     const bool pairs = runs_aligned(F, g, r, 2) && (r.z1 & 1) == 0;
-    hipLaunchKernelGGL(pairs ? k_bricks<true> : k_bricks<false>, dim3((unsigned)nb), dim3(kCutThreads), 0, s, F, g, r,
-                       static_cast<_Float16 *>(out), scales);
+    hipLaunchKernelGGL(pairs ? k_bricks<true> : k_bricks<false>, dim3((unsigned)nb),
+                       dim3(kCutThreads), 0, s, F, g, r, static_cast<_Float16 *>(out), scales);
     return hipGetLastError();
 }
 

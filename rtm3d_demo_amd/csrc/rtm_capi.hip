@@ -2130,11 +2130,9 @@ int rtmhip_batch_steps_noalloc(rtmhip_batch_shot *shots, int nshots, const float
 namespace {
 
 struct AeLayerDef {
-    int K, N, act;      // weights [K][N] row-major, then the bias [N]
-    long long rows;     // GEMM rows per brick
+    int K, N;  // weights [K][N] row-major, then the bias [N]
 };
-constexpr AeLayerDef kAe[4] = {{8, 8, 1, 4096}, {512, 32, 0, 64}, {32, 512, 1, 64},
-                               {8, 8, 0, 4096}};
+constexpr AeLayerDef kAe[4] = {{8, 8}, {512, 32}, {32, 512}, {8, 8}};
 constexpr long long kBrickCells = 32768, kCodes = 2048;
 
 long long ae_param_offset(int layer)
@@ -2150,108 +2148,12 @@ constexpr long long kAeParams = 8 * 8 + 8 + 512 * 32 + 32 + 32 * 512 + 512 + 8 *
 struct rtmhip_ae {
     int maxb = 0;
     float *w = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;  // kAeParams each
-    void *x0 = nullptr;     // FP16 input bricks [maxb][32768]
-    float *h1 = nullptr, *z = nullptr, *h3 = nullptr, *y = nullptr;
-    float *d1 = nullptr, *dz = nullptr, *d3 = nullptr, *dy = nullptr;
-    float *loss = nullptr;  // device accumulator
+    float *slabs = nullptr; // the blocks' partial gradients
+    float *loss = nullptr;  // sum of squares
     long long steps = 0;    // Adam steps taken
 };
 
 namespace {
-
-float *ae_w(const rtmhip_ae *a, int l) { return a->w + ae_param_offset(l); }
-float *ae_b(const rtmhip_ae *a, int l) { return ae_w(a, l) + (long long)kAe[l].K * kAe[l].N; }
-float *ae_gw(const rtmhip_ae *a, int l) { return a->g + ae_param_offset(l); }
-float *ae_gb(const rtmhip_ae *a, int l) { return ae_gw(a, l) + (long long)kAe[l].K * kAe[l].N; }
-
-// Row-major GEMM of one layer: out[rows][N] = act(in[rows][K] W + b).
-hipError_t ae_layer(const rtmhip_ae *a, int l, const void *in, int in_half, float *out, int n)
-{
-    AeGemm p{};
-    p.A = in;
-    p.sam = kAe[l].K;
-    p.sak = 1;
-    p.a_half = in_half;
-    p.B = ae_w(a, l);
-    p.sbk = kAe[l].N;
-    p.sbn = 1;
-    p.C = out;
-    p.ldc = kAe[l].N;
-    p.bias = ae_b(a, l);
-    p.M = kAe[l].rows * n;
-    p.N = kAe[l].N;
-    p.K = kAe[l].K;
-    p.act = kAe[l].act;
-    return launch_ae_gemm(p, g_state.stream);
-}
-
-hipError_t ae_forward(const rtmhip_ae *a, const void *x0, int n)
-{
-    hipError_t e;
-    if ((e = ae_layer(a, 0, x0, 1, a->h1, n)) != hipSuccess) return e;
-    if ((e = ae_layer(a, 1, a->h1, 0, a->z, n)) != hipSuccess) return e;
-    if ((e = ae_layer(a, 2, a->z, 0, a->h3, n)) != hipSuccess) return e;
-    return ae_layer(a, 3, a->h3, 0, a->y, n);
-}
-
-// Weight gradient of layer l: gW[K][N] += in^T (rows x K) * d (rows x N);
-// input gradient din[rows][K] = d * W^T (skipped when din is null).
-hipError_t ae_layer_back(const rtmhip_ae *a, int l, const void *in, int in_half, const float *d,
-                         float *din, int n)
-{
-    hipStream_t s = g_state.stream;
-    const long long rows = kAe[l].rows * n;
-    const int K = kAe[l].K, N = kAe[l].N;
-    AeGemm p{};
-    p.A = in;
-    p.sam = 1;
-    p.sak = K;
-    p.a_half = in_half;
-    p.B = d;
-    p.sbk = N;
-    p.sbn = 1;
-    p.C = ae_gw(a, l);
-    p.ldc = N;
-    p.M = K;
-    p.N = N;
-    p.K = rows;
-    p.accumulate = 1;
-    p.kchunk = 0;  // sized by the launcher
-    hipError_t e = launch_ae_gemm(p, s);
-    if (e != hipSuccess) return e;
-    if ((e = launch_colsum(d, rows, N, ae_gb(a, l), s)) != hipSuccess) return e;
-    if (!din) return hipSuccess;
-    AeGemm q{};
-    q.A = d;
-    q.sam = N;
-    q.sak = 1;
-    q.B = ae_w(a, l);  // B(k, n) = W[n][k]
-    q.sbk = 1;
-    q.sbn = N;
-    q.C = din;
-    q.ldc = K;
-    q.M = rows;
-    q.N = K;
-    q.K = N;
-    return launch_ae_gemm(q, s);
-}
-
-// Gradient of 0.5 * sum (Y - X)^2 over n bricks into a->g (zeroed first);
-// the sum of squares is added to *loss (device).
-hipError_t ae_backward(const rtmhip_ae *a, const void *x0, int n, float *loss)
-{
-    hipStream_t s = g_state.stream;
-    const long long cells = kBrickCells * n;
-    hipError_t e;
-    if ((e = launch_fill(a->g, (size_t)kAeParams, 0.f, s)) != hipSuccess) return e;
-    if ((e = launch_ae_residual(a->y, x0, a->dy, cells, loss, s)) != hipSuccess) return e;
-    if ((e = ae_layer_back(a, 3, a->h3, 0, a->dy, a->d3, n)) != hipSuccess) return e;
-    if ((e = launch_tanh_back(a->d3, a->h3, cells, s)) != hipSuccess) return e;
-    if ((e = ae_layer_back(a, 2, a->z, 0, a->d3, a->dz, n)) != hipSuccess) return e;
-    if ((e = ae_layer_back(a, 1, a->h1, 0, a->dz, a->d1, n)) != hipSuccess) return e;
-    if ((e = launch_tanh_back(a->d1, a->h1, cells, s)) != hipSuccess) return e;
-    return ae_layer_back(a, 0, x0, 1, a->d1, nullptr, n);
-}
 
 uint64_t splitmix64(uint64_t &x)
 {
@@ -2340,18 +2242,13 @@ int rtmhip_ae_create(rtmhip_ae **out, int max_bricks, unsigned long long seed)
         return fail(RTMHIP_ERR_INVALID, "max_bricks %d not in 1..4096", max_bricks);
     auto a = std::make_unique<rtmhip_ae>();
     a->maxb = max_bricks;
-    const long long cells = kBrickCells * max_bricks, codes = kCodes * max_bricks;
     struct Alloc {
         void **p;
         size_t bytes;
     } allocs[] = {
         {(void **)&a->w, kAeParams * 4}, {(void **)&a->g, kAeParams * 4},
         {(void **)&a->m, kAeParams * 4}, {(void **)&a->v, kAeParams * 4},
-        {&a->x0, (size_t)cells * 2},     {(void **)&a->h1, (size_t)cells * 4},
-        {(void **)&a->z, (size_t)codes * 4}, {(void **)&a->h3, (size_t)cells * 4},
-        {(void **)&a->y, (size_t)cells * 4}, {(void **)&a->d1, (size_t)cells * 4},
-        {(void **)&a->dz, (size_t)codes * 4}, {(void **)&a->d3, (size_t)cells * 4},
-        {(void **)&a->dy, (size_t)cells * 4}, {(void **)&a->loss, 4},
+        {(void **)&a->slabs, ae_gradient_floats(max_bricks) * 4}, {(void **)&a->loss, 4},
     };
     for (auto &al : allocs) {
         hipError_t e = hipMalloc(al.p, al.bytes);
@@ -2387,8 +2284,7 @@ int rtmhip_ae_destroy(rtmhip_ae *a)
 {
     if (!a) return RTMHIP_OK;
     if (g_state.init) (void)hipStreamSynchronize(g_state.stream);
-    void *ps[] = {a->w, a->g, a->m, a->v, a->x0, a->h1, a->z, a->h3,
-                  a->y, a->d1, a->dz, a->d3, a->dy, a->loss};
+    void *ps[] = {a->w, a->g, a->m, a->v, a->slabs, a->loss};
     for (void *p : ps)
         if (p) (void)hipFree(p);
     delete a;
@@ -2421,9 +2317,11 @@ int rtmhip_ae_gradient(rtmhip_ae *a, const void *bricks, int n, float *loss)
     NEED_INIT();
     if (!a || !bricks || !loss) return fail(RTMHIP_ERR_INVALID, "NULL pointer");
     if (n <= 0 || n > a->maxb) return fail(RTMHIP_ERR_INVALID, "n %d not in 1..%d", n, a->maxb);
-    HIPCHK(launch_fill(a->loss, 1, 0.f, g_state.stream), "fill");
-    HIPCHK(ae_forward(a, bricks, n), "autoencoder forward");
-    HIPCHK(ae_backward(a, bricks, n, a->loss), "autoencoder backward");
+    HIPCHK(launch_ae_gradient(bricks, nullptr, n, a->w, a->slabs, g_state.stream),
+           "autoencoder gradient");
+    HIPCHK(launch_ae_update(a->slabs, n, a->g, a->loss, nullptr, nullptr, nullptr, 0.f, 0.f, 0.f,
+                            0.f, g_state.stream),
+           "autoencoder gradient");
     HIPCHK(hipMemcpyAsync(loss, a->loss, 4, hipMemcpyDeviceToHost, g_state.stream), "copy");
     HIPCHK(hipStreamSynchronize(g_state.stream), "hipStreamSynchronize");
     *loss *= 0.5f;
@@ -2463,17 +2361,15 @@ int rtmhip_ae_train(rtmhip_ae *a, const void *bricks, int nbricks, int iters, in
     if (e == hipSuccess)
         e = hipMemcpyAsync(didx, picks.data(), sizeof(int) * picks.size(), hipMemcpyHostToDevice,
                            s);
-    if (e == hipSuccess) e = launch_fill(dl, (size_t)iters, 0.f, s);
     for (int it = 0; it < iters && e == hipSuccess; ++it) {
-        e = launch_gather_bricks(bricks, didx + (size_t)it * batch, a->x0, batch, s);
-        if (e == hipSuccess) e = ae_forward(a, a->x0, batch);
-        if (e == hipSuccess) e = ae_backward(a, a->x0, batch, dl + it);
+        e = launch_ae_gradient(bricks, didx + (size_t)it * batch, batch, a->w, a->slabs, s);
         a->steps++;
         const double c1 = 1.0 - std::pow((double)b1, (double)a->steps);
         const double c2 = 1.0 - std::pow((double)b2, (double)a->steps);
         const float lr_t = (float)(lr * std::sqrt(c2) / c1);
         if (e == hipSuccess)
-            e = launch_adam(a->w, a->g, a->m, a->v, (int)kAeParams, lr_t, b1, b2, eps, s);
+            e = launch_ae_update(a->slabs, batch, a->g, dl + it, a->w, a->m, a->v, lr_t, b1, b2,
+                                 eps, s);
     }
     std::vector<float> lhost(iters);
     if (e == hipSuccess)

@@ -284,13 +284,16 @@ struct AeRegion {
     int nbx, nby, nbz;
 };
 hipError_t launch_ae_gemm(const AeGemm &p, hipStream_t s);
-hipError_t launch_ae_residual(const float *Y, const void *X, float *dY, long long n, float *loss,
-                              hipStream_t s);
-hipError_t launch_tanh_back(float *dH, const float *H, long long n, hipStream_t s);
-hipError_t launch_colsum(const float *D, long long rows, int cols, float *db, hipStream_t s);
-hipError_t launch_adam(float *w, const float *g, float *m, float *v, int n, float lr_t, float b1,
-                       float b2, float eps, hipStream_t s);
-hipError_t launch_gather_bricks(const void *src, const int *idx, void *dst, int n, hipStream_t s);
+// Gradient of 0.5 * sum (Y - X)^2 over n bricks (idx: their numbers in
+// `bricks`, or null: the first n): partial sums into ae_gradient_floats(n)
+// floats, which launch_ae_update adds into grad and *loss (the sum of squares);
+// with w it then takes one Adam step.
+size_t ae_gradient_floats(int n);
+hipError_t launch_ae_gradient(const void *bricks, const int *idx, int n, const float *w,
+                              float *slabs, hipStream_t s);
+hipError_t launch_ae_update(const float *slabs, int n, float *grad, float *loss, float *w,
+                            float *m, float *v, float lr_t, float b1, float b2, float eps,
+                            hipStream_t s);
 hipError_t launch_bricks(const float *F, const Grid &g, const AeRegion &r, void *out,
                          float *scales, hipStream_t s);
 // Inference over n bricks in one launch (w: the flat parameters): FP16 bricks

@@ -192,6 +192,34 @@ def test_gradient_codes_and_decode_match_oracle(gpu):
         d.free()
 
 
+@pytest.mark.parametrize("n", [1, 63, 65, 130])
+def test_gradient_over_tiles(gpu, n):
+    """Blocks of none, one and several tiles (256 blocks, 4 tiles a brick), all
+    four quarters of a brick.  Bounds as above: FP16 operands' rounding."""
+    from rtm3d_demo_amd import ae
+    rng = np.random.default_rng(n)
+    B = np.clip(0.4 * rng.standard_normal((n, ae.BRICK)), -1, 1).astype(np.float16)
+    codec = ae.Codec(max_bricks=n, seed=3)
+    p = codec.params().astype(np.float64)
+    p += rng.uniform(-0.05, 0.05, p.shape)
+    codec.set_params(p.astype(np.float32))
+    dB = gpu.DeviceArray.from_host(B.view(np.uint16), np.uint16)
+    loss, g = codec.gradient(dB, n)
+    want_loss, want_g = ao.loss_and_grad(codec.params().astype(np.float64), B.astype(np.float64))
+    assert abs(loss - want_loss) <= 2e-3 * want_loss
+    o = 0
+    for li, (k, nn, _, _) in enumerate(ao.LAYERS):
+        for name, size in (("W", k * nn), ("b", nn)):
+            e = _rel(g[o:o + size], want_g[o:o + size])
+            print("layer %d %s gradient rel-L2 %.2e" % (li + 1, name, e), flush=True)
+            assert e < 2e-2, (li, name, e)
+            o += size
+    again = codec.gradient(dB, n)
+    assert again[0] == loss and np.array_equal(again[1], g)  # no atomics
+    codec.destroy()
+    dB.free()
+
+
 def _salt_case(gpu, seed_src):
     from rtm3d_demo_amd import host, workloads
     vel = workloads.salt_model(64, 64, 64, seed=2024)
