@@ -68,24 +68,24 @@ bool slab_fits(int radius, const Grid &g, const ImageFuse *fuse, const TaperFuse
             return false;
         if (taper->all == 3 && (taper->hold < 0 || taper->hold > taper->b)) return false;
     }
-    // A plane step takes 2.7-3.0 us (4.6-5.1 with imaging) whatever the row
-    // length; the waves of rtm_stencil.hip take 3.1-3.4 us (6.0-6.7) per
+    // A plane step takes 2.2-2.5 us (3.9-4.6 with imaging) whatever the row
+    // length; the waves of rtm_stencil.hip take 2.6-3.4 us (4.6-6.7) per
     // million cells, more where rows fill their tiles badly -- where part of
-    // this kernel's lanes idle too.  Measured, us, this kernel / the best
-    // waves or rows (plain; imaging): 592 x 592 x 336 374 / 403; 627 / 713,
-    // 336^3 125 / 134; 225 / 249, 302 x 278 x 256 64 / 65; 111 / 143,
-    // 880 x 880 x 480 1142 / 1260; 1917 / 2419.  Outside the rule: 192^3
-    // 29 / 24; 50 / 41, 300 x 300 x 272 91 / 85, 640 x 300 x 140 131 / 100,
-    // 301 x 277 x 259 75 / 74; 186 / 164.
+    // this kernel's lanes idle too.  The lines lie between the sizes measured
+    // on either side, us, this kernel / the best waves or rows (steps per
+    // million filled cells).  Plain: 302 x 278 x 256 59.6 / 64.1 (1.12), 240^3
+    // 42.8 / 45.1 (1.331), but 640 x 300 x 140 117 / 102 (1.348), 192^3
+    // 24.8 / 23.6 (1.71).  Imaging: 640 x 300 x 140 189 / 201 (1.348), but 200 x
+    // 180 x 300 72 / 67 (1.47); odd rows 301 x 277 x 259 153 / 169 (1.255), but
+    // 400 x 260 x 161 125 / 120 (1.326).
     const double fill = std::sqrt((double)((g.nz + 127) / 128 * 128) / g.nz);
-    const double line = (fuse && !(g.nz & 1) ? 1.35e-6 : 1.2e-6) * fill;
+    const double line = (!fuse ? 1.335e-6 : (g.nz & 1) ? 1.32e-6 : 1.4e-6) * fill;
     return (double)choose_march(y_tiles(g), g.nx - 8).steps <
            line * (double)g.nx * g.ny * g.nz;
 }
 
 hipError_t launch_slab(const float *P, float *PP, const float *V, const Coefs &cf, const Grid &g,
-                       const ImageFuse *fuse, const TaperFuse *taper, int *flag, hipStream_t s,
-                       const slab::SlabShell *shell)
+                       const ImageFuse *fuse, const TaperFuse *taper, int *flag, hipStream_t s)
 {
     using namespace slab;
     if (!slab_fits(4, g, fuse, taper)) return hipErrorInvalidValue;
@@ -98,23 +98,15 @@ hipError_t launch_slab(const float *P, float *PP, const float *V, const Coefs &c
     }
     const bool tap = taper && taper->b > 0;
     if (tap) tf = *taper;
-    SlabShell sh{};
-    if (shell) sh = *shell;
-    Form form = fuse ? (tap ? kImageOutUpper : kImage)
-                     : (!tap ? kPlain : (tf.all == 2 ? kOut : kOutUpper));
-    if (sh.save || sh.restore) {
-        if (sh.b < 8 || (sh.b & 1)) return hipErrorInvalidValue;
-        if (sh.save && form == kOutUpper) form = kOutUpperSave;
-        else if (sh.restore && form == kPlain) form = kPlainRestore;
-        else return hipErrorInvalidValue;
-    }
+    const Form form = fuse ? (tap ? kImageOutUpper : kImage)
+                           : (!tap ? kPlain : (tf.all == 2 ? kOut : kOutUpper));
     const int nzw = (g.nz + 127) / 128;
     SlabGrid sg;
     sg.nyt = y_tiles(g);
     sg.xchunk = choose_march(sg.nyt, g.nx - 8).chunk;
     sg.nxc = (g.nx - 8 + sg.xchunk - 1) / sg.xchunk;
-    return (g.nz & 1) ? launch_odd(nzw, form, P, PP, V, cf, g, sg, fz, tf, sh, flag, s)
-                      : launch_even(nzw, form, P, PP, V, cf, g, sg, fz, tf, sh, flag, s);
+    return (g.nz & 1) ? launch_odd(nzw, form, P, PP, V, cf, g, sg, fz, tf, flag, s)
+                      : launch_even(nzw, form, P, PP, V, cf, g, sg, fz, tf, flag, s);
 }
 
 }  // namespace rtmhip

@@ -20,14 +20,16 @@
 //     centre rows have been in the ring for R planes): one barrier per plane,
 //     with nothing to wait for behind it.
 // That is 17.0 bytes per cell (FETCH_SIZE + WRITE_SIZE).  Salt grid, 592 x 592
-// x 336, ms, against the best wave or row shape before: plain 0.370 (0.417),
-// upper taper on the output 0.383 (0.431), taper3D on the output 0.406
-// (0.474), imaging with the upper taper 0.613 (0.714); 4.8 TB/s of algorithmic
-// bytes for the plain step.  Halos loaded a plane ahead instead of with the
-// lead: 18.8 bytes per cell, 0.386 ms; cacheable streams: plain 0.376, imaging
-// 0.651; the x ring's 60 registers and the 20 of the waiting halo rows set 3
-// rows per wave (4 rows spill: 0.41-0.43), 12 waves per CU.  It is then bound
-// by about 5 TB/s and 57 % of the VALU issue slots together.
+// x 336, ms, against the best wave or row shape: plain 0.348 (0.417), upper
+// taper on the output 0.351 (0.431), taper3D on the output 0.365 (0.474),
+// imaging 0.595, with the upper taper 0.605 (0.714); 5.1 TB/s of algorithmic
+// bytes for the plain step.  With branches around the loads and stores (see
+// bounded_view) these were 0.373, 0.381, 0.404 and 0.605.  Halos loaded a
+// plane ahead instead of with the lead: 18.8 bytes per cell, 4 % slower;
+// cacheable streams: plain 2 %, imaging 6 % slower.  The x ring's 60 registers
+// and the 20 of the waiting halo rows set 3 rows per wave (4 rows spill),
+// 12 waves per CU.  It is then bound by the 5 to 6 TB/s beyond L2 and nearly as
+// much by the VALU (57 % of its issue slots).
 #pragma once
 #include "rtm_internal.hpp"
 #include "rtm_slab_launch.hpp"
@@ -51,6 +53,18 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t plane_view(const void *p)
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, -1, 0x00020000);
 }
 
+// The same with the plane's size: a store whose lane offset is kDropped is out
+// of range and discarded by the memory unit.  So a plane's step has no branch
+// around a load or a store, and its wait counts are exact: with branches the
+// compiler must assume at every join that the later loads were not issued, and
+// waits for all of them where only PP and V are needed (plain step, salt grid:
+// 0.373 ms with branches, 0.348 without).
+constexpr unsigned kDropped = 0x7ffffff0u;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t bounded_view(void *p, long long cells)
+{
+    return __builtin_amdgcn_make_buffer_rsrc(p, (short)0, (int)(cells * 4), 0x00020000);
+}
+
 // One z pair (8 bytes at 4-byte alignment).
 template <int POLICY = 0>
 __device__ __forceinline__ void ld_pair(__amdgpu_buffer_rsrc_t rs, unsigned soff, unsigned voff,
@@ -62,23 +76,21 @@ __device__ __forceinline__ void ld_pair(__amdgpu_buffer_rsrc_t rs, unsigned soff
     v[0] = __builtin_bit_cast(float, lo);
     v[1] = __builtin_bit_cast(float, hi);
 }
-// The elements of a pair that `on` selects.
 template <int POLICY>
 __device__ __forceinline__ void st_pair(__amdgpu_buffer_rsrc_t rs, unsigned soff, unsigned voff,
-                                        float a, float b, bool on0, bool on1)
+                                        float a, float b)
 {
-    if (on0 && on1) {
-        u32x2 u;
-        u.x = __builtin_bit_cast(unsigned, a);
-        u.y = __builtin_bit_cast(unsigned, b);
-        __builtin_amdgcn_raw_buffer_store_b64(u, rs, (int)voff, (int)soff, POLICY);
-    } else if (on0) {
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, a), rs, (int)voff,
-                                              (int)soff, POLICY);
-    } else if (on1) {
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, b), rs, (int)voff + 4,
-                                              (int)soff, POLICY);
-    }
+    u32x2 u;
+    u.x = __builtin_bit_cast(unsigned, a);
+    u.y = __builtin_bit_cast(unsigned, b);
+    __builtin_amdgcn_raw_buffer_store_b64(u, rs, (int)voff, (int)soff, POLICY);
+}
+template <int POLICY>
+__device__ __forceinline__ void st_one(__amdgpu_buffer_rsrc_t rs, unsigned soff, unsigned voff,
+                                       float a)
+{
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, a), rs, (int)voff,
+                                          (int)soff, POLICY);
 }
 
 __device__ __forceinline__ float uniform(float v)
@@ -97,16 +109,18 @@ __device__ __forceinline__ void lds_barrier()
 
 // IMG: img += ps * pp on z in [z0, z1) off the receiver cells.  TAPER 0 none;
 // 3 taper3D on the output; 4 the upper taper on the output (cells z < b -
-// hold), the centre PP tapered once; with sh.zframe (not with IMG, whose
-// registers are full) the step also tapers PP's z frame (z < R, twice: this step's PP and the next step's P).  HIST 1: the
-// upper-border layer (z in [b - R, b)) of the new values goes to sh.save; 2:
-// the new values of that layer come from sh.restore.  ODD: odd nz (the last
-// pair of a row is half outside; pairs may be updated by halves).
-template <int NZW, int NYW, int RY, bool IMG, int TAPER, bool ODD, int HIST>
+// hold), the centre PP tapered once.  ODD: odd nz (the last pair of a row is
+// half outside; pairs may be updated by halves).
+//
+// The frame taper and the upper-border history stay out of this kernel: its
+// first z wave would do them for the whole block, and the others wait at the
+// barrier (saving the layer and tapering the z frame here: 0.383 -> 0.437 ms,
+// more than the pass of their own takes).
+template <int NZW, int NYW, int RY, bool IMG, int TAPER, bool ODD>
 __global__ void __launch_bounds__(64 * NZW *NYW, 1)
     k_slab(const float *__restrict__ P, float *__restrict__ PP, const float *__restrict__ V,
            const Coefs cf, const Grid g, const SlabGrid sg, const ImageFuse fz,
-           const TaperFuse tf, const SlabShell sh, int *__restrict__ flag)
+           const TaperFuse tf, int *__restrict__ flag)
 {
     constexpr int TY = NYW * RY;
     constexpr int LW = 128 * NZW + 2 * R;  // LDS row: z in [-R, 128 NZW + R)
@@ -163,10 +177,21 @@ __global__ void __launch_bounds__(64 * NZW *NYW, 1)
         fzl[a] = 1.0f;
         if (ztap[a]) fzl[a] = OUT ? lat(za, g.nz) : tab[tf.b - 1 - (z + a)];
     }
-    // cells of the z frame (OUT)
-    const bool zframe[2] = {OUT && z < g.nz && !zcomp, OUT && z + 1 < g.nz && !zcomp1};
+    // lanes that store: every pair with an updated cell (an odd row's last one
+    // writes its other cell back unchanged), with OUT also the z frame's; an
+    // odd row's last cell alone
+    const bool wpair = OUT ? z + 1 < g.nz : zcomp;
+    const bool wone = ODD && OUT && z + 1 == g.nz;
+    // the image: pairs with an imaged cell, the imaged cells, the receivers'
+    const bool ipair = IMG && zcomp && z + 1 >= fz.z0 && z < fz.z1;
+    const bool icell[2] = {IMG && z >= fz.z0 && z < fz.z1,
+                           IMG && zcomp1 && z + 1 >= fz.z0 && z + 1 < fz.z1};
+    const bool rcell[2] = {IMG && z == fz.rz, IMG && z + 1 == fz.rz};
+    // cells whose stored value carries the upper taper
+    const bool ucell[2] = {OUTU && ztap[0] && z < tf.b - tf.hold,
+                           OUTU && ztap[1] && z + 1 < tf.b - tf.hold};
 
-    unsigned rowb[RY], rowh[RY];  // row byte offsets: wavefield, history layer
+    unsigned rowb[RY];
     unsigned ymask = 0, rmask = 0;
     float fyr[RY];
 #pragma unroll
@@ -174,7 +199,6 @@ __global__ void __launch_bounds__(64 * NZW *NYW, 1)
         const int y = y0 + yw * RY + r;
         const int yc = min(y, g.ny - 1);
         rowb[r] = (unsigned)yc * (unsigned)g.sy * 4u;
-        rowh[r] = (unsigned)yc * 4u * R;
         if (y < g.ny - R) ymask |= 1u << r;
         if (IMG) {
             const int dy = y - fz.ry0;
@@ -183,10 +207,6 @@ __global__ void __launch_bounds__(64 * NZW *NYW, 1)
         fyr[r] = 1.0f;
         if (wtap) fyr[r] = uniform(lat(yc, g.ny));
     }
-    // this lane's place in the upper-border layer (b even: pairs are whole)
-    const int hz = z - (sh.b - R);
-    const bool layer = HIST && hz >= 0 && hz < R;
-    const unsigned hoff = layer ? 4u * (unsigned)hz : 0u;
     // halo rows h = yw, yw + NYW, ... of the 2R around the block's rows
     unsigned hrow[NH];
     int hl[NH];
@@ -199,7 +219,9 @@ __global__ void __launch_bounds__(64 * NZW *NYW, 1)
     }
 
     float q[NR][RY][2];
-    constexpr int NHR = R + 1;  // halo planes in flight (divides NR)
+    // Halo planes in flight (divides NR).  Imaging with the taper has no
+    // registers for more than 2 (spilling 5: 0.624 ms, 2: 0.605)
+    constexpr int NHR = IMG && OUTU ? 2 : R + 1;
     static_assert(NR % NHR == 0);
     float hv[NHR][NH][2];
 
@@ -253,21 +275,21 @@ __global__ void __launch_bounds__(64 * NZW *NYW, 1)
 #pragma unroll
     for (int s = 0; s <= 2 * R; ++s) load_ring(xb - R + s, q[s]);
 #pragma unroll
-    for (int s = 0; s <= R; ++s) load_halo(min(xb + s, xe - 1), hv[s]);
+    for (int s = 0; s < NHR; ++s) load_halo(xb + s, hv[s]);
     stage(0, q[R], hv[0]);
     lds_barrier();
 
-    bool bad = false;
+    bool bad0 = false, bad1 = false;
     int x = xb;
     auto step = [&]<int K>(std::integral_constant<int, K>) -> bool {
         if (x >= xe) return false;
         constexpr int cur = K & 1;
         constexpr int ctr = (K + R) % NR;
         const size_t pl = (size_t)x * (size_t)g.sx;
-        const auto rpp = plane_view(PP + pl);
+        const auto rpp = bounded_view(PP + pl, g.sx);
         const auto rv = plane_view(V + pl);
         const auto rps = plane_view(IMG ? PS + pl : PP);
-        const auto rimg = plane_view(IMG ? fz.img + pl : PP);
+        const auto rimg = bounded_view(IMG ? fz.img + pl : PP, g.sx);
         float(*tl)[LW] = tile[cur];
         // this plane's PP, V (and imaging operands), used after the Laplacians
         float c_pp[RY][2], c_v[RY][2], c_ps[RY][2], c_img[RY][2];
@@ -284,20 +306,9 @@ __global__ void __launch_bounds__(64 * NZW *NYW, 1)
                 ld_pair<POL>(rimg, rowb[r], zoff, c_img[r]);
             }
         }
-        // layer [x][y][R] of the history
-        const auto rhist = plane_view(
-            HIST ? (HIST == 1 ? sh.save : sh.restore) + (size_t)x * (size_t)(g.ny * R) : PP);
-        float c_h[RY][2];
-        if (HIST == 2) {
-#pragma unroll
-            for (int r = 0; r < RY; ++r)
-                ld_pair<POL>(rhist, rowh[r], hoff, c_h[r]);
-        }
-        if (x + 1 < xe) {
-            load_ring(x + 1 + R, q[(K + 2 * R + 1) % NR]);
-            stage(cur ^ 1, q[(ctr + 1) % NR], hv[(K + 1) % NHR]);
-            load_halo(min(x + 1 + R, xe - 1), hv[K % NHR]);
-        }
+        load_ring(min(x + 1 + R, g.nx - 1), q[(K + 2 * R + 1) % NR]);
+        stage(cur ^ 1, q[(ctr + 1) % NR], hv[(K + 1) % NHR]);
+        load_halo(min(x + NHR, g.nx - 1), hv[K % NHR]);
         bool rcvx = false;
         if (IMG) {
             const int dx = x - fz.rx0;
@@ -348,59 +359,52 @@ __global__ void __launch_bounds__(64 * NZW *NYW, 1)
                     }
                 }
                 lapl[r][a] = ax + ay + az;
-                // pinned: otherwise it sinks into the store branch below
+                // pinned: otherwise it sinks into finish's two branches
                 asm volatile("" : "+v"(lapl[r][a]));
             }
         }
+        // the upper taper's arithmetic only in the waves that it reaches
+        auto finish = [&]<bool taped>(std::bool_constant<taped>) {
 #pragma unroll
         for (int r = 0; r < RY; ++r) {
-            float npp[2], ppt[2], o[2];
+            float npp[2], o[2];
 #pragma unroll
             for (int a = 0; a < 2; ++a) {
                 float pp = c_pp[r][a];
                 if (OUT) {
                     if (tf.pp_taps > 0) pp = tapo(pp, a, fxc, fyr[r]);
-                } else if (OUTU && wtap) {
+                } else if (taped) {
                     pp = tap(pp, a, fxc, fyr[r]);
                 }
-                ppt[a] = pp;
                 npp[a] = 2.f * q[ctr][r][a] - pp + c_v[r][a] * lapl[r][a];
                 o[a] = npp[a];
-                if (OUT) o[a] = tapo(npp[a], a, fxc, fyr[r]);
-                if (OUTU && wtap && ztap[a] && z + a < tf.b - tf.hold)
-                    o[a] = tap(npp[a], a, fxc, fyr[r]);
+                // (z frame: not updated; PP tapered once more as the next
+                // step's P)
+                if (OUT) o[a] = tapo((a ? zcomp1 : zcomp) ? npp[a] : pp, a, fxc, fyr[r]);
+                if (taped) o[a] = ucell[a] ? tap(npp[a], a, fxc, fyr[r]) : o[a];
             }
             const bool row = (ymask >> r) & 1u;
-            if (HIST == 2 && layer) {
-                o[0] = c_h[r][0];
-                o[1] = c_h[r][1];
-            }
-            if (HIST == 1 && row && layer)
-                st_pair<POL>(rhist, rowh[r], hoff, npp[0], npp[1], true, true);
-            if (OUTU && !IMG && sh.zframe && wtap && row && z < R)
-                st_pair<POL>(rpp, rowb[r], zoff, tap(ppt[0], 0, fxc, fyr[r]),
-                             tap(ppt[1], 1, fxc, fyr[r]), true, true);
-            // z frame (not updated): PP tapered once more as the next step's P
-            if (OUT && row && (zframe[0] || zframe[1]))
-                st_pair<POL>(rpp, rowb[r], 4u * (unsigned)z, tapo(ppt[0], 0, fxc, fyr[r]),
-                        tapo(ppt[1], 1, fxc, fyr[r]), zframe[0], zframe[1]);
-            if (row && zcomp) {
-                st_pair<POL>(rpp, rowb[r], zoff, o[0], o[1], true, zcomp1);
-                bad |= (npp[0] != npp[0]) || (zcomp1 && npp[1] != npp[1]);
-                if (IMG) {
-                    bool im[2];
-                    float iv[2];
+            if (ODD && !OUT) o[1] = zcomp1 ? o[1] : c_pp[r][1];
+            st_pair<POL>(rpp, rowb[r], row && wpair ? zoff : kDropped, o[0], o[1]);
+            if (ODD && OUT) st_one<POL>(rpp, rowb[r], row && wone ? zoff + 4u : kDropped, o[0]);
+            bad0 |= row && npp[0] != npp[0];
+            bad1 |= row && npp[1] != npp[1];
+            if (IMG) {
+                // cells of a pair outside [z0, z1) or under a receiver keep
+                // their value
+                const bool rc = rcvx && ((rmask >> r) & 1u);
+                float iv[2];
 #pragma unroll
-                    for (int a = 0; a < 2; ++a) {
-                        const int za = z + a;
-                        im[a] = za >= fz.z0 && za < fz.z1 &&
-                                !(rcvx && ((rmask >> r) & 1u) && za == fz.rz);
-                        iv[a] = c_img[r][a] + c_ps[r][a] * npp[a];
-                    }
-                    st_pair<POL>(rimg, rowb[r], zoff, iv[0], iv[1], im[0], im[1] && zcomp1);
+                for (int a = 0; a < 2; ++a) {
+                    const bool on = icell[a] && !(rc && rcell[a]);
+                    iv[a] = on ? c_img[r][a] + c_ps[r][a] * npp[a] : c_img[r][a];
                 }
+                st_pair<POL>(rimg, rowb[r], row && ipair ? zoff : kDropped, iv[0], iv[1]);
             }
         }
+        };
+        if (OUTU && wtap) finish(std::true_type{});
+        else finish(std::false_type{});
         lds_barrier();
         ++x;
         return true;
@@ -410,7 +414,7 @@ __global__ void __launch_bounds__(64 * NZW *NYW, 1)
             (step(std::integral_constant<int, Ks>{}) && ...);
         }(std::make_integer_sequence<int, NR>{});
     }
-    if (bad) atomicOr(flag, 1);
+    if ((zcomp && bad0) || (zcomp1 && bad1)) atomicOr(flag, 1);
 }
 
 }  // namespace slab

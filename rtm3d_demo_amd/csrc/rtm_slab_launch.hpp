@@ -11,26 +11,15 @@ struct SlabGrid {
     int nyt, nxc, xchunk;
 };
 
-// Work of a step on the cells around the updated ones, done in the same pass:
-// save / restore (at most one) point to the step's layer [nx][ny][4] of the
-// upper-border history (blen b, even, >= 8), zframe: see k_slab.  Covers the
-// rows that the step updates; the x and y frame is the caller's.
-struct SlabShell {
-    float *save;
-    const float *restore;
-    int b;
-    int zframe;
-};
-
 // Launches for even and odd row lengths: nzw waves of 128 z per row, `form`
 // the fusion (form_of).
-enum Form { kPlain, kPlainRestore, kOut, kOutUpper, kOutUpperSave, kImage, kImageOutUpper };
+enum Form { kPlain, kOut, kOutUpper, kImage, kImageOutUpper };
 hipError_t launch_even(int nzw, Form form, const float *P, float *PP, const float *V,
                        const Coefs &cf, const Grid &g, const SlabGrid &sg, const ImageFuse &fz,
-                       const TaperFuse &tf, const SlabShell &sh, int *flag, hipStream_t s);
+                       const TaperFuse &tf, int *flag, hipStream_t s);
 hipError_t launch_odd(int nzw, Form form, const float *P, float *PP, const float *V,
                       const Coefs &cf, const Grid &g, const SlabGrid &sg, const ImageFuse &fz,
-                      const TaperFuse &tf, const SlabShell &sh, int *flag, hipStream_t s);
+                      const TaperFuse &tf, int *flag, hipStream_t s);
 
 // y waves per block and rows per wave: 12 waves (3 per SIMD at up to 168
 // registers) whatever the row length.
@@ -44,7 +33,6 @@ constexpr int y_waves(int nzw) { return 12 / nzw; }
 // taper on the output.
 bool slab_fits(int radius, const Grid &g, const ImageFuse *fuse, const TaperFuse *taper);
 hipError_t launch_slab(const float *P, float *PP, const float *V, const Coefs &cf, const Grid &g,
-                       const ImageFuse *fuse, const TaperFuse *taper, int *flag, hipStream_t s,
-                       const slab::SlabShell *shell = nullptr);
+                       const ImageFuse *fuse, const TaperFuse *taper, int *flag, hipStream_t s);
 
 }  // namespace rtmhip

@@ -5,15 +5,15 @@ namespace rtmhip {
 namespace slab {
 namespace {
 
-template <int NZW, bool IMG, int TAPER, int HIST = 0>
+template <int NZW, bool IMG, int TAPER>
 hipError_t run(const float *P, float *PP, const float *V, const Coefs &cf, const Grid &g,
-               const SlabGrid &sg, const ImageFuse &fz, const TaperFuse &tf,
-               const SlabShell &sh, int *flag, hipStream_t s)
+               const SlabGrid &sg, const ImageFuse &fz, const TaperFuse &tf, int *flag,
+               hipStream_t s)
 {
     constexpr int NYW = y_waves(NZW);
-    hipLaunchKernelGGL((k_slab<NZW, NYW, kRows, IMG, TAPER, true, HIST>),
+    hipLaunchKernelGGL((k_slab<NZW, NYW, kRows, IMG, TAPER, true>),
                        dim3((unsigned)(sg.nyt * sg.nxc)), dim3(64 * NZW, NYW), 0, s, P, PP, V, cf,
-                       g, sg, fz, tf, sh, flag);
+                       g, sg, fz, tf, flag);
     return hipGetLastError();
 }
 
@@ -22,10 +22,8 @@ hipError_t by_form(Form form, A &&...a)
 {
     switch (form) {
     case kPlain: return run<NZW, false, 0>(a...);
-    case kPlainRestore: return run<NZW, false, 0, 2>(a...);
     case kOut: return run<NZW, false, 3>(a...);
     case kOutUpper: return run<NZW, false, 4>(a...);
-    case kOutUpperSave: return run<NZW, false, 4, 1>(a...);
     case kImage: return run<NZW, true, 0>(a...);
     default: return run<NZW, true, 4>(a...);
     }
@@ -35,12 +33,12 @@ hipError_t by_form(Form form, A &&...a)
 
 hipError_t launch_odd(int nzw, Form form, const float *P, float *PP, const float *V,
                        const Coefs &cf, const Grid &g, const SlabGrid &sg, const ImageFuse &fz,
-                       const TaperFuse &tf, const SlabShell &sh, int *flag, hipStream_t s)
+                       const TaperFuse &tf, int *flag, hipStream_t s)
 {
     switch (nzw) {
-    case 2: return by_form<2>(form, P, PP, V, cf, g, sg, fz, tf, sh, flag, s);
-    case 3: return by_form<3>(form, P, PP, V, cf, g, sg, fz, tf, sh, flag, s);
-    case 4: return by_form<4>(form, P, PP, V, cf, g, sg, fz, tf, sh, flag, s);
+    case 2: return by_form<2>(form, P, PP, V, cf, g, sg, fz, tf, flag, s);
+    case 3: return by_form<3>(form, P, PP, V, cf, g, sg, fz, tf, flag, s);
+    case 4: return by_form<4>(form, P, PP, V, cf, g, sg, fz, tf, flag, s);
     default: return hipErrorInvalidValue;
     }
 }
