@@ -864,6 +864,43 @@ __global__ void __launch_bounds__(kThreads)
     img[o] = im;
 }
 
+// The same on groups of four z cells (nz, b and the rows multiples of four,
+// every array 16-byte aligned): 16-byte accesses, the accumulators -- nearly
+// all of the bytes, each touched once a step -- past the caches.  Salt grid, 4
+// frequencies (9.7 GB a step): 1.99 ms with 4-byte accesses, 1.75 so (5.5 TB/s).
+typedef float vec4_t __attribute__((ext_vector_type(4)));
+__global__ void __launch_bounds__(kThreads)
+    k_freq_image_v(vec4_t *__restrict__ img, const vec4_t *__restrict__ PS,
+                   const vec4_t *__restrict__ PR, vec4_t *__restrict__ sre,
+                   vec4_t *__restrict__ sim, vec4_t *__restrict__ rre, vec4_t *__restrict__ rim,
+                   const float *__restrict__ kre, const float *__restrict__ kim,
+                   const float *__restrict__ w2, Grid g, int b, int vol, FastDiv dnz, FastDiv dny,
+                   int nz4, int ny, int nwstep, int iw0, int nw, int nt, int st)
+{
+    const int i = (int)(blockIdx.x * kThreads + threadIdx.x);  // vol < 2^31 (launcher)
+    if (i >= vol) return;
+    const int r = fdiv(i, dnz);
+    const int iz = i - r * nz4;
+    const int ix = fdiv(r, dny), iy = r - ix * ny;
+    const long long o = goff(g, ix + b, iy + b, 4 * iz + b) >> 2;
+    const vec4_t ps = PS[o], pr = PR[o];
+    vec4_t im = img[o];
+    for (int lw = 0, iw = iw0; lw < nwstep && iw < nw; ++lw, ++iw) {
+        const float kr = kre[(long long)iw * nt + st], ki = kim[(long long)iw * nt + st];
+        const long long f = (long long)lw * vol + i;
+        const vec4_t a = __builtin_nontemporal_load(&sre[f]) + kr * ps;
+        const vec4_t c2 = __builtin_nontemporal_load(&sim[f]) + ki * ps;
+        const vec4_t c = __builtin_nontemporal_load(&rre[f]) + kr * pr;
+        const vec4_t d = __builtin_nontemporal_load(&rim[f]) + ki * pr;
+        __builtin_nontemporal_store(a, &sre[f]);
+        __builtin_nontemporal_store(c2, &sim[f]);
+        __builtin_nontemporal_store(c, &rre[f]);
+        __builtin_nontemporal_store(d, &rim[f]);
+        im = im + w2[iw] * (a * c - c2 * d);
+    }
+    img[o] = im;
+}
+
 __global__ void __launch_bounds__(kThreads) k_fill(float *__restrict__ p, size_t n, float v)
 {
     for (size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x; i < n;
@@ -1498,6 +1535,17 @@ hipError_t launch_freq_image(float *img, const float *PS, const float *PR, float
     const int nx = g.nx - 2 * b, ny = g.ny - 2 * b, nz = g.nz - 2 * b;
     const long long vol = (long long)nx * ny * nz;
     if (vol <= 0 || nwstep <= 0 || iw0 >= nw) return hipSuccess;
+    const void *arrays[] = {img, PS, PR, sre, sim, rre, rim};
+    bool quads = ((nz | b | g.sy) & 3) == 0 && (g.sx & 3) == 0 && vol / 4 + kThreads < (1LL << 31);
+    for (const void *p : arrays) quads = quads && ((uintptr_t)p & 15) == 0;
+    if (quads) {
+        auto v = [](const float *p) { return reinterpret_cast<vec4_t *>(const_cast<float *>(p)); };
+        hipLaunchKernelGGL(k_freq_image_v, dim3(nblocks(vol / 4)), dim3(kThreads), 0, s, v(img),
+                           v(PS), v(PR), v(sre), v(sim), v(rre), v(rim), kre, kim, w2, g, b,
+                           (int)(vol / 4), fast_div((uint32_t)(nz / 4)), fast_div((uint32_t)ny),
+                           nz / 4, ny, nwstep, iw0, nw, nt, st);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(k_freq_image, dim3(nblocks(vol)), dim3(kThreads), 0, s, img, PS, PR, sre,
                        sim, rre, rim, kre, kim, w2, g, b, nx, ny, nz, nwstep, iw0, nw, nt, st);
     return hipGetLastError();

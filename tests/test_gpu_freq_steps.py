@@ -9,6 +9,8 @@ The default taper form applies the tapers to the new fields' output (even
 nz: two-z waves, odd nz: one-z waves); a receiver line that reaches the x
 border falls back to the in-place passes, as does taper fusion mode 0.
 """
+import sys
+
 import numpy as np
 import pytest
 
@@ -86,6 +88,13 @@ def test_freq_steps_match_operator_sequence(gpu, oracle, shape, kind, fusion, sp
     want = [Ps, PPs, Pr, PPr, img] + acc
     for k, (a, w) in enumerate(zip(got, want)):
         assert np.array_equal(a.view(np.uint32), w.view(np.uint32)), k
+
+
+# borders and rows that are and are not multiples of four (16-byte accumulators)
+@pytest.mark.parametrize("shape, b", [((40, 44, 36), 8), ((41, 43, 40), 12), ((40, 44, 38), 8)])
+def test_freq_steps_accumulator_groups(gpu, oracle, monkeypatch, shape, b):
+    monkeypatch.setattr(sys.modules[__name__], "B", b)
+    test_freq_steps_match_operator_sequence(gpu, oracle, shape, "inside", -1, (4, 2, 6))
 
 
 def test_freq_steps_reject_a_call_across_receiver_chunks(gpu, oracle):
