@@ -162,9 +162,25 @@ __global__ void __launch_bounds__(kThreads)
                 true, 1);
 }
 
-// taper3D over 16-byte groups (the front-right edge's interior-z cells
-// excepted): the z-border groups of the rows with x and y interior, then
-// every group of the rows with x or y in a border, as k_taper_all.
+// The front-right edge of taper3D (RTMCPUPlatform.cpp:900-904): its cells x <
+// blen, y >= ny-blen, z interior are written from the face-tapered cell (blen,
+// y, z), ((P(blen,y,z)*gy)*gx)*gy with the face pass's product as stored.  The
+// thread that tapers (blen, y, z) writes the edge's cells with that y and z
+// (v: that cell's stored value; p: the cell at x = 0).
+template <typename T>
+__device__ __forceinline__ void taper_edge(T *__restrict__ p, const float *__restrict__ t,
+                                           const Grid &g, int b, float v, float gy)
+{
+    for (int x = 0; x < b; ++x) {
+        float w = v * t[b - 1 - x];
+        w *= gy;
+        p[(long long)x * g.sx] = wst<T>(w);
+    }
+}
+
+// taper3D over 16-byte groups (the front-right edge's interior-z cells by the
+// threads of plane b): the z-border groups of the rows with x and y interior,
+// then every group of the rows with x or y in a border, as k_taper_all.
 template <typename T>
 __global__ void __launch_bounds__(kThreads)
     k_taper_all_v(T *__restrict__ P0, T *__restrict__ P1, const float *__restrict__ t, Grid g,
@@ -218,6 +234,9 @@ __global__ void __launch_bounds__(kThreads)
     } else {
         // (bx and by: gx gy) | gy | gx
         taper_group(p, t, z0, g.nz, b, bx ? gx : gy, bx && by ? gy : 1.0f, false, 0);
+        if (!bx && x == b && y >= g.ny - b)
+            for (int k = 0; k < G; ++k)
+                taper_edge(p + k - (long long)b * g.sx, t, g, b, wld(p[k]), gy);
     }
 }
 
@@ -458,38 +477,9 @@ __global__ void __launch_bounds__(kThreads)
     P[goff(g, x, y, z)] = wst<T>(v);
 }
 
-// The front-right edge of taper3D (RTMCPUPlatform.cpp:900-904) writes cells
-// x < blen, y >= ny-blen, z interior from the face-tapered cell
-// (blen, y, z).  This kernel runs before k_taper_all so it reads that cell
-// before the face pass rescales it:  ((P(blen,y,z)*gy)*gx)*gy, where the
-// face pass's product P*gy is the value it stored (rounded to T).
-template <typename T>
-__global__ void __launch_bounds__(kThreads)
-    k_taper_front_right(T *__restrict__ P0, T *__restrict__ P1, const float *__restrict__ t,
-                        Grid g, int b)
-{
-    T *__restrict__ P = blockIdx.y ? P1 : P0;  // one grid per blockIdx.y
-    const int lz = g.nz - 2 * b;
-    const long long n = (long long)b * b * lz;
-    const long long i = (long long)blockIdx.x * kThreads + threadIdx.x;
-    if (i >= n) return;
-    const int z = b + (int)(i % lz);
-    const long long r = i / lz;
-    const int iy = (int)(r % b);
-    const int x = (int)(r / b);
-    const int y = g.ny - b + iy;
-    const float gy = t[iy];
-    float v = wld(P[goff(g, b, y, z)]);
-    v *= gy;
-    v = wrnd<T>(v);
-    v *= t[b - 1 - x];
-    v *= gy;
-    P[goff(g, x, y, z)] = wst<T>(v);
-}
-
-// taper3D (RTMCPUPlatform.cpp:710-920) for every border cell except the
-// front-right edge's interior-z cells, of one or two grids (blockIdx.y picks
-// the grid), over two packed index ranges:
+// taper3D (RTMCPUPlatform.cpp:710-920) of one or two grids (blockIdx.y picks the
+// grid), over two packed index ranges (the front-right edge's interior-z cells
+// by the threads of plane blen):
 //   [0, nA)        the z-border cells (z < b or z >= nz-b) of the rows with x
 //                  and y interior: 2b consecutive cells per row, z factor only;
 //   [nA, nA + nB)  every cell of the rows with x or y in a border (the x
@@ -504,6 +494,7 @@ struct TaperCell {
     long long off;
     float f1, f2, f3;
     bool ok;
+    int edge;  // index of the y factor where the cell feeds the front-right edge, else -1
 };
 
 struct TaperDivs {
@@ -513,7 +504,7 @@ struct TaperDivs {
 __device__ __forceinline__ TaperCell taper_cell(const float *__restrict__ t, const Grid &g, int b,
                                                 int nA, int nB, const TaperDivs &dv, int i)
 {
-    TaperCell c{0, 1.0f, 1.0f, 1.0f, false};
+    TaperCell c{0, 1.0f, 1.0f, 1.0f, false, -1};
     const int b2 = 2 * b;
     int x, y, z;
     bool bx, by;
@@ -560,6 +551,7 @@ __device__ __forceinline__ TaperCell taper_cell(const float *__restrict__ t, con
         // (bx and by: gx gy) | gy | gx
         c.f1 = bx ? gx : gy;
         c.f2 = bx && by ? gy : 1.0f;
+        if (!bx && x == b && y >= g.ny - b) c.edge = y - (g.ny - b);
     }
     c.off = (long long)x * g.sx + (long long)y * g.sy + z;
     c.ok = true;
@@ -586,7 +578,10 @@ __global__ void __launch_bounds__(kThreads)
         float w = v[k] * c[k].f1;
         w *= c[k].f2;
         w *= c[k].f3;
+        w = wrnd<T>(w);
         P[c[k].off] = wst<T>(w);
+        if (c[k].edge >= 0)
+            taper_edge(P + (c[k].off - (long long)b * g.sx), t, g, b, w, t[c[k].edge]);
     }
 }
 
@@ -1362,14 +1357,6 @@ hipError_t launch_taper_all2(T *P, T *Q, const float *taper, const Grid &g, int 
     if (b <= 0) return hipSuccess;
     if ((long long)g.nx * g.ny >= (1LL << 31)) return hipErrorInvalidValue;
     const unsigned ng = Q ? 2 : 1;
-    // the front-right edge first: it reads (blen, y, z) before the face pass
-    // rescales that cell
-    const long long lz = g.nz - 2 * b;
-    const long long nfr = (long long)b * b * lz;
-    if (nfr > 0 && g.nx > 2 * b) {
-        hipLaunchKernelGGL(k_taper_front_right<T>, dim3(nblocks(nfr), ng), dim3(kThreads), 0, s,
-                           P, Q, taper, g, b);
-    }
     const long long nA = (long long)(g.nx - 2 * b) * (g.ny - 2 * b) * 2 * b;
     const long long nB = ((long long)2 * b * g.ny + (long long)(g.nx - 2 * b) * 2 * b) * g.nz;
     const long long per = (long long)kThreads * kTaperPer;
