@@ -1,13 +1,16 @@
 """Tile-shape autotuner for the stencil kernels.
 
-For a given grid, every compiled tile shape is timed for the three stencil
-kernel classes (0 plain step, 1 fused receiver step, 2 tapered HBC forward
-step) with HIP events around each launch, by running a few steps of the
-forward and fused backward loops on the caller's buffers; the fastest shape
-per class is installed with rtmhip_set_tiling.  Results are identical for
+For a given grid, the library's default ((0, 0, 0): the full-row blocks where
+they fit) and every compiled tile shape are timed for the three stencil kernel
+classes (0 plain step, 1 fused receiver step, 2 tapered HBC forward step) with
+HIP events around each launch, by running a few steps of the forward and fused
+backward loops on the caller's buffers; the fastest shape per class is
+installed with rtmhip_set_tiling.  Results are identical for
 every shape (tested), so tuning only changes speed.
 """
 import numpy as np
+
+DEFAULT = (0, 0, 0)
 
 
 def tune(hip, shot, V, coefs, g, src, F, R, upb, rcv, img, steps=6, rounds=2, log=None):
@@ -17,7 +20,7 @@ def tune(hip, shot, V, coefs, g, src, F, R, upb, rcv, img, steps=6, rounds=2, lo
     overwritten); `shot` must allow `steps` time steps."""
     best = {}
     nt = shot.nt
-    for tiling in hip.TILINGS:
+    for tiling in [DEFAULT] + list(hip.TILINGS):
         for cls in range(3):
             hip.set_tiling(cls, *tiling, 0)
         # one untimed pass to settle clocks and caches
@@ -38,12 +41,12 @@ def tune(hip, shot, V, coefs, g, src, F, R, upb, rcv, img, steps=6, rounds=2, lo
             if cls not in best or avg < best[cls][1]:
                 best[cls] = (tiling, avg)
     # With the forward upper taper on the output (the FP32 default) every
-    # class-2 shape but the one-z 64x1x6 / 64x1x8 waves launches the same
-    # two-z 128x1x4 kernel: record that shape
+    # class-2 shape but the default and the one-z 64x1x6 / 64x1x8 waves
+    # launches the same two-z 128x1x4 kernel: record that shape
     fmt = {0: "f32", 1: "f16", 2: "bf16"}.get(getattr(shot, "wave_format", 0), "f32")
     if 2 in best and hip.get_taper_fusion(fmt) in (-1, 4) and fmt == "f32":
         t2 = tuple(best[2][0])
-        if not (t2[0] == 64 and t2[1] == 1 and t2[2] in (6, 8)):
+        if t2 != DEFAULT and not (t2[0] == 64 and t2[1] == 1 and t2[2] in (6, 8)):
             best[2] = ((128, 1, 4), best[2][1])
     for cls in range(3):
         if cls in best:
@@ -55,7 +58,8 @@ def tune(hip, shot, V, coefs, g, src, F, R, upb, rcv, img, steps=6, rounds=2, lo
     return best
 
 
-BATCH_SHOT_TILINGS = [(1, 4, 4), (1, 2, 6), (1, 2, 7), (2, 4, 3), (64, 1, 8), (128, 1, 4)]
+BATCH_SHOT_TILINGS = [DEFAULT, (1, 4, 4), (1, 2, 6), (1, 2, 7), (2, 4, 3), (64, 1, 8),
+                      (128, 1, 4)]
 
 
 def tune_batch(hip, batch, nt, steps=17, log=None):
@@ -112,13 +116,13 @@ def tune_batch(hip, batch, nt, steps=17, log=None):
                 best_mode = (mode, ms)
         batch.set_stencil(cls, best_mode[0])
         out[cls] = {"mode": best_mode[0], "ms_per_step": round(best_mode[1], 3),
-                    "tile": "%dx%dx%d" % best_tile[0],
+                    "tile": "%dx%dx%d" % best_tile[0] if best_tile[0][0] else "default",
                     "tile_ms_per_step": round(best_tile[1], 3)}
     return out
 
 
 def describe(best):
-    return {str(c): {"tile": "%dx%dx%d" % t, "avg_ms": round(ms, 4)} for c, (t, ms) in
+    return {str(c): {"tile": "%dx%dx%d" % t if t[0] else "default", "avg_ms": round(ms, 4)} for c, (t, ms) in
             sorted(best.items())}
 
 
