@@ -359,6 +359,20 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t plane_rsrc(const void *p)
 {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, -1, 0x00020000);
 }
+
+// A plane as a view of its size: a store at lane offset kDropped is out of
+// range of it (less the row offset, which is at least R rows) and discarded, so a plane's step has no branch around a load or a
+// store and the compiler's wait counts are exact (at a join it must assume
+// that neither branch's accesses were issued, and waits for more).  With
+// branches / so, ms: FP16 two-z waves on 592 x 592 x 336, 6 x chunks, plain 0.334 /
+// 0.294, imaging 0.600 / 0.541; FP32 one-z 8-row waves, taper3D on the output,
+// 192^3 0.060 / 0.053.
+constexpr unsigned kDropped = 0xfffffff0u;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t plane_bounded(const void *p, size_t bytes)
+{
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)(unsigned)bytes,
+                                             0x00020000);
+}
 // Loads and stores of one element of type T, widened to / rounded from
 // float.  The builtins move raw bits: reinterpret, never convert.
 template <typename T>
@@ -850,18 +864,20 @@ __device__ __forceinline__ void wave_tile(const T *__restrict__ P, T *__restrict
         taper_ring(x + R, q[(K + 2 * R) % NR]);
         taper_halo(x, cur);
         const size_t pl = (size_t)x * (size_t)g.sx;
-        const auto rpp = plane_rsrc(PP + pl);
+        const auto rpp = plane_bounded(PP + pl, (size_t)g.sx * ES);
         const auto rv = plane_rsrc(V + pl);
         const auto rps = plane_rsrc(IMG ? (const void *)(PS + pl) : (const void *)PP);
-        const auto rimg = plane_rsrc(IMG ? (const void *)(fz.img + pl) : (const void *)PP);
+        const auto rimg = plane_bounded(IMG ? (const void *)(fz.img + pl) : (const void *)PP,
+                                        (size_t)g.sx * 4u);
         float c_pp[RY], c_v[RY], c_ps[RY], c_img[RY];
         // front-right cells read PP at plane b, which this wave updates later
         // in its march (the launcher makes the first x chunk reach b)
         const bool qxc = ALL && x < tf.b;
         const unsigned ppq = qxc && zmid ? zoff + qdelta(x) : zoff;
+        const auto rppb = plane_rsrc(PP + pl);  // reaches plane b
 #pragma unroll
         for (int r = 0; r < RY; ++r) {
-            c_pp[r] = ld_buf<T>(rpp, rowb[r], ((qmask >> r) & 1u) ? ppq : zoff);
+            c_pp[r] = ld_buf<T>(ALL ? rppb : rpp, rowb[r], ((qmask >> r) & 1u) ? ppq : zoff);
             c_v[r] = ld_buf<float>(rv, rowb[r] * VS, zoffv);
         }
         if (IMG) {
@@ -880,10 +896,9 @@ __device__ __forceinline__ void wave_tile(const T *__restrict__ P, T *__restrict
         float yc[2 * R];  // this plane's y-halo values (registers)
 #pragma unroll
         for (int h = 0; h < 2 * R; ++h) yc[h] = yh[cur][h];
-        if (x + 1 < xe) {
-            load_ring(x + 1 + R, q[(K + 2 * R + 1) % NR]);
-            fetch_halo(x + 1, cur ^ 1);
-        }
+        // past the chunk's last plane too (clamped): no branch, exact waits
+        load_ring(min(x + 1 + R, g.nx - 1), q[(K + 2 * R + 1) % NR]);
+        fetch_halo(min(x + 1, g.nx - 1), cur ^ 1);
         bool rcvx = false;
         if (IMG) {
             const int dx = x - fz.rx0;
@@ -896,15 +911,23 @@ __device__ __forceinline__ void wave_tile(const T *__restrict__ P, T *__restrict
         for (int r = 0; r < RY; ++r) {
             const float *t = &lt[r][R + lane];
             const float p = q[ctr][r];
-            float ax = 0.f, ay = 0.f, az = 0.f;
+            float ax, ay, az;
 #pragma unroll
             for (int io = 0; io <= 2 * R; ++io) {
                 const int ry = r + io - R;  // compile-time row of the y tap
                 const float vy = ry < 0 ? yc[ry + R] : (ry >= RY ? yc[R + ry - RY] : q[ctr][ry]);
                 const float vz = (io == R) ? p : t[io - R];
-                ax += q[(K + io) % NR][r] * cf.c[0][io];
-                ay += vy * cf.c[1][io];
-                az += vz * cf.c[2][io];
+                const float vx = q[(K + io) % NR][r];
+                if (io == 0) {
+                    // 0 + v*c: one rounding, and -0 becomes +0 as in the sum
+                    ax = __builtin_fmaf(vx, cf.c[0][io], 0.f);
+                    ay = __builtin_fmaf(vy, cf.c[1][io], 0.f);
+                    az = __builtin_fmaf(vz, cf.c[2][io], 0.f);
+                } else {
+                    ax += vx * cf.c[0][io];
+                    ay += vy * cf.c[1][io];
+                    az += vz * cf.c[2][io];
+                }
             }
             lapl[r] = ax + ay + az;
             asm volatile("" : "+v"(lapl[r]));
@@ -926,20 +949,22 @@ __device__ __forceinline__ void wave_tile(const T *__restrict__ P, T *__restrict
                 if (tf.pp_taps > 1 && !qk) pp = tap(pp, fxc, fyr[r]);
             }
             const float npp = 2.f * p - pp + c_v[r] * lapl[r];
-            // z frame (not updated): PP tapered, and with OUT once more as
-            // the next step's P
-            if (EVERY && zframe && ((ymask >> r) & 1u))
-                st_buf<T>(rpp, rowb[r], zoff,
-                          OUT ? tapv(pp, fxc, fyr[r], ztap, fzl, false) : pp);
-            if (((ymask >> r) & 1u) && zcomp) {
-                // OUT: the value the step stores (rounded), then taper3D
-                const bool otap = OUT || (OUTU && ztap && z < tf.b - tf.hold);
-                st_buf<T>(rpp, rowb[r], zoff,
-                          otap ? tapv(wrnd<T>(npp), fxc, fyr[r], ztap, fzl, false) : npp);
-                bad |= (npp != npp);
-                if (IMG && (z >= fz.z0) && (z < fz.z1) &&
-                    !(rcvx && ((rmask >> r) & 1u) && z == fz.rz))
-                    st_buf<float>(rimg, rowb[r] * VS, zoffv, c_img[r] + c_ps[r] * wrnd<T>(npp));
+            // one store, discarded where the cell is not updated.  OUT: the
+            // value the step stores (rounded), then taper3D.  z frame (not
+            // updated): PP tapered, and with OUT once more as the next step's P
+            const bool row = (ymask >> r) & 1u;
+            const bool otap = OUTU && ztap && z < tf.b - tf.hold;
+            float o = npp;
+            if (OUT) o = tapv(zcomp ? wrnd<T>(npp) : pp, fxc, fyr[r], ztap, fzl, false);
+            else if (ALL) o = zcomp ? npp : pp;
+            else if (OUTU) o = otap ? tapv(wrnd<T>(npp), fxc, fyr[r], ztap, fzl, false) : npp;
+            st_buf<T>(rpp, rowb[r], row && (zcomp || zframe) ? zoff : kDropped, o);
+            bad |= row && zcomp && npp != npp;
+            if (IMG) {
+                const bool on = row && zcomp && z >= fz.z0 && z < fz.z1 &&
+                                !(rcvx && ((rmask >> r) & 1u) && z == fz.rz);
+                st_buf<float>(rimg, rowb[r] * VS, on ? zoffv : kDropped,
+                              c_img[r] + c_ps[r] * wrnd<T>(npp));
             }
         }
         ++x;
@@ -1213,10 +1238,11 @@ __device__ __forceinline__ void wave_tile2(const T *__restrict__ P, T *__restric
         taper_ring(x + R, q[(K + 2 * R) % NR]);
         taper_halo(x, cur);
         const size_t pl = (size_t)x * (size_t)g.sx;
-        const auto rpp = plane_rsrc(PP + pl);
+        const auto rpp = plane_bounded(PP + pl, (size_t)g.sx * ES);
         const auto rv = plane_rsrc(V + pl);
         const auto rps = plane_rsrc(IMG ? (const void *)(PS + pl) : (const void *)PP);
-        const auto rimg = plane_rsrc(IMG ? (const void *)(fz.img + pl) : (const void *)PP);
+        const auto rimg = plane_bounded(IMG ? (const void *)(fz.img + pl) : (const void *)PP,
+                                        (size_t)g.sx * 4u);
         float c_pp[RY][2], c_v[RY][2], c_ps[RY][2], c_img[RY][2];
 #pragma unroll
         for (int r = 0; r < RY; ++r) {
@@ -1244,10 +1270,9 @@ __device__ __forceinline__ void wave_tile2(const T *__restrict__ P, T *__restric
             yc[h][0] = yh[cur][h][0];
             yc[h][1] = yh[cur][h][1];
         }
-        if (x + 1 < xe) {
-            load_ring(x + 1 + R, q[(K + 2 * R + 1) % NR]);
-            fetch_halo(x + 1, cur ^ 1);
-        }
+        // past the chunk's last plane too (clamped): no branch, exact waits
+        load_ring(min(x + 1 + R, g.nx - 1), q[(K + 2 * R + 1) % NR]);
+        fetch_halo(min(x + 1, g.nx - 1), cur ^ 1);
         bool rcvx = false;
         if (IMG) {
             const int dx = x - fz.rx0;
@@ -1270,16 +1295,24 @@ __device__ __forceinline__ void wave_tile2(const T *__restrict__ P, T *__restric
 #pragma unroll
             for (int a = 0; a < 2; ++a) {
                 const float p = q[ctr][r][a];
-                float ax = 0.f, ay = 0.f, az = 0.f;
+                float ax, ay, az;
 #pragma unroll
                 for (int io = 0; io <= 2 * R; ++io) {
                     const int ry = r + io - R;  // compile-time row of the y tap
                     const float vy = ry < 0 ? yc[ry + R][a]
                                             : (ry >= RY ? yc[R + ry - RY][a] : q[ctr][ry][a]);
                     const float vz = (io == R) ? p : w[io + a];
-                    ax += q[(K + io) % NR][r][a] * cf.c[0][io];
-                    ay += vy * cf.c[1][io];
-                    az += vz * cf.c[2][io];
+                    const float vx = q[(K + io) % NR][r][a];
+                    if (io == 0) {
+                        // 0 + v*c: one rounding, and -0 becomes +0 as in the sum
+                        ax = __builtin_fmaf(vx, cf.c[0][io], 0.f);
+                        ay = __builtin_fmaf(vy, cf.c[1][io], 0.f);
+                        az = __builtin_fmaf(vz, cf.c[2][io], 0.f);
+                    } else {
+                        ax += vx * cf.c[0][io];
+                        ay += vy * cf.c[1][io];
+                        az += vz * cf.c[2][io];
+                    }
                 }
                 lapl[r][a] = ax + ay + az;
                 asm volatile("" : "+v"(lapl[r][a]));
@@ -1302,41 +1335,39 @@ __device__ __forceinline__ void wave_tile2(const T *__restrict__ P, T *__restric
                 ppt[a] = pp;
                 npp[a] = 2.f * q[ctr][r][a] - pp + c_v[r][a] * lapl[r][a];
             }
-            // z frame (not updated): PP tapered once more as the next step's P
-            if (OUT && zframe && ((ymask >> r) & 1u))
-                st_buf2<T>(rpp, rowb[r], zoff, tapo(ppt[0], 0, fxc, fyr[r]),
-                           tapo(ppt[1], 1, fxc, fyr[r]));
-            if (((ymask >> r) & 1u) && zcomp) {
-                if (OUT) {
-                    st_buf2<T>(rpp, rowb[r], zoff, tapo(wrnd<T>(npp[0]), 0, fxc, fyr[r]),
-                               tapo(wrnd<T>(npp[1]), 1, fxc, fyr[r]));
-                } else if (OUTU && wtap) {
-                    // cells z < b - hold: the value stored, then the upper taper
-                    float o[2];
+            // one store of the pair (out of range, so discarded, where the row
+            // or the pair is not updated): OUT also writes the z frame (not
+            // updated: PP tapered once more as the next step's P); OUTU cells
+            // z < b - hold the value stored, then the upper taper
+            const bool row = (ymask >> r) & 1u;
+            float o[2];
 #pragma unroll
-                    for (int a = 0; a < 2; ++a)
-                        o[a] = (ztap[a] && z + a < tf.b - tf.hold)
-                                   ? tap(wrnd<T>(npp[a]), a, fxc, fyr[r])
-                                   : npp[a];
-                    st_buf2<T>(rpp, rowb[r], zoff, o[0], o[1]);
-                } else {
-                    st_buf2<T>(rpp, rowb[r], zoff, npp[0], npp[1]);
-                }
-                bad |= (npp[0] != npp[0]) || (npp[1] != npp[1]);
-                if (IMG) {
-                    bool im[2];
-                    float iv[2];
+            for (int a = 0; a < 2; ++a) {
+                if (OUT)
+                    o[a] = tapo(zcomp ? wrnd<T>(npp[a]) : ppt[a], a, fxc, fyr[r]);
+                else if (OUTU)
+                    o[a] = ztap[a] && z + a < tf.b - tf.hold
+                               ? tap(wrnd<T>(npp[a]), a, fxc, fyr[r])
+                               : npp[a];
+                else
+                    o[a] = npp[a];
+            }
+            st_buf2<T>(rpp, rowb[r], row && (zcomp || zframe) ? zoff : kDropped, o[0], o[1]);
+            bad |= row && zcomp && (npp[0] != npp[0] || npp[1] != npp[1]);
+            if (IMG) {
+                // a pair's cell outside [z0, z1) or under a receiver keeps its
+                // value
+                const bool rc = rcvx && ((rmask >> r) & 1u);
+                float iv[2];
 #pragma unroll
-                    for (int a = 0; a < 2; ++a) {
-                        const int za = z + a;
-                        im[a] = za >= fz.z0 && za < fz.z1 &&
-                                !(rcvx && ((rmask >> r) & 1u) && za == fz.rz);
-                        iv[a] = c_img[r][a] + c_ps[r][a] * wrnd<T>(npp[a]);
-                    }
-                    if (im[0] && im[1]) st_buf2<float>(rimg, rowb[r] * VS, zoffv, iv[0], iv[1]);
-                    else if (im[0]) st_buf<float>(rimg, rowb[r] * VS, zoffv, iv[0]);
-                    else if (im[1]) st_buf<float>(rimg, rowb[r] * VS, zoffv + 4u, iv[1]);
+                for (int a = 0; a < 2; ++a) {
+                    const int za = z + a;
+                    const bool on = za >= fz.z0 && za < fz.z1 && !(rc && za == fz.rz);
+                    iv[a] = on ? c_img[r][a] + c_ps[r][a] * wrnd<T>(npp[a]) : c_img[r][a];
                 }
+                st_buf2<float>(rimg, rowb[r] * VS,
+                               row && zcomp && z + 1 >= fz.z0 && z < fz.z1 ? zoffv : kDropped,
+                               iv[0], iv[1]);
             }
         }
         ++x;
@@ -2328,6 +2359,7 @@ bool wave2_fits(const T *P, const T *PP, const float *V, const ImageFuse *fuse, 
 {
     auto al = [](const void *p, size_t a) { return ((uintptr_t)p % a) == 0; };
     if ((g.nz & 1) || (g.sy & 1) || (g.sx & 1)) return false;
+    if (g.sx * 4 >= (long long)kDropped) return false;
     if (!al(P, 2 * sizeof(T)) || !al(PP, 2 * sizeof(T)) || !al(V, 8)) return false;
     if (fuse && (!al(fuse->ps, 2 * sizeof(T)) || !al(fuse->img, 8))) return false;
     return true;
@@ -2538,8 +2570,9 @@ hipError_t launch_radius(const T *P, T *PP, const float *V, const Coefs &cf, con
         // (plain, RBC imaging) on two-z 128 x 1 x 4 waves where pairs fit;
         // tapered ones on one-z waves (64 x 1 x 6 with imaging, 64 x 1 x 8
         // otherwise) split into tapered and untapered tiles.  Salt grid,
-        // FP16: plain 0.305 ms (one-z 0.317), untapered imaging 0.545
-        // (0.605), tapered 0.398, tapered imaging 0.672; two-z waves behind
+        // FP16: plain 0.289 ms, untapered imaging 0.52; before the branches
+        // around loads and stores went, plain 0.305 (one-z 0.317), imaging
+        // 0.545 (0.605), tapered 0.398, tapered imaging 0.672; two-z waves behind
         // the tapered tiles (launch_wave_deep2) made the HBC shot slower,
         // 4.49 s against 4.40 (the 272 deep cells fill three 128-cell tiles);
         // full rows 2 x 6: 0.546 / - / 0.562 / 0.744; pairs: 0.517 / - /
