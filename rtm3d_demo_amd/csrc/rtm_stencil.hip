@@ -361,18 +361,19 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t plane_rsrc(const void *p)
 }
 
 // A plane as a view of its size: a store at lane offset kDropped is out of
-// range of it (less the row offset, which is at least R rows) and discarded, so a plane's step has no branch around a load or a
-// store and the compiler's wait counts are exact (at a join it must assume
-// that neither branch's accesses were issued, and waits for more).  With
-// branches / so, ms: FP16 two-z waves on 592 x 592 x 336, 6 x chunks, plain 0.334 /
-// 0.294, imaging 0.600 / 0.541; FP32 one-z 8-row waves, taper3D on the output,
-// 192^3 0.060 / 0.053.
+// range of it (less the row offset, which is at least R rows) and discarded, so
+// a plane's step has no branch around a load or a store and the compiler's wait
+// counts are exact (at a join it must assume that neither branch's accesses
+// were issued, and waits for more).  With branches / so, ms: FP16 two-z waves on
+// 592 x 592 x 336, 6 x chunks, plain 0.334 / 0.294, imaging 0.600 / 0.541; FP32
+// one-z 8-row waves, taper3D on the output, 192^3 0.060 / 0.053.
 constexpr unsigned kDropped = 0xfffffff0u;
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t plane_bounded(const void *p, size_t bytes)
 {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)(unsigned)bytes,
                                              0x00020000);
 }
+
 // Loads and stores of one element of type T, widened to / rounded from
 // float.  The builtins move raw bits: reinterpret, never convert.
 template <typename T>
