@@ -500,8 +500,9 @@ int rtmhip_get_tiling(int kernel_class, int *tz, int *by, int *ry, int *xchunk);
  * each step's output with modes 3 and 4 (used when the source and receivers
  * lie off the borders, else the separate pass runs), fused on load with
  * mode 2 (upper tapers as mode 1), one in-place pass with modes 0 and 1.
- * Mode -1 restores the default: mode 4 for F32; for F16 and BF16 the upper
- * tapers in separate passes and the every-border tapers on the output.
+ * Mode -1 restores the default: mode 4 for F32; for F16 and BF16 as mode 4
+ * where nze is even, with upper tapers in separate passes in the HBC backward
+ * loop and where nze is odd.
  * Batches and fused = 2 always fuse the upper tapers on load.
  * rtmhip_get_taper_fusion returns the last mode set (-1 for the default). */
 int rtmhip_set_taper_fusion(int wave_format, int mode);

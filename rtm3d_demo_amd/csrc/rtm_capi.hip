@@ -58,13 +58,13 @@ struct State {
     bool taper_sep[3] = {false, true, true};
     int taper_all_mode[3] = {2, 2, 2};  // modeling taper3D: 0 separate, 1 on load, 2 on output
     int taper_mode[3] = {-1, -1, -1};   // the last rtmhip_set_taper_fusion mode
-    bool taper_outu[3] = {true, false, false};  // forward upper tapers on the output
+    bool taper_outu[3] = {true, true, true};  // forward upper tapers on the output
 };
 constexpr bool kTaperSepDefault[3] = {false, true, true};
-// forward upper tapers on the output by default for F32; for 16-bit fields
-// the separate pass before the two-z step is as fast (salt grid, 300 forward
-// steps: FP32 0.136 s against 0.154 fused on load; FP16 0.110 against 0.107)
-constexpr bool kTaperOutDefault[3] = {true, false, false};
+// the forward (and snapshot receiver) upper tapers on the output by default;
+// for 16-bit fields on rows of pairs (upper_on_output).  FP32, 300 forward
+// steps on the salt grid: 0.136 s against 0.154 fused on load
+constexpr bool kTaperOutDefault[3] = {true, true, true};
 
 State g_state;
 thread_local std::string g_err;
@@ -273,6 +273,18 @@ bool off_borders(const rtmhip_shot *shot, const ShotCtx &c)
     return in(c.rz, c.g.nz) && in(c.rx0, c.g.nx) && in(c.ry0, c.g.ny) &&
            in(c.rx0 + (long long)(r.count_x - 1) * r.dist_x, c.g.nx) &&
            in(c.ry0 + (long long)(r.count_y - 1) * r.dist_y, c.g.ny);
+}
+
+// The upper taper goes onto each forward step's output.  16-bit fields by
+// default only where the two-z waves run (pairs: even rows and planes): FP16,
+// us a step, own pass / on the output: 592 x 592 x 336 330 / 322, 192^3 30.3 / 27.5,
+// 96^3 14.5 / 12.1, but odd rows 301 x 277 x 259 70.5 / 71.7 (BF16 70.4 / 73.4),
+// 400 x 260 x 161 60.1 / 60.5 (59.7 / 62.2).
+bool upper_on_output(int fmt, const Grid &g)
+{
+    if (!g_state.taper_outu[fmt]) return false;
+    return fmt == RTMHIP_WAVE_F32 || g_state.taper_mode[fmt] >= 0 ||
+           ((g.nz | g.sy | g.sx) & 1) == 0;
 }
 
 // The shot's receivers of one record chunk at time lt (mode as TailReceivers).
@@ -746,13 +758,13 @@ int forward_loop(const rtmhip_shot *shot, const ShotCtx &c, int hbc, const float
     //   twice -- once on the first step of a call, whose PP already carries
     //   one taper; the taper still pending on P is applied in place after the
     //   last step, so the state between calls is the reference's.
-    // * separate (mode 0, the 16-bit default): the two tapers run in place
+    // * separate (mode 0): the two tapers run in place
     //   (one pass over both fields) before a plain step, as the reference
     //   orders them.
     const bool sep = g_state.taper_sep[shot->wave_format];
     const int b = shot->blen;
     // (b >= 2R keeps the layer off the z frame)
-    const bool outu = hbc && g_state.taper_outu[shot->wave_format] && c.radius == 4 &&
+    const bool outu = hbc && upper_on_output(shot->wave_format, c.g) && c.radius == 4 &&
                       shot->sze >= b && b >= 2 * c.radius;
     const size_t layer = (size_t)c.g.nx * c.g.ny * c.hf;
     for (int it = it0; it < it0 + nsteps; ++it) {
@@ -966,7 +978,7 @@ int snap_forward_run(const rtmhip_shot *shot, const ShotCtx &c, const float *V2D
     const bool sep = g_state.taper_sep[shot->wave_format];
     // the upper taper on the output as in forward_loop (no history planes
     // held: the snapshots cover z >= blen only)
-    const bool outu = g_state.taper_outu[shot->wave_format] && c.radius == 4 && shot->sze >= b;
+    const bool outu = upper_on_output(shot->wave_format, c.g) && c.radius == 4 && shot->sze >= b;
     for (int it = it0; it < it0 + nsteps; ++it) {
         T *t = *P;
         *P = *PP;
@@ -1034,7 +1046,7 @@ int snap_backward_run(const rtmhip_shot *shot, const ShotCtx &c, const float *V2
     const bool sep = g_state.taper_sep[shot->wave_format];
     // the receiver-only steps take the upper taper on the output like the
     // forward loops (the receivers and the imaged range lie at z >= blen)
-    const bool outu = g_state.taper_outu[shot->wave_format] && c.radius == 4 && c.rz >= b;
+    const bool outu = upper_on_output(shot->wave_format, c.g) && c.radius == 4 && c.rz >= b;
     for (int it = it_hi; it > it_hi - nsteps; --it) {
         TailLayer<T> w{0, 0, nullptr, nullptr, nullptr};  // the frame after the step
         if (outu && it > it_hi - nsteps + 1) {
@@ -1569,9 +1581,10 @@ int batch_tab(const rtmhip_batch *b, int cls) { return b->mode[cls] == 6 ? 0 : 1
 // per-shot launches, and every source lies at z >= blen.
 bool batch_fwd_out(const rtmhip_batch *b)
 {
-    if (!g_state.taper_outu[b->wave_format] || b->mode[2] || b->radius != 4) return false;
+    if (b->mode[2] || b->radius != 4) return false;
     for (int i = 0; i < b->n; ++i) {
         const BatchShot &h = b->hs[0][i];
+        if (!upper_on_output(b->wave_format, h.g)) return false;
         if (h.src_off % h.g.sy < b->blen) return false;
     }
     return true;

@@ -476,8 +476,8 @@ def set_taper_fusion(fmt, mode):
     off the borders, else the separate pass runs); 4: also the forward
     loops' upper tapers applied to each step's output (backward loops fused
     on load); 0: separate in-place passes; -1: the format's default (F32:
-    mode 4; 16-bit formats: upper tapers in separate passes, every-border
-    tapers on the output)."""
+    mode 4; 16-bit formats: as mode 4, but the HBC backward loop and odd
+    rows in separate passes)."""
     check(load().rtmhip_set_taper_fusion(WAVE_FORMATS[fmt][0], mode))
 
 
