@@ -19,6 +19,7 @@
 #include "rtm_internal.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace rtmhip {
 namespace {
@@ -226,7 +227,9 @@ __global__ void __launch_bounds__(kCutThreads)
 // of a 16 x 16 tile -- is the second product's B operand as it stands: the
 // second product's weights take the k order {4 g + v, 16 + 4 g + v} instead of the
 // natural one, and no value crosses lanes.  The 8 x 8 layers take four
-// patches at a time as one 32 x 32 block-diagonal product (K = 32 filled).
+// patches at a time as one 32 x 32 block-diagonal product (K = 32 filled); where
+// an infinity or a NaN meets the zeros off its diagonal, one patch at a time
+// (patch_product), so that no patch hears of another's.
 // Rounding is the separate layers': FP16 operands, FP32 sums, bias and tanh
 // in FP32, FP16 again for the next layer.
 //
@@ -245,6 +248,27 @@ constexpr long long kOffW1 = 0, kOffB1 = 64, kOffW2 = 72, kOffB2 = kOffW2 + 512 
 __device__ __forceinline__ int frag_pos(int i, int k)
 {
     return (i + 16 * ((k >> 2) & 3)) * 8 + (k & 3) + 4 * (k >> 4);
+}
+
+// A tile of the block-diagonal product of four patches, one patch's operand at
+// a time, the others' zeroed: kp(s) is the patch of slot s, op(v) that of
+// result item v.
+template <typename K, typename O>
+__device__ __forceinline__ float4_t patch_product(const half8_t &a, const half8_t &b, K &&kp,
+                                                  O &&op)
+{
+    const float4_t zero = {0.f, 0.f, 0.f, 0.f};
+    float4_t d = zero;
+#pragma unroll 1
+    for (int p = 0; p < 4; ++p) {
+        half8_t m;
+#pragma unroll
+        for (int s = 0; s < 8; ++s) m[s] = kp(s) == p ? b[s] : (_Float16)0.f;
+        const float4_t dp = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, m, zero, 0, 0, 0);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) d[v] = op(v) == p ? dp[v] : d[v];
+    }
+    return d;
 }
 
 __global__ void __launch_bounds__(kAeThreads)
@@ -277,14 +301,19 @@ __global__ void __launch_bounds__(kAeThreads)
     if (c >= chunks) return;
     {
         const _Float16 *x = X + (c * 16 + j) * 512 + g * 8;
-        float4_t acc[2] = {zero, zero};
-#pragma unroll
+        float4_t acc[2];
+        auto layers = [&]<bool apart>(std::bool_constant<apart>) {
+        acc[0] = acc[1] = zero;
+#pragma unroll(apart ? 1 : 16)
         for (int q = 0; q < 16; ++q) {
             const half8_t xb = *reinterpret_cast<const half8_any *>(x + q * 32);
             half8_t h;
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
-                const float4_t d = __builtin_amdgcn_mfma_f32_16x16x32_f16(w1[t], xb, zero, 0, 0, 0);
+                const float4_t d =
+                    apart ? patch_product(w1[t], xb, [&](int) { return g; },
+                                          [&](int) { return 2 * t + (g >> 1); })
+                          : __builtin_amdgcn_mfma_f32_16x16x32_f16(w1[t], xb, zero, 0, 0, 0);
 #pragma unroll
                 for (int v = 0; v < 4; ++v) h[4 * t + v] = wst<_Float16>(tanhf(d[v] + b1[v]));
             }
@@ -294,6 +323,10 @@ __global__ void __launch_bounds__(kAeThreads)
                     *reinterpret_cast<const half8_t *>(&w2[((q * 2 + t) * 64 + lane) * 8]), h,
                     acc[t], 0, 0, 0);
         }
+        };
+        layers(std::false_type{});
+        // a NaN anywhere in a row makes all its codes NaN
+        if (__any(acc[0][0] != acc[0][0])) layers(std::true_type{});
         _Float16 *z = codes + (c * 16 + j) * 32 + 4 * g;
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
@@ -352,7 +385,10 @@ __global__ void __launch_bounds__(kAeThreads)
         const int x0 = r.x0 + 32 * bx + 8 * ax + (g >> 1);
         const int y0 = r.y0 + 32 * by + 8 * (j >> 2);
         const int z0 = r.z0 + 32 * bz + 8 * (j & 3) + 4 * (g & 1);
-#pragma unroll
+        float4_t nans = zero;  // 0, or NaN in a column with a NaN
+        const half8_t none = {};
+        auto layers = [&]<bool apart>(std::bool_constant<apart>) {
+#pragma unroll(apart ? 1 : 16)
         for (int q = 0; q < 16; ++q) {
             half8_t h;
 #pragma unroll
@@ -365,11 +401,17 @@ __global__ void __launch_bounds__(kAeThreads)
 #pragma unroll
                 for (int v = 0; v < 4; ++v) h[4 * t + v] = wst<_Float16>(tanhf(d[v] + bb[v]));
             }
+            if (!apart)
+                nans = __builtin_amdgcn_mfma_f32_16x16x32_f16(none, h, nans, 0, 0, 0);
             const int x = x0 + 2 * (q >> 2), y = y0 + 2 * (q & 3);
             float *p = F + (long long)x * gr.sx + (long long)y * gr.sy + z0;
 #pragma unroll
             for (int t = 0; t < 2; ++t, p += gr.sy) {
-                const float4_t d = __builtin_amdgcn_mfma_f32_16x16x32_f16(w4[t], h, zero, 0, 0, 0);
+                const float4_t d =
+                    apart ? patch_product(
+                                w4[t], h, [&](int s) { return (g >> 1) + 2 * (s >> 2); },
+                                [&](int v) { return 2 * (g & 1) + (v >> 1); })
+                          : __builtin_amdgcn_mfma_f32_16x16x32_f16(w4[t], h, zero, 0, 0, 0);
                 float4_t o;
 #pragma unroll
                 for (int v = 0; v < 4; ++v) o[v] = (d[v] + b4[t][v & 1]) * scale;
@@ -384,6 +426,9 @@ __global__ void __launch_bounds__(kAeThreads)
                 }
             }
         }
+        };
+        layers(std::false_type{});
+        if (__any(nans[0] != nans[0])) layers(std::true_type{});
     }
 }
 
@@ -437,6 +482,22 @@ __global__ void __launch_bounds__(kAeThreads)
             for (int i = 0; i < 4; ++i) h[4 * t + i] = wst<_Float16>(v[t][i]);
         return h;
     };
+    // both tiles of a block-diagonal product (kp as in patch_product)
+    auto diagonal = [&](const half8_t(&a)[2], const half8_t &b, float4_t(&d)[2], auto kp) {
+        float s = 0.f;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            d[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[t], b, zero, 0, 0, 0);
+            s += d[t][0] + d[t][1] + d[t][2] + d[t][3];
+        }
+        if (__any(s != s)) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+                d[t] = patch_product(a[t], b, kp, [&](int) { return 2 * t + (g >> 1); });
+        }
+    };
+    auto natural = [&](int) { return g; };                       // k = 8 g + s
+    auto result = [&](int s) { return (g >> 1) + 2 * (s >> 2); };  // k = kel(s)
     // 32 elements of the lane's row into LDS, element-major
     auto put = [&](_Float16(*dst)[kRowPad], const half8_t &h) {
 #pragma unroll
@@ -476,19 +537,22 @@ __global__ void __launch_bounds__(kAeThreads)
 #pragma unroll
                     for (int v = 0; v < 4; ++v) xd[q][4 * t + v] = u[v];
                 }
+                half8_t a1[2];
 #pragma unroll
                 for (int t = 0; t < 2; ++t) {
                     const int o = 16 * t + j;  // row: patch o / 8, channel o % 8
-                    half8_t a;
 #pragma unroll
                     for (int s = 0; s < 8; ++s)
-                        a[s] = (o >> 3) == g ? (_Float16)wt[kOffW1 + s * 8 + (o & 7)]
-                                             : (_Float16)0.f;
-                    const float4_t d = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, xb, zero, 0, 0, 0);
+                        a1[t][s] = (o >> 3) == g ? (_Float16)wt[kOffW1 + s * 8 + (o & 7)]
+                                                 : (_Float16)0.f;
+                }
+                float4_t d[2];
+                diagonal(a1, xb, d, natural);
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
 #pragma unroll
                     for (int v = 0; v < 4; ++v)
-                        h1[q][t][v] = tanhf(d[v] + wt[kOffB1 + ((4 * g + v) & 7)]);
-                }
+                        h1[q][t][v] = tanhf(d[t][v] + wt[kOffB1 + ((4 * g + v) & 7)]);
                 const half8_t h = half8(h1[q]);
                 const float *w2 = wt + kOffW2 + (wv * 64 + q * 32) * 32 + j;
 #pragma unroll
@@ -533,19 +597,23 @@ __global__ void __launch_bounds__(kAeThreads)
                     h3[t][v] = tanhf(d[v] + wt[kOffB3 + wv * 64 + q * 32 + 16 * t + 4 * g + v]);
             }
             const half8_t h3h = half8(h3);
+            half8_t a4[2];
+            float4_t d4[2];
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
                 const int o = 16 * t + j;
-                half8_t a;
 #pragma unroll
                 for (int s = 0; s < 8; ++s)
-                    a[s] = (o >> 3) == (kel(s) >> 3)
-                               ? (_Float16)wt[kOffW4 + (kel(s) & 7) * 8 + (o & 7)]
-                               : (_Float16)0.f;
-                const float4_t d = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, h3h, zero, 0, 0, 0);
+                    a4[t][s] = (o >> 3) == (kel(s) >> 3)
+                                   ? (_Float16)wt[kOffW4 + (kel(s) & 7) * 8 + (o & 7)]
+                                   : (_Float16)0.f;
+            }
+            diagonal(a4, h3h, d4, result);
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
-                    dy[t][v] = d[v] + wt[kOffB4 + ((4 * g + v) & 7)] - (float)xd[q][4 * t + v];
+                    dy[t][v] = d4[t][v] + wt[kOffB4 + ((4 * g + v) & 7)] - (float)xd[q][4 * t + v];
                     loss += dy[t][v] * dy[t][v];
                     gb4[v] += dy[t][v];
                 }
@@ -557,16 +625,18 @@ __global__ void __launch_bounds__(kAeThreads)
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
                 const int o = 16 * t + j;
-                half8_t a;
 #pragma unroll
                 for (int s = 0; s < 8; ++s)
-                    a[s] = (o >> 3) == (kel(s) >> 3)
-                               ? (_Float16)wt[kOffW4 + (o & 7) * 8 + (kel(s) & 7)]
-                               : (_Float16)0.f;
-                const float4_t d = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, dyh, zero, 0, 0, 0);
+                    a4[t][s] = (o >> 3) == (kel(s) >> 3)
+                                   ? (_Float16)wt[kOffW4 + (o & 7) * 8 + (kel(s) & 7)]
+                                   : (_Float16)0.f;
+            }
+            diagonal(a4, dyh, d4, result);
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
-                    d3[q][t][v] = d[v] * (1.0f - h3[t][v] * h3[t][v]);
+                    d3[q][t][v] = d4[t][v] * (1.0f - h3[t][v] * h3[t][v]);
                     gb3[q][t][v] += d3[q][t][v];
                 }
             }

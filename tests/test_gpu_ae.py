@@ -220,6 +220,67 @@ def test_gradient_over_tiles(gpu, n):
     dB.free()
 
 
+def test_infinities_stay_in_their_patch(gpu):
+    """Four 2^3 patches share a matrix product, block-diagonal: a patch with an
+    infinite cell, or whose hidden values or residual are not finite, leaves
+    the others' values alone.  Tolerances as above (FP16 operands)."""
+    from rtm3d_demo_amd import ae
+    rng = np.random.default_rng(31)
+    n = 3
+    B = np.clip(0.4 * rng.standard_normal((n, ae.BRICK)), -1, 1).astype(np.float16)
+    B[0, 8 * 77 + 3] = np.inf
+    B[2, 8 * 4000 + 1] = -np.inf
+    codec = ae.Codec(max_bricks=n, seed=3)
+    p = codec.params().astype(np.float64)
+    p += rng.uniform(-0.05, 0.05, p.shape)
+    # two code channels that add in every column of layer 3 but one
+    W3 = ao.unpack(p)[2][0]
+    W3[4], W3[9] = 0.25, 0.5
+    W3[9, 8 * 21 + 6] = -0.5
+    codec.set_params(p.astype(np.float32))
+    p = codec.params().astype(np.float64)
+    dB = gpu.DeviceArray.from_host(B.view(np.uint16), np.uint16)
+    dC = gpu.DeviceArray((n, ao.CODES), np.uint16)
+    codec.encode(dB, n, dC)
+    codes = dC.download().view(np.float16)
+    want = ao.encode(p, B)  # tanh(+-inf) = +-1: every code is finite
+    assert np.isfinite(want).all()
+    assert _rel(codes, want) < 5e-3
+
+    # decoding: infinite codes cancel to NaN in patch 21 of one row only
+    Z = want.astype(np.float16)
+    Z[1].reshape(64, 32)[13, [4, 9]] = np.inf
+    dC.upload(Z.view(np.uint16))
+    S = np.ones(n, np.float32)
+    dS = gpu.DeviceArray.from_host(S)
+    region, shape = (0, 0, 0, 96, 32, 32), (96, 32, 32)
+    dF = gpu.DeviceArray(shape).zero()
+    codec.decode(dC, dS, n, dF, region)
+    want_f = np.zeros(shape, np.float32)
+    with np.errstate(invalid="ignore"):
+        ao.unbricks(ao.decode(p, Z.astype(np.float64)), S, want_f, region)
+    got = dF.download()
+    bad = np.isnan(want_f)
+    assert bad.sum() == 8
+    assert np.array_equal(np.isnan(got), bad)
+    assert _rel(got[~bad], want_f[~bad].astype(np.float64)) < 5e-3
+
+    # gradient: the same parameters are finite, infinite or NaN
+    with np.errstate(invalid="ignore"):
+        want_loss, want_g = ao.loss_and_grad(p, B.astype(np.float64))
+    loss, g = codec.gradient(dB, n)
+    assert np.isinf(want_loss) and loss == want_loss
+    assert np.isfinite(want_g).any() and not np.isfinite(want_g).all()
+    assert np.array_equal(np.isnan(g), np.isnan(want_g))
+    inf = np.isinf(want_g)
+    assert np.array_equal(g[inf].astype(np.float64), want_g[inf])
+    fin = np.isfinite(want_g)
+    assert _rel(g[fin], want_g[fin]) < 2e-2
+    codec.destroy()
+    for d in (dB, dC, dS, dF):
+        d.free()
+
+
 def _salt_case(gpu, seed_src):
     from rtm3d_demo_amd import host, workloads
     vel = workloads.salt_model(64, 64, 64, seed=2024)
