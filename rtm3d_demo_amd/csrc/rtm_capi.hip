@@ -763,9 +763,13 @@ int forward_loop(const rtmhip_shot *shot, const ShotCtx &c, int hbc, const float
     //   orders them.
     const bool sep = g_state.taper_sep[shot->wave_format];
     const int b = shot->blen;
-    // (b >= 2R keeps the layer off the z frame)
+    // (by default 16-bit fields only with b >= 2R: FP16, 592 x 592 x 336, us a
+    // step with the pass of its own / so: b = 6 308 / 313, b = 40 330 / 322.
+    // FP32, b = 6: on load 431, so 372)
     const bool outu = hbc && upper_on_output(shot->wave_format, c.g) && c.radius == 4 &&
-                      shot->sze >= b && b >= 2 * c.radius;
+                      shot->sze >= b &&
+                      (std::is_same<T, float>::value || b >= 2 * c.radius ||
+                       g_state.taper_mode[shot->wave_format] >= 0);
     const size_t layer = (size_t)c.g.nx * c.g.ny * c.hf;
     for (int it = it0; it < it0 + nsteps; ++it) {
         // history layer: every step held (hbc 1) or one receiver chunk (hbc 2)

@@ -1167,7 +1167,8 @@ __global__ void __launch_bounds__(kThreads)
 //           and then, with hold (a step that left the layer untapered),
 //           tapered once;
 //   frame   the cells of PP's slab frame tapered `taps` times (outside the
-//           layer with hold: the layer's items do those);
+//           layer with hold: the layer's items do those, which for b < 2R
+//           are z < R cells too);
 //   rcv     the receivers of PP;  image  img += ps * PP on the imaged cells
 //           that the step does not visit;  src  the source cell of PP.
 //
@@ -1236,26 +1237,32 @@ __global__ void __launch_bounds__(kThreads)
             const float fy = by ? gfac(t, y, g.ny, b) : 1.0f;
             const float fx = bx ? gfac(t, x, g.nx, b) : 1.0f;
             const bool rim = x < R || x >= g.nx - R || y < R || y >= g.ny - R;
-            auto taper = [&](int taps) {
+            // cells e < n of the run
+            auto taper = [&](int taps, int n) {
                 for (int k = 0; k < taps; ++k)
 #pragma unroll
                     for (int e = 0; e < R; ++e) {
                         float w = wld(v[e]) * fy;
                         w *= fx;
                         w *= t[b - 1 - z - e];
-                        v[e] = wst<T>(w);
+                        if (e < n) v[e] = wst<T>(w);
                     }
             };
             if (!lay) {
-                taper(u.taps);
+                taper(u.taps, R);
+                if (u.hold && b < 2 * R) {  // z >= b - R: the layer's
+#pragma unroll
+                    for (int e = 0; e < R; ++e)
+                        if (e < b - R) PP[o + e] = v[e];
+                    return;
+                }
                 st_run<T, R, VEC>(PP + o, v);
                 return;
             }
-            // a row of the frame; elsewhere the step tapers nothing here
-            // (b >= 2R, or its z < R cells would be frame cells too)
-            if (rim) taper(u.taps - 1);
+            // the frame's cells: a whole row of the rim, else z < R
+            taper(u.taps - 1, rim ? R : 2 * R - b);
             st_run<T, R, VEC>(save + (long long)row * R, v);
-            taper(1);
+            taper(1, R);
             st_run<T, R, VEC>(PP + o, v);
             return;
         }
@@ -1691,7 +1698,7 @@ hipError_t launch_tail_upper(T *PP, const float *taper, const Grid &g, int b, in
         nf = tail_frame_count(g, b, R) - rows * R;
     }
     if (img) ni = (long long)2 * R * (g.ny + g.nx - 2 * R) * std::max(0, z1 - z0);
-    if (w.hold && (!w.save || w.taps < 1 || b < 2 * R)) return hipErrorInvalidValue;
+    if (w.hold && (!w.save || w.taps < 1)) return hipErrorInvalidValue;
     if ((nl || nf) && b < R) return hipErrorInvalidValue;
     const long long n = nl + na + nf + (r.mode ? (long long)r.rnx * r.rny : 0) + ni + 1;
     if (n + kThreads >= (1LL << 31) || (nl && rows * R >= (1LL << 31)))

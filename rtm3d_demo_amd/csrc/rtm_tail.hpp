@@ -32,7 +32,7 @@ hipError_t launch_tail_all(T *PP, const float *taper, const Grid &g, int b, int 
 // (at most one), the receivers, with img the imaging condition img += ps * PP
 // off the step's cells, the source (z >= b).  hold: the step left the layer
 // untapered; it is saved with its frame cells tapered taps - 1 times, then
-// tapered once (b >= 2R).
+// tapered once.
 template <typename T>
 struct TailLayer {
     int taps, hold;
