@@ -178,6 +178,36 @@ __device__ __forceinline__ void taper_edge(T *__restrict__ p, const float *__res
     }
 }
 
+// The same for the group at p, by vectors and with eight factors loaded at a
+// time.  us (a launch of its own before the tapers, cell by cell, so): FP32
+// field, border 40, 96^3 7.2, 10.4, 6.6; 192^3 12.1, 15.1, 10.7; two FP16 fields
+// and a step, border 24, 96^3 19.1, 21.9, 15.6; 192^3 38.3, 41.9, 33.9.
+template <typename T>
+__device__ __forceinline__ void taper_edge_group(T *__restrict__ p, const float *__restrict__ t,
+                                                 const Grid &g, int b, float gy)
+{
+    constexpr int U = 8;
+    const Group16<T> v = *reinterpret_cast<const Group16<T> *>(p);
+    p -= (long long)b * g.sx;
+    for (int x0 = 0; x0 < b; x0 += U) {
+        float f[U];
+#pragma unroll
+        for (int k = 0; k < U; ++k) f[k] = t[max(b - 1 - x0 - k, 0)];
+#pragma unroll
+        for (int k = 0; k < U; ++k) {
+            if (x0 + k >= b) break;
+            Group16<T> w;
+#pragma unroll
+            for (int e = 0; e < Group16<T>::G; ++e) {
+                float a = wld(v.v[e]) * f[k];
+                a *= gy;
+                w.v[e] = wst<T>(a);
+            }
+            *reinterpret_cast<Group16<T> *>(p + (long long)(x0 + k) * g.sx) = w;
+        }
+    }
+}
+
 // taper3D over 16-byte groups (the front-right edge's interior-z cells by the
 // threads of plane b): the z-border groups of the rows with x and y interior,
 // then every group of the rows with x or y in a border, as k_taper_all.
@@ -234,9 +264,7 @@ __global__ void __launch_bounds__(kThreads)
     } else {
         // (bx and by: gx gy) | gy | gx
         taper_group(p, t, z0, g.nz, b, bx ? gx : gy, bx && by ? gy : 1.0f, false, 0);
-        if (!bx && x == b && y >= g.ny - b)
-            for (int k = 0; k < G; ++k)
-                taper_edge(p + k - (long long)b * g.sx, t, g, b, wld(p[k]), gy);
+        if (!bx && x == b && y >= g.ny - b) taper_edge_group(p, t, g, b, gy);
     }
 }
 

@@ -92,3 +92,12 @@ def test_model_steps_match_operator_sequence(gpu, oracle, fmt, shape, b, splits,
     assert np.array_equal(got_rec.view(np.uint32), rec.view(np.uint32))
     assert np.array_equal(gotP.view(np.uint8), P.view(np.uint8))
     assert np.array_equal(gotPP.view(np.uint8), PP.view(np.uint8))
+
+
+@pytest.mark.parametrize("shape, b", [((40, 44, 96), 8), ((44, 40, 72), 16), ((60, 64, 56), 24)])
+@pytest.mark.parametrize("fmt", ["f32", "f16", "bf16"])
+def test_separate_pass_in_groups(gpu, oracle, fmt, shape, b):
+    """Borders and rows of whole 16-byte groups for every format: the separate
+    pass moves groups, the front-right edge with them, below, at and past eight
+    planes."""
+    test_model_steps_match_operator_sequence(gpu, oracle, fmt, shape, b, (2, 1, 2), 0, RCV_IN, None)
