@@ -1728,6 +1728,8 @@ hipError_t launch_tail_upper(T *PP, const float *taper, const Grid &g, int b, in
     if (img) ni = (long long)2 * R * (g.ny + g.nx - 2 * R) * std::max(0, z1 - z0);
     if (w.hold && (!w.save || w.taps < 1)) return hipErrorInvalidValue;
     if ((nl || nf) && b < R) return hipErrorInvalidValue;
+    // the slab frame numbers its cells in 32 bits, the z < R ones first
+    if (na && rows * R + nf + kThreads >= (1LL << 31)) return hipErrorInvalidValue;
     const long long n = nl + na + nf + (r.mode ? (long long)r.rnx * r.rny : 0) + ni + 1;
     if (n + kThreads >= (1LL << 31) || (nl && rows * R >= (1LL << 31)))
         return hipErrorInvalidValue;

@@ -1,0 +1,87 @@
+"""Which counts the launches after a step take: the launchers number cells in 32
+bits and must refuse what would overflow, and only that.  A small program
+calls them without a device (so nothing is ever launched) and prints each
+result: hipErrorInvalidValue where the launcher refused, another error where it
+went on to launch.
+"""
+import os
+import subprocess
+
+import pytest
+
+from rtm3d_demo_amd import build
+
+REFUSED = 1  # hipErrorInvalidValue
+
+PROGRAM = r"""
+#include "rtm_internal.hpp"
+#include "rtm_tail.hpp"
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+using namespace rtmhip;
+static Grid grid(int nx, int ny, int nz)
+{
+    Grid g{};
+    g.nx = nx;
+    g.ny = ny;
+    g.nz = nz;
+    g.sy = nz;
+    g.sx = (long long)ny * nz;
+    return g;
+}
+int main(int argc, char **argv)
+{
+    int n = 0;
+    if (hipGetDeviceCount(&n) == hipSuccess && n > 0) return 2;
+    (void)hipGetLastError();
+    const auto arg = [&](int i) { return atoi(argv[i]); };
+    const Grid g = grid(arg(2), arg(3), arg(4));
+    const int b = arg(5), R = arg(6), taps = arg(7);
+    float *p = reinterpret_cast<float *>(4096);
+    const TailSource src{p, (long long)g.nx / 2 * g.sx + g.ny / 2 * g.sy + g.nz / 2, 0};
+    hipError_t e;
+    if (!strcmp(argv[1], "all")) {
+        e = launch_tail_all<float>(p, p, g, b, R, taps, nullptr, &src, nullptr);
+    } else {
+        const bool layer = arg(8), image = arg(9);
+        const TailLayer<float> w{taps, 0, nullptr, p, layer ? p : nullptr};
+        e = launch_tail_upper<float>(p, p, g, b, R, w, nullptr, &src, image ? p : nullptr, p,
+                                     nullptr);
+    }
+    printf("%d\n", (int)e);
+    return 0;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def program(tmp_path_factory):
+    d = tmp_path_factory.mktemp("limits")
+    src, exe = d / "limits.hip", d / "limits"
+    src.write_text(PROGRAM)
+    subprocess.run([build.HIPCC, *build.HIP_FLAGS, "-I" + build.CSRC, "--cuda-host-only",
+                    "-c", str(src), "-o", str(d / "limits.o")], check=True, capture_output=True)
+    subprocess.run([build.HIPCC, str(d / "limits.o"), "-o", str(exe), "-L" + build.LIBDIR,
+                    "-lrtm3d_hip", "-Wl,-rpath," + build.LIBDIR], check=True, capture_output=True)
+    return str(exe)
+
+
+def _result(program, *args):
+    env = dict(os.environ, HIP_VISIBLE_DEVICES="-1", ROCR_VISIBLE_DEVICES="")
+    r = subprocess.run([program, *map(str, args)], env=env, capture_output=True, text=True,
+                       timeout=60)
+    assert r.returncode == 0, r
+    return int(r.stdout)
+
+
+@pytest.mark.parametrize("grid, R, layer, refused", [
+    ((23171, 23170, 9), 4, 0, True),   # 2^31 + 4632 cells with z < R
+    ((23171, 23170, 9), 4, 1, True),
+    ((23000, 23000, 9), 4, 0, False),  # 2.116e9
+    ((46340, 46340, 9), 1, 0, True),   # 2^31 - 88048 with z < R, 556068 on the rims
+    ((46340, 46300, 9), 1, 0, False),  # 2145542000 and 555828
+])
+def test_slab_frame_bound(program, grid, R, layer, refused):
+    b = 4
+    assert (_result(program, "upper", *grid, b, R, 2, layer, 0) == REFUSED) == refused
