@@ -1664,6 +1664,16 @@ TailRcv tail_rcv(const TailReceivers *r)
     return o;
 }
 
+// A launch numbers its items in 32 bits; parts that fit by themselves but not
+// together go in launches of their own (their cells are disjoint).
+bool tail_items_fit(long long n) { return n + kThreads < (1LL << 31); }
+
+// The items of the receivers and the source.
+long long tail_points(const TailRcv &r, const TailSrc &q)
+{
+    return (r.mode ? (long long)r.rnx * r.rny : 0) + (q.table ? 1 : 0);
+}
+
 // The source, and whether a sampled receiver sits on its cell.
 TailSrc tail_src(const TailSource *q, const TailRcv &r, const Grid &g)
 {
@@ -1696,14 +1706,22 @@ hipError_t launch_tail_all(T *PP, const float *taper, const Grid &g, int b, int 
         nF = nX + (long long)(g.nx - 2 * R) * 2 * R * g.nz;
         nQ = (long long)b * (b - R) * (g.nz - 2 * b);
     }
-    const long long n = nF + nQ + (r.mode ? (long long)r.rnx * r.rny : 0) + 1;
-    if (n + kThreads >= (1LL << 31)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_tail_all<T>, dim3(nblocks(n)), dim3(kThreads), 0, s, PP, taper, g, b, R,
-                       taps, (int)nX, (int)nF, (int)nQ, fast_div((uint32_t)g.nz),
-                       fast_div((uint32_t)g.ny), fast_div((uint32_t)(2 * R)),
-                       fast_div((uint32_t)std::max(1, g.nz - 2 * b)),
-                       fast_div((uint32_t)std::max(1, b - R)), r, q);
-    return hipGetLastError();
+    const auto go = [&](long long frame, long long edge, const TailRcv &rc, const TailSrc &sr) {
+        const long long n = frame + edge + tail_points(rc, sr);
+        if (n <= 0) return hipSuccess;
+        if (!tail_items_fit(n)) return hipErrorInvalidValue;
+        hipLaunchKernelGGL(k_tail_all<T>, dim3(nblocks(n)), dim3(kThreads), 0, s, PP, taper, g, b,
+                           R, taps, (int)std::min(nX, frame), (int)frame, (int)edge,
+                           fast_div((uint32_t)g.nz), fast_div((uint32_t)g.ny),
+                           fast_div((uint32_t)(2 * R)),
+                           fast_div((uint32_t)std::max(1, g.nz - 2 * b)),
+                           fast_div((uint32_t)std::max(1, b - R)), rc, sr);
+        return hipGetLastError();
+    };
+    if (tail_items_fit(nF + nQ + tail_points(r, q))) return go(nF, nQ, r, q);
+    hipError_t e = go(nF, 0, TailRcv{}, TailSrc{});
+    if (e == hipSuccess) e = go(0, nQ, TailRcv{}, TailSrc{});
+    return e == hipSuccess ? go(0, 0, r, q) : e;
 }
 
 template <typename T>
@@ -1728,15 +1746,10 @@ hipError_t launch_tail_upper(T *PP, const float *taper, const Grid &g, int b, in
     if (img) ni = (long long)2 * R * (g.ny + g.nx - 2 * R) * std::max(0, z1 - z0);
     if (w.hold && (!w.save || w.taps < 1)) return hipErrorInvalidValue;
     if ((nl || nf) && b < R) return hipErrorInvalidValue;
-    // the slab frame numbers its cells in 32 bits, the z < R ones first
-    if (na && rows * R + nf + kThreads >= (1LL << 31)) return hipErrorInvalidValue;
-    const long long n = nl + na + nf + (r.mode ? (long long)r.rnx * r.rny : 0) + ni + 1;
-    if (n + kThreads >= (1LL << 31) || (nl && rows * R >= (1LL << 31)))
-        return hipErrorInvalidValue;
-    u.nl = (int)nl;
-    u.na = (int)na;
-    u.nf = (int)nf;
-    u.ni = (int)ni;
+    // 32-bit cell numbers: in the layer, and in the slab frame with its z < R
+    // cells first
+    if (nl && !tail_items_fit(rows * R)) return hipErrorInvalidValue;
+    if (na && !tail_items_fit(rows * R + nf)) return hipErrorInvalidValue;
     u.fd = frame_divs(R, b - R, g.ny);
     u.id = frame_divs(R, z1 - z0, g.ny);
     u.dny = fast_div((uint32_t)g.ny);
@@ -1745,18 +1758,32 @@ hipError_t launch_tail_upper(T *PP, const float *taper, const Grid &g, int b, in
     const auto al = [](const void *p) { return ((uintptr_t)p % (4 * sizeof(T))) == 0; };
     const bool vec = R == 4 && ((g.sy | b) & 3) == 0 && (g.sx & 3) == 0 && al(PP) && al(w.save) &&
                      al(w.field) && al(w.restore);
-    const auto go = [&](auto kern) {
-        hipLaunchKernelGGL(kern, dim3(nblocks(n)), dim3(kThreads), 0, s, PP, taper, g, b, u,
-                           w.save, w.field, w.restore, r, q, img, ps);
-        return hipGetLastError();
+    const auto go = [&](long long lay, long long frows, long long frame, long long image,
+                        const TailRcv &rc, const TailSrc &sr) {
+        const long long n = lay + frows + frame + image + tail_points(rc, sr);
+        if (n <= 0) return hipSuccess;
+        if (!tail_items_fit(n)) return hipErrorInvalidValue;
+        u.nl = (int)lay;
+        u.na = (int)frows;
+        u.nf = (int)frame;
+        u.ni = (int)image;
+        const auto run = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3(nblocks(n)), dim3(kThreads), 0, s, PP, taper, g, b, u,
+                               w.save, w.field, w.restore, rc, sr, img, ps);
+            return hipGetLastError();
+        };
+        switch (R) {
+        case 4: return vec ? run(k_tail_upper<T, 4, true>) : run(k_tail_upper<T, 4, false>);
+        case 3: return run(k_tail_upper<T, 3, false>);
+        case 2: return run(k_tail_upper<T, 2, false>);
+        case 1: return run(k_tail_upper<T, 1, false>);
+        default: return hipErrorInvalidValue;
+        }
     };
-    switch (R) {
-    case 4: return vec ? go(k_tail_upper<T, 4, true>) : go(k_tail_upper<T, 4, false>);
-    case 3: return go(k_tail_upper<T, 3, false>);
-    case 2: return go(k_tail_upper<T, 2, false>);
-    case 1: return go(k_tail_upper<T, 1, false>);
-    default: return hipErrorInvalidValue;
-    }
+    if (tail_items_fit(nl + na + nf + ni + tail_points(r, q))) return go(nl, na, nf, ni, r, q);
+    hipError_t e = go(nl, 0, 0, 0, TailRcv{}, TailSrc{});
+    if (e == hipSuccess) e = go(0, na, nf, 0, TailRcv{}, TailSrc{});
+    return e == hipSuccess ? go(0, 0, 0, ni, r, q) : e;
 }
 
 hipError_t launch_tick(int *p, int d, bool set, hipStream_t s)

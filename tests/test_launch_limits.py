@@ -85,3 +85,18 @@ def _result(program, *args):
 def test_slab_frame_bound(program, grid, R, layer, refused):
     b = 4
     assert (_result(program, "upper", *grid, b, R, 2, layer, 0) == REFUSED) == refused
+
+
+# parts that fit one by one go on, together past 2^31 items or not
+@pytest.mark.parametrize("args, refused", [
+    # layer 4e8 rows, frame 4e8 rows + 3.2e5 cells, imaged frame 1.6e9 cells
+    (("upper", 20000, 20000, 5000, 5, 4, 2, 1, 1), False),
+    # the imaged frame alone: 2.2e9
+    (("upper", 20000, 20000, 7000, 5, 4, 0, 0, 1), True),
+    # frame 2.076e9 cells, front-right edge 1.5e8
+    (("all", 240, 16000, 16000, 100, 4, 2), False),
+    # the frame alone: 2.176e9
+    (("all", 1000, 16000, 16000, 100, 4, 2), True),
+])
+def test_parts_that_fit_by_themselves(program, args, refused):
+    assert (_result(program, *args) == REFUSED) == refused
