@@ -13,6 +13,28 @@ import numpy as np
 DEFAULT = (0, 0, 0)
 
 
+def _format(shot):
+    return {0: "f32", 1: "f16", 2: "bf16"}[shot.wave_format]
+
+
+def _forward_on_output(hip, shot):
+    """The forward steps store the upper taper of their output."""
+    fmt = _format(shot)
+    mode = hip.get_taper_fusion(fmt)
+    if shot.order != 8 or shot.sze < shot.blen or mode not in (-1, 4):
+        return False
+    return mode == 4 or fmt == "f32" or (shot.nze % 2 == 0 and shot.blen >= 8)
+
+
+def _output_shape(tiling, shot):
+    """The shape that a request for `tiling` runs in that form: the one-z waves
+    as asked, FP32's default by itself, all else the two-z waves (even rows) or
+    the 8-row one-z waves, one kernel under many names."""
+    if tiling in ((64, 1, 6), (64, 1, 8)) or (tiling == DEFAULT and _format(shot) == "f32"):
+        return tiling
+    return (128, 1, 4) if shot.nze % 2 == 0 else (64, 1, 8)
+
+
 def tune(hip, shot, V, coefs, g, src, F, R, upb, rcv, img, steps=6, rounds=2, log=None):
     """Returns {class: ((tz, by, ry), avg_ms)} and installs the winners.
 
@@ -40,14 +62,8 @@ def tune(hip, shot, V, coefs, g, src, F, R, upb, rcv, img, steps=6, rounds=2, lo
                 log("tile %s class %d: %.4f ms" % (tiling, cls, avg))
             if cls not in best or avg < best[cls][1]:
                 best[cls] = (tiling, avg)
-    # With the forward upper taper on the output (the FP32 default) every
-    # class-2 shape but the default and the one-z 64x1x6 / 64x1x8 waves
-    # launches the same two-z 128x1x4 kernel: record that shape
-    fmt = {0: "f32", 1: "f16", 2: "bf16"}.get(getattr(shot, "wave_format", 0), "f32")
-    if 2 in best and hip.get_taper_fusion(fmt) in (-1, 4) and fmt == "f32":
-        t2 = tuple(best[2][0])
-        if t2 != DEFAULT and not (t2[0] == 64 and t2[1] == 1 and t2[2] in (6, 8)):
-            best[2] = ((128, 1, 4), best[2][1])
+    if 2 in best and _forward_on_output(hip, shot):
+        best[2] = (_output_shape(tuple(best[2][0]), shot), best[2][1])
     for cls in range(3):
         if cls in best:
             hip.set_tiling(cls, *best[cls][0], 0)
