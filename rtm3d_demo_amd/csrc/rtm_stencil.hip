@@ -361,17 +361,33 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t plane_rsrc(const void *p)
 }
 
 // A plane as a view of its size: a store at lane offset kDropped is out of
-// range of it (less the row offset, which is at least R rows) and discarded, so
-// a plane's step has no branch around a load or a store and the compiler's wait
-// counts are exact (at a join it must assume that neither branch's accesses
-// were issued, and waits for more).  With branches / so, ms: FP16 two-z waves on
-// 592 x 592 x 336, 6 x chunks, plain 0.334 / 0.294, imaging 0.600 / 0.541; FP32
-// one-z 8-row waves, taper3D on the output, 192^3 0.060 / 0.053.
+// range of it (less the row offset, which is at least R rows) and discarded.
 constexpr unsigned kDropped = 0xfffffff0u;
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t plane_bounded(const void *p, size_t bytes)
 {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)(unsigned)bytes,
                                              0x00020000);
+}
+
+// Whether a plane's step (nz z cells per lane) has no branch around its loads
+// and stores: at the join after a branch the compiler must assume that neither
+// side's accesses were issued, and waits for more than it needs.  The price is
+// 3 to 11 registers, a second load of the chunk's last plane (from L2) and
+// stores that are dropped.  16-bit steps and the FP32 batches gain; most other
+// FP32 steps lose more by the registers, the 8-row one tapered on load by
+// spills.  us, with branches / so: FP16 592 x 592 x 336 plain 295 / 268, upper
+// taper on the output 345 / 312; 301 x 277 x 259 plain 56.8 / 52.3, imaging 128 /
+// 121.  FP32 592 x 592 x 336 imaging, 6 rows 883 / 767, 6 rows tapered on load 495
+// / 480; 3 batched shots of 301 x 277 x 259, backward, 8 rows 735 / 684; but 592 x
+// 592 x 336 8 rows tapered on load 503 / 651 (the batch forward 367 / 459), plain
+// 409 / 419 (two-z 400 / 418), upper taper on the output 443 / 463 (two-z 440 /
+// 461), taper3D on the output 421 / 437; imaging, 8 rows, 200 x 180 x 300 57 / 61.
+template <typename T>
+constexpr bool branch_free(int nz, int ry, bool img, int taper, bool batch = false)
+{
+    if (sizeof(T) == 2) return true;
+    if (batch) return img || ry != 8 || taper != 1;
+    return img ? taper == 1 || nz == 2 || ry == 6 : taper == 1 && nz == 1 && ry == 6;
 }
 
 // Loads and stores of one element of type T, widened to / rounded from
@@ -681,7 +697,8 @@ struct WaveGrid {
 // the frame are written by separate kernels, so this form needs no plane-b
 // loads (the pointwise chain only).  TAPER 4 does the same with the upper
 // taper, leaving the planes [b - hold, b) of the output untapered.
-template <typename T, int R, int RY, bool IMG, int TAPER>
+// FREE: branch_free.
+template <typename T, int R, int RY, bool IMG, int TAPER, bool FREE>
 __device__ __forceinline__ void wave_tile(const T *__restrict__ P, T *__restrict__ PP,
                                           const float *__restrict__ V, const Coefs &cf,
                                           const Grid &g, int zt, int yt, int xb, int xe,
@@ -897,9 +914,12 @@ __device__ __forceinline__ void wave_tile(const T *__restrict__ P, T *__restrict
         float yc[2 * R];  // this plane's y-halo values (registers)
 #pragma unroll
         for (int h = 0; h < 2 * R; ++h) yc[h] = yh[cur][h];
-        // past the chunk's last plane too (clamped): no branch, exact waits
-        load_ring(min(x + 1 + R, g.nx - 1), q[(K + 2 * R + 1) % NR]);
-        fetch_halo(min(x + 1, g.nx - 1), cur ^ 1);
+        // FREE: once more at the chunk's last plane
+        if (FREE || x + 1 < xe) {
+            const int xn = x + 1 < xe ? x + 1 : x;
+            load_ring(xn + R, q[(K + 2 * R + 1) % NR]);
+            fetch_halo(xn, cur ^ 1);
+        }
         bool rcvx = false;
         if (IMG) {
             const int dx = x - fz.rx0;
@@ -954,6 +974,7 @@ __device__ __forceinline__ void wave_tile(const T *__restrict__ P, T *__restrict
             // value the step stores (rounded), then taper3D.  z frame (not
             // updated): PP tapered, and with OUT once more as the next step's P
             const bool row = (ymask >> r) & 1u;
+            if (!FREE && !(row && (zcomp || zframe))) continue;
             const bool otap = OUTU && ztap && z < tf.b - tf.hold;
             float o = npp;
             if (OUT) o = tapv(zcomp ? wrnd<T>(npp) : pp, fxc, fyr[r], ztap, fzl, false);
@@ -964,8 +985,9 @@ __device__ __forceinline__ void wave_tile(const T *__restrict__ P, T *__restrict
             if (IMG) {
                 const bool on = row && zcomp && z >= fz.z0 && z < fz.z1 &&
                                 !(rcvx && ((rmask >> r) & 1u) && z == fz.rz);
-                st_buf<float>(rimg, rowb[r] * VS, on ? zoffv : kDropped,
-                              c_img[r] + c_ps[r] * wrnd<T>(npp));
+                if (FREE || on)
+                    st_buf<float>(rimg, rowb[r] * VS, on ? zoffv : kDropped,
+                                  c_img[r] + c_ps[r] * wrnd<T>(npp));
             }
         }
         ++x;
@@ -1027,7 +1049,8 @@ __global__ void __launch_bounds__(64 * WPB, (wave_min_occupancy<T, RY, IMG, TAPE
     const int xc = (int)(w2 / wg.nyt);
     const int xb = R + xc * wg.xchunk;
     const int xe = min(xb + wg.xchunk, g.nx - R);
-    wave_tile<T, R, RY, IMG, TAPER>(P, PP, V, cf, g, zt, yt, xb, xe, fz, tf, tab, tile[wid], flag);
+    wave_tile<T, R, RY, IMG, TAPER, branch_free<T>(1, RY, IMG, TAPER)>(
+        P, PP, V, cf, g, zt, yt, xb, xe, fz, tf, tab, tile[wid], flag);
 }
 
 // ---------------------------------------------------------------------------
@@ -1098,6 +1121,7 @@ __device__ __forceinline__ void wave_tile2(const T *__restrict__ P, T *__restric
     static_assert(NZH * RY <= 64, "one z-halo load per lane");
     constexpr unsigned ES = sizeof(T);
     constexpr unsigned VS = 4u / sizeof(T);
+    constexpr bool FREE = branch_free<T>(2, RY, IMG, TAPER);
     const T *__restrict__ PS = static_cast<const T *>(fz.ps);
     const int lane = threadIdx.x;
     const int y0 = R + yt * RY;
@@ -1271,9 +1295,12 @@ __device__ __forceinline__ void wave_tile2(const T *__restrict__ P, T *__restric
             yc[h][0] = yh[cur][h][0];
             yc[h][1] = yh[cur][h][1];
         }
-        // past the chunk's last plane too (clamped): no branch, exact waits
-        load_ring(min(x + 1 + R, g.nx - 1), q[(K + 2 * R + 1) % NR]);
-        fetch_halo(min(x + 1, g.nx - 1), cur ^ 1);
+        // FREE: once more at the chunk's last plane
+        if (FREE || x + 1 < xe) {
+            const int xn = x + 1 < xe ? x + 1 : x;
+            load_ring(xn + R, q[(K + 2 * R + 1) % NR]);
+            fetch_halo(xn, cur ^ 1);
+        }
         bool rcvx = false;
         if (IMG) {
             const int dx = x - fz.rx0;
@@ -1341,6 +1368,7 @@ __device__ __forceinline__ void wave_tile2(const T *__restrict__ P, T *__restric
             // updated: PP tapered once more as the next step's P); OUTU cells
             // z < b - hold the value stored, then the upper taper
             const bool row = (ymask >> r) & 1u;
+            if (!FREE && !(row && (zcomp || zframe))) continue;
             float o[2];
 #pragma unroll
             for (int a = 0; a < 2; ++a) {
@@ -1366,9 +1394,9 @@ __device__ __forceinline__ void wave_tile2(const T *__restrict__ P, T *__restric
                     const bool on = za >= fz.z0 && za < fz.z1 && !(rc && za == fz.rz);
                     iv[a] = on ? c_img[r][a] + c_ps[r][a] * wrnd<T>(npp[a]) : c_img[r][a];
                 }
-                st_buf2<float>(rimg, rowb[r] * VS,
-                               row && zcomp && z + 1 >= fz.z0 && z < fz.z1 ? zoffv : kDropped,
-                               iv[0], iv[1]);
+                const bool on = row && zcomp && z + 1 >= fz.z0 && z < fz.z1;
+                if (FREE || on)
+                    st_buf2<float>(rimg, rowb[r] * VS, on ? zoffv : kDropped, iv[0], iv[1]);
             }
         }
         ++x;
@@ -1473,8 +1501,8 @@ __global__ void __launch_bounds__(64 * WPB, (wave_min_occupancy<T, RY, IMG, TAPE
         fz.rdy = sh.rdy;
         fz.rny = sh.rny;
     }
-    wave_tile<T, R, RY, IMG, TAPER>(P, PP, sh.V, cf, sh.g, zt, yt, xb, xe, fz, tf, tab,
-                                    tile[wid], flag);
+    wave_tile<T, R, RY, IMG, TAPER, branch_free<T>(1, RY, IMG, TAPER, true)>(
+        P, PP, sh.V, cf, sh.g, zt, yt, xb, xe, fz, tf, tab, tile[wid], flag);
 }
 
 // ---------------------------------------------------------------------------
