@@ -371,7 +371,12 @@ __global__ void __launch_bounds__(kDctThreads)
 // 0.56 ms for the 56,628 bricks of a 528 x 528 x 400 grid, 9 times the time
 // of reading the coefficients).  A brick whose scale is below the threshold is
 // not read.  528 x 528 x 400: 0.562 ms, now 0.139.
-constexpr int kPackBricks = 8;
+//
+// Eight bricks to a block, but two for up to kPackFew bricks, which eight to a
+// block would leave most of the chip without (us, two / eight: 64 bricks 4.3 /
+// 9.5, 288 5.6 / 10.9, 684 10.2 / 11.0, 2880 24.9 / 15.5).
+constexpr long long kPackFew = 768;
+template <int kPackBricks>
 __global__ void __launch_bounds__(kDctThreads)
     k_dct_pack(const float *__restrict__ coef, DctLayout L, unsigned *__restrict__ meta,
                unsigned *__restrict__ entries, unsigned *__restrict__ table)
@@ -586,8 +591,8 @@ hipError_t launch_dct_encode(const T *F, const Grid &g, int z0, int z1, const Dc
     if ((e = hipGetLastError()) != hipSuccess) return e;
     hipLaunchKernelGGL(k_dct_select, dim3(1), dim3(kDctThreads), 0, s, hist, K, meta);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_dct_pack, dim3(L.nblk), dim3(kDctThreads), 0, s, coef, L, meta, entries,
-                       table);
+    hipLaunchKernelGGL(L.nbr <= kPackFew ? k_dct_pack<2> : k_dct_pack<8>, dim3(L.nblk),
+                       dim3(kDctThreads), 0, s, coef, L, meta, entries, table);
     return hipGetLastError();
 }
 

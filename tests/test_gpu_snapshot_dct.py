@@ -55,7 +55,7 @@ def coder(f, b, keep_div, basis=None):
     else:
         dz, dx, dy = basis
     br, padded = _bricks(np.asarray(f, np.float64), b)
-    c = np.einsum("ui,vj,wk,nijk->nuvw", dx, dy, dz, br)
+    c = np.einsum("ui,vj,wk,nijk->nuvw", dx, dy, dz, br, optimize=True)
     c32 = c.astype(np.float32)
     bits = c32.view(np.uint32) & 0x7FFFFFFF
     K = max(1, f.shape[0] * f.shape[1] * (f.shape[2] - 2 * b) // keep_div)
@@ -71,7 +71,7 @@ def coder(f, b, keep_div, basis=None):
     safe = np.where(scale > 0, scale, np.float32(1.0))[:, None, None, None]
     q = (c32 / safe).astype(np.float16).astype(np.float64)
     q = np.where(keep, q * scale[:, None, None, None].astype(np.float64), 0.0)
-    rec = np.einsum("ui,vj,wk,nuvw->nijk", dx, dy, dz, q)
+    rec = np.einsum("ui,vj,wk,nuvw->nijk", dx, dy, dz, q, optimize=True)
     return _unbricks(rec, f.shape, padded, b), int(keep.sum())
 
 
@@ -117,12 +117,16 @@ def test_coder_matches_restatement(gpu, shape, b, keep_div):
 
 @pytest.mark.parametrize("keep_div", [1, 16])
 @pytest.mark.parametrize("shape, b", [((8, 8, 64), 16), ((50, 8, 64), 16), ((24, 24, 64), 16),
-                                      ((17, 31, 75), 5)])
+                                      ((17, 31, 75), 5), ((128, 192, 64), 16),
+                                      ((245, 199, 32), 4), ((200, 248, 32), 4)])
 def test_coder_groups_of_bricks(gpu, shape, b, keep_div):
-    """2, 14, 18 and 36 bricks (they are packed in groups of 8): some all zero,
-    some far below the others (every coefficient under the threshold at 1/16).
-    Same bounds as above, from FP16 quantisation and the threshold's rounding."""
-    f = np.ascontiguousarray(_wavefield((56, 40, 80), 5)[:shape[0], :shape[1], :shape[2]])
+    """2, 14, 18, 36, 768, 775 and 775 bricks (they are packed in groups of 2, or
+    8 past 768): some all zero, some far below the others (every coefficient
+    under the threshold at 1/16).  Same bounds as above, from FP16 quantisation
+    and the threshold's rounding."""
+    f = _wavefield((56, 40, 80), 5)
+    f = np.tile(f, [-(-n // m) for n, m in zip(shape, f.shape)])
+    f = np.ascontiguousarray(f[:shape[0], :shape[1], :shape[2]])
     if shape[0] > 8:
         f[:8, :8] = 0.0
         f[16:, :8] *= np.float32(1e-20)
