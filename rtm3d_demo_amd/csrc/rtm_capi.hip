@@ -175,14 +175,18 @@ const StencilTiling *class_tiling(int cls)
 // One step of kernel class cls.  FP32 steps without a requested tile shape run
 // on full-row blocks where those fit (order 8, rows of 129..512 cells, tapers
 // on the output); everything else on the shapes of launch_stencil.
-// slab_fits holds the line between them and its measurements.
+// slab_plan holds the line between them and its measurements.
 template <typename T>
 hipError_t step_launch(int cls, int radius, const T *P, T *PP, const float *V, const Coefs &cf,
                        const Grid &g, const ImageFuse *fuse, const TaperFuse *taper)
 {
     if constexpr (std::is_same<T, float>::value) {
-        if (!class_tiling(cls) && slab_fits(radius, g, fuse, taper))
-            return launch_slab(P, PP, V, cf, g, fuse, taper, g_state.flag, g_state.stream);
+        if (!class_tiling(cls)) {
+            const slab::SlabGrid plan = slab_plan(radius, g, fuse, taper);
+            if (plan.nyt > 0)
+                return launch_slab(plan, P, PP, V, cf, g, fuse, taper, g_state.flag,
+                                   g_state.stream);
+        }
     }
     return launch_stencil(radius, P, PP, V, cf, g, fuse, taper, g_state.flag, g_state.stream,
                           class_tiling(cls));
@@ -198,7 +202,7 @@ bool image_outu(int wave_format, int radius, const Grid &g, const float *taper, 
         return false;
     const ImageFuse fz{};
     const TaperFuse tf{taper, b, 1, 3, 0};
-    return b > 0 && slab_fits(radius, g, &fz, &tf);
+    return b > 0 && slab_plan(radius, g, &fz, &tf).nyt > 0;
 }
 
 template <typename T>

@@ -54,19 +54,20 @@ int y_tiles(const Grid &g)
 
 }  // namespace
 
-bool slab_fits(int radius, const Grid &g, const ImageFuse *fuse, const TaperFuse *taper)
+slab::SlabGrid slab_plan(int radius, const Grid &g, const ImageFuse *fuse, const TaperFuse *taper)
 {
     using namespace slab;
-    if (radius != 4 || g.nx <= 8 || g.ny <= 8 || g.nz <= 128 || g.nz > 512) return false;
-    if (g.sy != g.nz || g.sx != (long long)g.ny * g.nz) return false;
+    const SlabGrid none{0, 0, 0};
+    if (radius != 4 || g.nx <= 8 || g.ny <= 8 || g.nz <= 128 || g.nz > 512) return none;
+    if (g.sy != g.nz || g.sx != (long long)g.ny * g.nz) return none;
     // 32-bit byte offsets inside a plane
-    if (g.sx * 4 >= (1LL << 31)) return false;
+    if (g.sx * 4 >= (1LL << 31)) return none;
     if (taper && taper->b > 0) {
-        if (taper->b > kSlabTaper || (taper->all != 2 && taper->all != 3)) return false;
+        if (taper->b > kSlabTaper || (taper->all != 2 && taper->all != 3)) return none;
         if (taper->all == 2 && (fuse || taper->b < 4 || 2 * taper->b >= g.nx ||
                                 2 * taper->b >= g.ny || 2 * taper->b >= g.nz))
-            return false;
-        if (taper->all == 3 && (taper->hold < 0 || taper->hold > taper->b)) return false;
+            return none;
+        if (taper->all == 3 && (taper->hold < 0 || taper->hold > taper->b)) return none;
     }
     // A plane step takes 2.2-2.5 us (3.9-4.6 with imaging) whatever the row
     // length; the waves of rtm_stencil.hip take 2.6-3.4 us (4.6-6.7) per
@@ -80,15 +81,18 @@ bool slab_fits(int radius, const Grid &g, const ImageFuse *fuse, const TaperFuse
     // 400 x 260 x 161 125 / 120 (1.326).
     const double fill = std::sqrt((double)((g.nz + 127) / 128 * 128) / g.nz);
     const double line = (!fuse ? 1.335e-6 : (g.nz & 1) ? 1.32e-6 : 1.4e-6) * fill;
-    return (double)choose_march(y_tiles(g), g.nx - 8).steps <
-           line * (double)g.nx * g.ny * g.nz;
+    const int nyt = y_tiles(g);
+    const March m = choose_march(nyt, g.nx - 8);
+    if ((double)m.steps >= line * (double)g.nx * g.ny * g.nz) return none;
+    return SlabGrid{nyt, (g.nx - 8 + m.chunk - 1) / m.chunk, m.chunk};
 }
 
-hipError_t launch_slab(const float *P, float *PP, const float *V, const Coefs &cf, const Grid &g,
-                       const ImageFuse *fuse, const TaperFuse *taper, int *flag, hipStream_t s)
+hipError_t launch_slab(const slab::SlabGrid &plan, const float *P, float *PP, const float *V,
+                       const Coefs &cf, const Grid &g, const ImageFuse *fuse,
+                       const TaperFuse *taper, int *flag, hipStream_t s)
 {
     using namespace slab;
-    if (!slab_fits(4, g, fuse, taper)) return hipErrorInvalidValue;
+    if (plan.nyt <= 0) return hipErrorInvalidValue;
     ImageFuse fz{};
     TaperFuse tf{};
     if (fuse) {
@@ -101,12 +105,8 @@ hipError_t launch_slab(const float *P, float *PP, const float *V, const Coefs &c
     const Form form = fuse ? (tap ? kImageOutUpper : kImage)
                            : (!tap ? kPlain : (tf.all == 2 ? kOut : kOutUpper));
     const int nzw = (g.nz + 127) / 128;
-    SlabGrid sg;
-    sg.nyt = y_tiles(g);
-    sg.xchunk = choose_march(sg.nyt, g.nx - 8).chunk;
-    sg.nxc = (g.nx - 8 + sg.xchunk - 1) / sg.xchunk;
-    return (g.nz & 1) ? launch_odd(nzw, form, P, PP, V, cf, g, sg, fz, tf, flag, s)
-                      : launch_even(nzw, form, P, PP, V, cf, g, sg, fz, tf, flag, s);
+    return (g.nz & 1) ? launch_odd(nzw, form, P, PP, V, cf, g, plan, fz, tf, flag, s)
+                      : launch_even(nzw, form, P, PP, V, cf, g, plan, fz, tf, flag, s);
 }
 
 }  // namespace rtmhip

@@ -7,6 +7,7 @@ namespace slab {
 
 constexpr int kSlabTaper = 1024;  // longest taper table held in LDS
 
+// y tiles, x chunks and their length; nyt 0: the kernel does not serve the step
 struct SlabGrid {
     int nyt, nxc, xchunk;
 };
@@ -30,9 +31,10 @@ constexpr int y_waves(int nzw) { return 12 / nzw; }
 
 // The step (radius 4, FP32) that the full-row kernel serves: no taper, taper3D
 // or the upper taper on the output, imaging without a taper or with the upper
-// taper on the output.
-bool slab_fits(int radius, const Grid &g, const ImageFuse *fuse, const TaperFuse *taper);
-hipError_t launch_slab(const float *P, float *PP, const float *V, const Coefs &cf, const Grid &g,
-                       const ImageFuse *fuse, const TaperFuse *taper, int *flag, hipStream_t s);
+// taper on the output.  launch_slab takes the plan of the same step.
+slab::SlabGrid slab_plan(int radius, const Grid &g, const ImageFuse *fuse, const TaperFuse *taper);
+hipError_t launch_slab(const slab::SlabGrid &plan, const float *P, float *PP, const float *V,
+                       const Coefs &cf, const Grid &g, const ImageFuse *fuse,
+                       const TaperFuse *taper, int *flag, hipStream_t s);
 
 }  // namespace rtmhip

@@ -1,8 +1,10 @@
-"""Which counts the launches after a step take: the launchers number cells in 32
-bits and must refuse what would overflow, and only that.  A small program
-calls them without a device (so nothing is ever launched) and prints each
-result: hipErrorInvalidValue where the launcher refused, another error where it
-went on to launch.
+"""What the launchers' rules take, asked without a device (so nothing is ever
+launched) by a small program that calls them and prints the answer.
+
+* Counts of the launches after a step: cells are numbered in 32 bits, and what
+  would overflow must be refused, and only that (hipErrorInvalidValue where the
+  launcher refused, another error where it went on to launch).
+* Which steps the FP32 full-row kernel serves (for 256 compute units).
 """
 import os
 import subprocess
@@ -15,6 +17,7 @@ REFUSED = 1  # hipErrorInvalidValue
 
 PROGRAM = r"""
 #include "rtm_internal.hpp"
+#include "rtm_slab_launch.hpp"
 #include "rtm_tail.hpp"
 #include <cstdio>
 #include <cstdlib>
@@ -40,6 +43,12 @@ int main(int argc, char **argv)
     const int b = arg(5), R = arg(6), taps = arg(7);
     float *p = reinterpret_cast<float *>(4096);
     const TailSource src{p, (long long)g.nx / 2 * g.sx + g.ny / 2 * g.sy + g.nz / 2, 0};
+    if (!strcmp(argv[1], "full-row")) {  // R: the stencil radius, taps: the taper's form
+        const ImageFuse fz{};
+        const TaperFuse tf{p, b, 1, taps, 0};
+        printf("%d\n", slab_plan(R, g, arg(8) ? &fz : nullptr, taps ? &tf : nullptr).nyt);
+        return 0;
+    }
     hipError_t e;
     if (!strcmp(argv[1], "all")) {
         e = launch_tail_all<float>(p, p, g, b, R, taps, nullptr, &src, nullptr);
@@ -100,3 +109,25 @@ def test_slab_frame_bound(program, grid, R, layer, refused):
 ])
 def test_parts_that_fit_by_themselves(program, args, refused):
     assert (_result(program, *args) == REFUSED) == refused
+
+
+# taper: 0 none, 1 the upper taper on load, 2 taper3D and 3 the upper taper on
+# the output
+@pytest.mark.parametrize("grid, b, radius, taper, image, served", [
+    ((592, 592, 336), 40, 4, 0, 0, True),
+    ((592, 592, 336), 40, 4, 2, 0, True),
+    ((592, 592, 336), 40, 4, 3, 0, True),
+    ((592, 592, 336), 40, 4, 0, 1, True),
+    ((592, 592, 336), 40, 4, 3, 1, True),
+    ((592, 592, 336), 40, 4, 1, 0, False),
+    ((592, 592, 336), 40, 4, 2, 1, False),   # no imaging with taper3D
+    ((592, 592, 336), 40, 3, 0, 0, False),
+    ((592, 592, 128), 40, 4, 0, 0, False),   # rows of 129 to 512 cells
+    ((592, 592, 129), 40, 4, 0, 0, False),   # a second wave of one cell
+    ((592, 592, 513), 40, 4, 0, 0, False),
+    ((301, 277, 259), 21, 4, 0, 1, True),
+    ((192, 192, 192), 24, 4, 0, 0, False),
+    ((40, 44, 90), 12, 4, 0, 0, False),
+])
+def test_full_row_steps(program, grid, b, radius, taper, image, served):
+    assert (_result(program, "full-row", *grid, b, radius, taper, image) > 0) == served
