@@ -177,10 +177,9 @@ hipError_t launch_taper_all2(T *P, T *Q, const float *taper, const Grid &g, int 
                              hipStream_t s);
 // Upper taper (applied `taps` times) of the slab cells the stencil never
 // updates (z < R or the x / y frame of width R), in place.
-// With hold > 0 the planes z in [b - hold, b) get one application fewer.
 template <typename T>
 hipError_t launch_taper_frame(T *P, const float *taper, const Grid &g, int b, int R, int taps,
-                              hipStream_t s, int hold = 0);
+                              hipStream_t s);
 // taper3D's counterpart of launch_taper_frame (fused every-border taper):
 // the cells within R of any grid face, `taps` times in place, the front-right
 // edge's cells from the cell (b, y, z) as taper3D reads it.  Runs before the

@@ -407,13 +407,13 @@ inline FrameDivs frame_divs(int R, int lz, int ny)
 template <typename T>
 __global__ void __launch_bounds__(kThreads)
     k_taper_frame(T *__restrict__ P, const float *__restrict__ t, Grid g, int b, int R, int taps,
-                  FrameDivs dv, int zhold)
+                  FrameDivs dv)
 {
     const int i = (int)(blockIdx.x * kThreads + threadIdx.x);  // count < 2^31 (launcher)
     int x, y, z;
     if (!frame_cell_fd(g, b, R, i, dv, x, y, z)) return;
     const long long o = goff(g, x, y, z);
-    P[o] = wst<T>(frame_taper<T>(wld(P[o]), t, g, b, x, y, z, z >= zhold ? taps - 1 : taps));
+    P[o] = wst<T>(frame_taper<T>(wld(P[o]), t, g, b, x, y, z, taps));
 }
 
 // taper3D at one cell, `taps` times (rounded to T between applications):
@@ -1413,16 +1413,15 @@ hipError_t launch_taper_all2(T *P, T *Q, const float *taper, const Grid &g, int 
 
 template <typename T>
 hipError_t launch_taper_frame(T *P, const float *taper, const Grid &g, int b, int R, int taps,
-                              hipStream_t s, int hold)
+                              hipStream_t s)
 {
     if (b <= 0 || taps <= 0) return hipSuccess;
-    if (hold < 0 || hold > b) return hipErrorInvalidValue;
     const long long lz = b - R;
     const long long n = (long long)g.nx * g.ny * R + (long long)2 * R * g.ny * lz +
                         (long long)(g.nx - 2 * R) * 2 * R * lz;
     if (n + kThreads >= (1LL << 31)) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_taper_frame<T>, dim3(nblocks(n)), dim3(kThreads), 0, s, P, taper, g, b, R,
-                       taps, frame_divs(R, b - R, g.ny), b - hold);
+                       taps, frame_divs(R, b - R, g.ny));
     return hipGetLastError();
 }
 
@@ -1807,7 +1806,7 @@ hipError_t launch_tick(int *p, int d, bool set, hipStream_t s)
     template hipError_t launch_taper_upper2<T>(T *, T *, const float *, const Grid &, int,      \
                                                hipStream_t);                                    \
     template hipError_t launch_taper_frame<T>(T *, const float *, const Grid &, int, int, int,  \
-                                              hipStream_t, int);                                \
+                                              hipStream_t);                                     \
     template hipError_t launch_taper_frame_all<T>(T *, const float *, const Grid &, int, int,   \
                                                   int, hipStream_t);                            \
     template hipError_t launch_source<T>(T *, long long, const float *, int, float, hipStream_t); \
