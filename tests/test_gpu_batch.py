@@ -22,6 +22,9 @@ SHOTS = [
     ((34, 38, 70), (15, 17, B - 2), (0, 0, 0, 2, 2, 5, 7)),       # source in the UPB layer
     ((46, 40, 130), (2, 19, B - 6), (4, 3, 2, 0, 5, 1, 3)),       # source in the frame
 ]
+# one grid that the FP32 full-row step serves (test_launch_limits.py checks it)
+# and two that it does not
+MIXED = [SHOTS[0], ((104, 500, 384), (52, 250, B + 2), (1, 2, 3, 3, 4, 7, 6)), SHOTS[1]]
 
 
 def _wave(rng, shape, fmt):
@@ -32,7 +35,7 @@ def _wave(rng, shape, fmt):
 class Shots:
     """Host inputs of the batch and device copies for one run."""
 
-    def __init__(self, gpu, fmt, seed=5):
+    def __init__(self, gpu, fmt, seed=5, shots=SHOTS):
         self.gpu, self.fmt = gpu, fmt
         self.wd = gpu.WAVE_FORMATS[fmt][1]
         rng = np.random.default_rng(seed)
@@ -43,7 +46,7 @@ class Shots:
             self.coefs[d * 9:(d + 1) * 9] = (c8 / (h * h)).astype(np.float32)
         self.g = np.exp(-(np.sqrt(-np.log(0.9)) / B * np.arange(B)) ** 2).astype(np.float32)
         self.host = []
-        for grid, src, rg in SHOTS:
+        for grid, src, rg in shots:
             nx, ny, nz = grid
             h = dict(grid=grid, src=src, rg=rg,
                      V=rng.uniform(0.0, 0.15, grid).astype(np.float32),
@@ -150,6 +153,22 @@ def test_batch_matches_single_shots(gpu, fmt, modes, graph_steps):
     sh.free(ref)
     mem = sh.device()
     got = _run_batch(gpu, sh, mem, FWD, BWD, modes, graph_steps)
+    sh.free(mem)
+    assert np.abs(want[-1][0][5]).max() > 0
+    _compare(want, got)
+
+
+@pytest.mark.parametrize("shots", [MIXED, MIXED[1:2] * 2], ids=["some-full-row", "all-full-row"])
+@pytest.mark.parametrize("fmt", ["f32", "f16"])
+def test_batch_of_full_row_shots(gpu, fmt, shots):
+    """Grids on either side of the full-row kernel's line in one batch, and two
+    beyond it (whose receiver steps store the upper taper on their output)."""
+    sh = Shots(gpu, fmt, shots=shots)
+    ref = sh.device()
+    want = _run_single(gpu, sh, ref, FWD, BWD)
+    sh.free(ref)
+    mem = sh.device()
+    got = _run_batch(gpu, sh, mem, FWD, BWD, (0, 0, 0), 4)
     sh.free(mem)
     assert np.abs(want[-1][0][5]).max() > 0
     _compare(want, got)

@@ -9,7 +9,7 @@ for bit.
 import numpy as np
 import pytest
 
-import test_gpu_slab as windows
+import windows
 
 pytestmark = pytest.mark.gpu
 
@@ -25,31 +25,22 @@ CASES = [
 ]
 
 
-@pytest.fixture
-def window(monkeypatch):
-    setup = windows._setup
-
-    def use(cell, geo):
-        def patched(gpu, po, shape, blen, seed):
-            c = setup(gpu, po, shape, blen, seed)
-            rng = np.random.default_rng(seed + 10)
-            rcv = rng.standard_normal((geo[5], geo[6], c["nt"])).astype(np.float32)
-            return dict(c, cell=cell, geo=geo, rcv=rcv)
-        monkeypatch.setattr(windows, "_setup", patched)
-    return use
+def _window(oracle, shape, blen, cell, geo, seed):
+    c = windows.setup(oracle, shape, blen, seed, cell, geo)
+    rng = np.random.default_rng(seed + 10)
+    c["rcv"] = rng.standard_normal((geo[5], geo[6], c["nt"])).astype(np.float32)
+    return c
 
 
 @pytest.mark.parametrize("shape,blen,cell,geo", CASES)
-def test_modeling(gpu, oracle, window, shape, blen, cell, geo):
-    window(cell, geo)
-    windows.test_modeling_window(gpu, oracle, shape, blen)
+def test_modeling(gpu, oracle, shape, blen, cell, geo):
+    windows.modeling(gpu, oracle, _window(oracle, shape, blen, cell, geo, 1))
 
 
 @pytest.mark.parametrize("hbc", [1, 0])
 @pytest.mark.parametrize("shape,blen,cell,geo", CASES)
-def test_migration(gpu, oracle, window, shape, blen, cell, geo, hbc):
-    window(cell, geo)
-    windows.test_migration_window(gpu, oracle, shape, blen, hbc)
+def test_migration(gpu, oracle, shape, blen, cell, geo, hbc):
+    windows.migration(gpu, oracle, _window(oracle, shape, blen, cell, geo, 2), hbc)
 
 
 # borders down to the stencil's radius: the layer and the z frame share cells
@@ -59,10 +50,11 @@ NARROW = [((44, 40, 48), 4), ((43, 41, 47), 5), ((44, 40, 48), 6), ((33, 36, 131
 
 
 @pytest.mark.parametrize("shape,blen", NARROW)
-def test_narrow_borders(gpu, oracle, window, shape, blen):
+def test_narrow_borders(gpu, oracle, shape, blen):
     nx, ny, nz = shape
-    window((nx // 2, ny // 2, blen), (0, 0, 0, 3, 2, (nx - 2 * blen) // 3, (ny - 2 * blen) // 2))
-    windows.test_migration_window(gpu, oracle, shape, blen, 1)
+    cell = (nx // 2, ny // 2, blen)
+    geo = (0, 0, 0, 3, 2, (nx - 2 * blen) // 3, (ny - 2 * blen) // 2)
+    windows.migration(gpu, oracle, _window(oracle, shape, blen, cell, geo, 2), 1)
 
 
 @pytest.mark.parametrize("fmt,mode", [("f32", -1), ("f16", 4)])

@@ -11,6 +11,8 @@ import subprocess
 
 import pytest
 
+import test_gpu_batch
+import test_gpu_slab
 from rtm3d_demo_amd import build
 
 REFUSED = 1  # hipErrorInvalidValue
@@ -131,3 +133,14 @@ def test_parts_that_fit_by_themselves(program, args, refused):
 ])
 def test_full_row_steps(program, grid, b, radius, taper, image, served):
     assert (_result(program, "full-row", *grid, b, radius, taper, image) > 0) == served
+
+
+@pytest.mark.parametrize("taper, image", [(0, 0), (2, 0), (3, 0), (0, 1), (3, 1)])
+def test_windows_of_the_full_row_kernel_run_it(program, taper, image):
+    """The grids of test_gpu_slab.py, and of the mixed batch, lie where those
+    tests say."""
+    for grid, b in test_gpu_slab.SHAPES:
+        assert _result(program, "full-row", *grid, b, 4, taper, image) > 0, grid
+    served = [_result(program, "full-row", *shot[0], test_gpu_batch.B, 4, taper, image) > 0
+              for shot in test_gpu_batch.MIXED]
+    assert served == [False, True, False]
