@@ -2619,14 +2619,21 @@ hipError_t launch_radius(const T *P, T *PP, const float *V, const Coefs &cf, con
         // waves (64 x 1 x 8 waves where pairs do not fit or fill), the tapered
         // step on 64 x 1 x 8 waves (salt grid: 0.412 and 0.463 ms against
         // 0.447 and 0.498 for full rows 2 x 6).  The imaging step keeps the
-        // full rows below on large grids (salt grid 0.699 ms against 0.79 or
-        // more on every wave shape) and runs 64 x 1 x 8 waves on short rows
-        // and on grids that its blocks of 12 rows would not fill (us, waves
-        // against rows: 192^3 41 / 63, 256^3 105 / 122, 500 x 500 x 130 245 /
-        // 334, 200 x 180 x 300 72 / 78, 301 x 277 x 259 164 / 178; 336^3
-        // 260 / 249).
-        const bool small = g.nz <= 256 || (long long)(g.ny / 12) * (g.nx / 16) < 500;
-        if (!t && fuse && small && (!taper || taper->b <= 8192))
+        // full rows below where 4 x 4 blocks of one, two or four waves a row
+        // cover it (us, rows against 64 x 1 x 8 waves, untapered and tapered on
+        // load: 64^3 9.1 / 12.4, 12.8 / 16.5; 250 x 240 x 70 29 / 33, 36 / 41; 700 x 500 x
+        // 90 186 / 207, 199 / 223; 592 x 592 x 128 281 / 304, 286 / 303; 240 x 230 x 193
+        // 60 / 63, 66 / 70) and on large grids (2 x 6: salt grid 699 / 790).  It runs
+        // the waves on rows of three (420 x 330 x 129 127 / 123, 148 / 131; 400 x 300 x
+        // 140 118 / 110, 133 / 122; 350 x 350 x 160 127 / 115, 139 / 125; 192^3 37 / 37, 43
+        // / 42) unless the grid is small (80 x 80 x 140 12.5 / 13.2, 14.8 / 16.7; 120 x
+        // 110 x 170 18.1 / 18.6, 21.4 / 22.1) and where the 2 x 6 blocks would leave the
+        // chip idle (100 x 120 x 300 30 / 24, 31 / 27; 200 x 180 x 300 68 / 57, 69 / 62;
+        // but 336^3 239 / 240).
+        const bool waves = g.nz > 256 ? (long long)(g.ny / 12) * (g.nx / 16) < 500
+                                      : (g.nz + 63) / 64 == 3 &&
+                                            (long long)g.nx * g.ny * g.nz > 4000000;
+        if (!t && fuse && waves && (!taper || taper->b <= 8192))
             return launch_wave<T, R, 8, 4>(P, PP, V, cf, g, fuse, taper, flag, s, xchunk);
         if (!t && !fuse && (!taper || taper->b <= 8192)) {
             const bool tapered = taper && taper->b > 0;
