@@ -363,10 +363,16 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t plane_rsrc(const void *p)
 // A plane as a view of its size: a store at lane offset kDropped is out of
 // range of it (less the row offset, which is at least R rows) and discarded.
 constexpr unsigned kDropped = 0xfffffff0u;
+constexpr unsigned plane_records(size_t bytes)
+{
+    return bytes < kDropped ? (unsigned)bytes : kDropped;
+}
+// (a plane of exactly 4 GB has no cell that the step stores past kDropped)
+static_assert(plane_records((size_t)1 << 32) == kDropped && plane_records(4096) == 4096);
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t plane_bounded(const void *p, size_t bytes)
 {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)(unsigned)bytes,
-                                             0x00020000);
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0,
+                                             (int)plane_records(bytes), 0x00020000);
 }
 
 // Whether a plane's step (nz z cells per lane) has no branch around its loads
