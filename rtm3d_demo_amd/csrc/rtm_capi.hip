@@ -178,11 +178,12 @@ const StencilTiling *class_tiling(int cls)
 // slab_plan holds the line between them and its measurements.
 template <typename T>
 hipError_t step_launch(int cls, int radius, const T *P, T *PP, const float *V, const Coefs &cf,
-                       const Grid &g, const ImageFuse *fuse, const TaperFuse *taper)
+                       const Grid &g, const ImageFuse *fuse, const TaperFuse *taper,
+                       int arrays = 3)
 {
     if constexpr (std::is_same<T, float>::value) {
         if (!class_tiling(cls)) {
-            const slab::SlabGrid plan = slab_plan(radius, g, fuse, taper);
+            const slab::SlabGrid plan = slab_plan(radius, g, fuse, taper, arrays);
             if (plan.nyt > 0)
                 return launch_slab(plan, P, PP, V, cf, g, fuse, taper, g_state.flag,
                                    g_state.stream);
@@ -191,6 +192,9 @@ hipError_t step_launch(int cls, int radius, const T *P, T *PP, const float *V, c
     return launch_stencil(radius, P, PP, V, cf, g, fuse, taper, g_state.flag, g_state.stream,
                           class_tiling(cls));
 }
+
+// The grid's arrays in a backward loop: both fields' pairs, V and the image.
+constexpr int kBackArrays = 6;
 
 // The receiver step with imaging takes the upper taper on its output (and the
 // loops order their in-place tapers accordingly) where the full-row kernel
@@ -207,11 +211,13 @@ bool image_outu(int wave_format, int radius, const Grid &g, const float *taper, 
 
 template <typename T>
 hipError_t stencil(int radius, const T *P, T *PP, const float *V, const Coefs &cf, const Grid &g,
-                   const ImageFuse *fuse, const TaperFuse *taper = nullptr)
+                   const ImageFuse *fuse, const TaperFuse *taper = nullptr, int arrays = 3)
 {
     // kernel class: 0 plain step, 1 fused receiver step, 2 tapered HBC step
     const int cls = fuse ? 1 : (taper ? 2 : 0);
-    return timed(cls, [&] { return step_launch(cls, radius, P, PP, V, cf, g, fuse, taper); });
+    return timed(cls, [&] {
+        return step_launch(cls, radius, P, PP, V, cf, g, fuse, taper, arrays);
+    });
 }
 
 
@@ -616,6 +622,7 @@ int rtmhip_freq_steps(const rtmhip_shot *shot, const float *V2DT2, const float *
     // the call's last step.
     const bool out = c.radius == 4 && b > 0 && g_state.taper_all_mode[RTMHIP_WAVE_F32] == 2 &&
                      off_borders(shot, c);
+    const int arrays = kBackArrays + 4 * std::min(nwstep, nw);  // the accumulators
     for (int k = 0; k < nsteps; ++k) {
         const int rt = it_hi - k, st = nt - 1 - rt, lt = rt % shot->ntstep;
         if (out) {
@@ -623,12 +630,14 @@ int rtmhip_freq_steps(const rtmhip_shot *shot, const float *V2DT2, const float *
             float **fields[2][2] = {{Ps, PPs}, {Pr, PPr}};
             for (auto &f : fields)
                 HIPCHK(stencil(c.radius, (const float *)*f[0], *f[1], V2DT2, c.cf, c.g, nullptr,
-                               &tf),
+                               &tf, arrays),
                        "stencil");
         } else {
-            HIPCHK(stencil(c.radius, (const float *)*Ps, *PPs, V2DT2, c.cf, c.g, nullptr),
+            HIPCHK(stencil(c.radius, (const float *)*Ps, *PPs, V2DT2, c.cf, c.g, nullptr, nullptr,
+                           arrays),
                    "source stencil");
-            HIPCHK(stencil(c.radius, (const float *)*Pr, *PPr, V2DT2, c.cf, c.g, nullptr),
+            HIPCHK(stencil(c.radius, (const float *)*Pr, *PPr, V2DT2, c.cf, c.g, nullptr, nullptr,
+                           arrays),
                    "receiver stencil");
             HIPCHK(launch_taper_all2(*Ps, *PPs, taper, c.g, b, s), "taper");
             HIPCHK(launch_taper_all2(*Pr, *PPr, taper, c.g, b, s), "taper");
@@ -900,7 +909,8 @@ int backward_loop(const rtmhip_shot *shot, const ShotCtx &c, int hbc, const floa
             S = *Ps;   // snap0 (entry state: Ps = snap0, PPs = snap1)
         } else {
             if (hbc) restore = upb + (size_t)ul * layer;
-            HIPCHK(stencil(c.radius, *Ps, *PPs, V2DT2, c.cf, c.g, nullptr), "stencil");
+            HIPCHK(stencil(c.radius, *Ps, *PPs, V2DT2, c.cf, c.g, nullptr, nullptr, kBackArrays),
+                   "stencil");
             if (hbc && !fused)
                 HIPCHK(launch_upb(*PPs, const_cast<T *>(upb), c.g, b, c.hf, ul, true, s),
                        "upb restore");
@@ -943,7 +953,8 @@ int backward_loop(const rtmhip_shot *shot, const ShotCtx &c, int hbc, const floa
                                         S, s),
                    "frame, history, receivers and image");
         } else {
-            HIPCHK(stencil(c.radius, *Pr, *PPr, V2DT2, c.cf, c.g, nullptr), "stencil");
+            HIPCHK(stencil(c.radius, *Pr, *PPr, V2DT2, c.cf, c.g, nullptr, nullptr, kBackArrays),
+                   "stencil");
             HIPCHK(launch_receivers(*PPr, const_cast<float *>(rcv_chunk), c.g, c.rx0, c.ry0,
                                     c.rz, shot->rcv.dist_x, shot->rcv.dist_y, shot->rcv.count_x,
                                     shot->rcv.count_y, shot->ntstep, lt, true, s),
@@ -967,6 +978,10 @@ inline int snap_slot(int it, int nt, int k)
     return d % k == 0 ? d / k : -1;
 }
 
+// The arrays of the grid's size that a snapshot loop touches per step: P, PP and V,
+// and about three more at every k-th (the coder's or the image and snapshot).
+inline int snap_arrays(int k) { return 3 + 3 / k; }
+
 inline size_t snap_cells(const rtmhip_shot *shot)
 {
     return (size_t)shot->nxe * shot->nye * (size_t)(shot->nze - 2 * shot->blen);
@@ -987,6 +1002,9 @@ int snap_forward_run(const rtmhip_shot *shot, const ShotCtx &c, const float *V2D
     // the upper taper on the output as in forward_loop (no history planes
     // held: the snapshots cover z >= blen only)
     const bool outu = upper_on_output(shot->wave_format, c.g) && c.radius == 4 && shot->sze >= b;
+    const auto step = [&](const T *p, T *pp, const TaperFuse *taps) {
+        return stencil(c.radius, p, pp, V2DT2, c.cf, c.g, nullptr, taps, snap_arrays(k));
+    };
     for (int it = it0; it < it0 + nsteps; ++it) {
         T *t = *P;
         *P = *PP;
@@ -995,20 +1013,20 @@ int snap_forward_run(const rtmhip_shot *shot, const ShotCtx &c, const float *V2D
         if (outu && it < it0 + nsteps - 1) {
             if (it == it0) HIPCHK(launch_taper(*P, taper, c.g, b, true, s), "taper");
             const TaperFuse tf{taper, b, 1, 3, 0};
-            HIPCHK(stencil(c.radius, *P, *PP, V2DT2, c.cf, c.g, nullptr, &tf), "stencil");
+            HIPCHK(step(*P, *PP, &tf), "stencil");
             w.taps = 2;
         } else if (outu) {
             if (it == it0)
                 HIPCHK(launch_taper_upper2(*P, *PP, taper, c.g, b, s), "taper");
             else
                 HIPCHK(launch_taper(*PP, taper, c.g, b, true, s), "taper");
-            HIPCHK(stencil(c.radius, *P, *PP, V2DT2, c.cf, c.g, nullptr), "stencil");
+            HIPCHK(step(*P, *PP, nullptr), "stencil");
         } else if (sep) {
             HIPCHK(launch_taper_upper2(*P, *PP, taper, c.g, b, s), "taper");
-            HIPCHK(stencil(c.radius, *P, *PP, V2DT2, c.cf, c.g, nullptr), "stencil");
+            HIPCHK(step(*P, *PP, nullptr), "stencil");
         } else {
             const TaperFuse tf{taper, b, it == it0 ? 1 : 2};
-            HIPCHK(stencil(c.radius, *P, *PP, V2DT2, c.cf, c.g, nullptr, &tf), "stencil");
+            HIPCHK(step(*P, *PP, &tf), "stencil");
             HIPCHK(launch_taper_frame(*PP, taper, c.g, b, c.radius, tf.pp_taps, s),
                    "frame taper");
         }
@@ -1055,25 +1073,28 @@ int snap_backward_run(const rtmhip_shot *shot, const ShotCtx &c, const float *V2
     // the receiver-only steps take the upper taper on the output like the
     // forward loops (the receivers and the imaged range lie at z >= blen)
     const bool outu = upper_on_output(shot->wave_format, c.g) && c.radius == 4 && c.rz >= b;
+    const auto step = [&](const T *p, T *pp, const TaperFuse *taps) {
+        return stencil(c.radius, p, pp, V2DT2, c.cf, c.g, nullptr, taps, snap_arrays(k));
+    };
     for (int it = it_hi; it > it_hi - nsteps; --it) {
         TailLayer<T> w{0, 0, nullptr, nullptr, nullptr};  // the frame after the step
         if (outu && it > it_hi - nsteps + 1) {
             if (it == it_hi) HIPCHK(launch_taper(*Pr, taper, c.g, b, true, s), "taper");
             const TaperFuse tf{taper, b, 1, 3, 0};
-            HIPCHK(stencil(c.radius, *Pr, *PPr, V2DT2, c.cf, c.g, nullptr, &tf), "stencil");
+            HIPCHK(step(*Pr, *PPr, &tf), "stencil");
             w.taps = 2;
         } else if (outu) {
             if (it == it_hi)
                 HIPCHK(launch_taper_upper2(*Pr, *PPr, taper, c.g, b, s), "taper");
             else
                 HIPCHK(launch_taper(*PPr, taper, c.g, b, true, s), "taper");
-            HIPCHK(stencil(c.radius, *Pr, *PPr, V2DT2, c.cf, c.g, nullptr), "stencil");
+            HIPCHK(step(*Pr, *PPr, nullptr), "stencil");
         } else if (sep) {
             HIPCHK(launch_taper_upper2(*Pr, *PPr, taper, c.g, b, s), "taper");
-            HIPCHK(stencil(c.radius, *Pr, *PPr, V2DT2, c.cf, c.g, nullptr), "stencil");
+            HIPCHK(step(*Pr, *PPr, nullptr), "stencil");
         } else {
             const TaperFuse tf{taper, b, it == it_hi ? 1 : 2};
-            HIPCHK(stencil(c.radius, *Pr, *PPr, V2DT2, c.cf, c.g, nullptr, &tf), "stencil");
+            HIPCHK(step(*Pr, *PPr, &tf), "stencil");
             HIPCHK(launch_taper_frame(*PPr, taper, c.g, b, c.radius, tf.pp_taps, s),
                    "frame taper");
         }
@@ -1627,7 +1648,7 @@ int batch_fwd_step(rtmhip_batch *b, int taps, const int *itp, int itoff, int for
             const BatchShot &h = b->hs[0][i];
             HIPCHK(step_launch<T>(form == 1 ? cls : 0, b->radius, (const T *)h.fs[b->cs],
                                   (T *)h.fs[b->cs ^ 1], h.V, b->cf, h.g, nullptr,
-                                  form == 1 ? &to : nullptr),
+                                  form == 1 ? &to : nullptr, 3 * b->n),
                    "stencil");
         }
         HIPCHK(launch_tail_fwd<T>(b->ds[0], b->n, b->fwd_blocks, b->cs, b->taper, b->blen,
@@ -1645,7 +1666,7 @@ int batch_fwd_step(rtmhip_batch *b, int taps, const int *itp, int itoff, int for
         for (int i = 0; i < b->n; ++i) {
             const BatchShot &h = b->hs[0][i];
             HIPCHK(step_launch<T>(cls, b->radius, (const T *)h.fs[b->cs], (T *)h.fs[b->cs ^ 1],
-                                  h.V, b->cf, h.g, nullptr, &tf),
+                                  h.V, b->cf, h.g, nullptr, &tf, 3 * b->n),
                    "stencil");
         }
     }
@@ -1698,7 +1719,7 @@ int batch_bwd_step(rtmhip_batch *b, int taps, const int *itp, int itoff, int for
         for (int i = 0; i < b->n; ++i) {
             const BatchShot &h = b->hs[0][i];
             HIPCHK(step_launch<T>(0, b->radius, (const T *)h.fs[b->cs], (T *)h.fs[b->cs ^ 1], h.V,
-                                  b->cf, h.g, nullptr, nullptr),
+                                  b->cf, h.g, nullptr, nullptr, kBackArrays * b->n),
                    "stencil");
         }
     }

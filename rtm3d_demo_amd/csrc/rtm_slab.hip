@@ -3,7 +3,6 @@
 
 #include <algorithm>
 #include <atomic>
-#include <cmath>
 
 namespace rtmhip {
 namespace {
@@ -54,7 +53,8 @@ int y_tiles(const Grid &g)
 
 }  // namespace
 
-slab::SlabGrid slab_plan(int radius, const Grid &g, const ImageFuse *fuse, const TaperFuse *taper)
+slab::SlabGrid slab_plan(int radius, const Grid &g, const ImageFuse *fuse, const TaperFuse *taper,
+                         int arrays)
 {
     using namespace slab;
     const SlabGrid none{0, 0, 0};
@@ -69,21 +69,41 @@ slab::SlabGrid slab_plan(int radius, const Grid &g, const ImageFuse *fuse, const
             return none;
         if (taper->all == 3 && (taper->hold < 0 || taper->hold > taper->b)) return none;
     }
-    // A plane step takes 2.2-2.5 us (3.9-4.6 with imaging) whatever the row
-    // length; the waves of rtm_stencil.hip take 2.6-3.4 us (4.6-6.7) per
-    // million cells, more where rows fill their tiles badly -- where part of
-    // this kernel's lanes idle too.  The lines lie between the sizes measured
-    // on either side, us, this kernel / the best waves or rows (steps per
-    // million filled cells).  Plain: 302 x 278 x 256 59.6 / 64.1 (1.12), 240^3
-    // 42.8 / 45.1 (1.331), but 640 x 300 x 140 117 / 102 (1.348), 192^3
-    // 24.8 / 23.6 (1.71).  Imaging: 640 x 300 x 140 189 / 201 (1.348), but 200 x
-    // 180 x 300 72 / 67 (1.47); odd rows 301 x 277 x 259 153 / 169 (1.255), but
-    // 400 x 260 x 161 125 / 120 (1.326).
-    const double fill = std::sqrt((double)((g.nz + 127) / 128 * 128) / g.nz);
-    const double line = (!fuse ? 1.335e-6 : (g.nz & 1) ? 1.32e-6 : 1.4e-6) * fill;
+    // A plane step of every block takes 2.3-2.7 us (plain), 2.5-2.8 (upper taper
+    // on the output), 2.7-2.9 (taper3D on the output) or 3.8-5 (imaging), what
+    // its lanes do not fill included; the waves take 3.0-3.3 us per million
+    // cells while the loop's arrays stay in the Infinity Cache (256 MB; the line
+    // is at 360), 3.4-3.9 beyond, and full rows or waves with imaging 5.5-7.  So
+    // the kernel serves a step below a number of plane steps per million cells,
+    // us on either side of it, this kernel / the best other (plane steps per
+    // million cells):
+    //   plain: 302 x 278 x 256 61.9 / 64.6 (1.12), but 240 x 200 x 400 67.7 / 58.5
+    //     (1.46), 350 x 350 x 160 78.3 / 62.3 (1.68); odd rows, whose stores are
+    //     cacheable, 400 x 260 x 161 53.3 / 56.1 (1.67); past the cache 448 x 448 x
+    //     300 199 / 222 (1.33), but 592 x 592 x 161 217 / 213 (1.60); between the
+    //     receiver steps of a backward loop, 6 arrays, both steps together 250 x
+    //     250 x 300 168 / 174 (1.44);
+    //   upper taper: 330 x 330 x 256 78.4 / 90.5 (1.04), but 280 x 280 x 256 64.7 /
+    //     61.8 (1.15); odd 301 x 277 x 259 69.3 / 73.3 (1.53), 400 x 260 x 161 57.9 /
+    //     58.0 (1.67); past the cache 448 x 448 x 300 207 / 222 (1.33), but 592 x
+    //     592 x 161 232 / 215;
+    //   taper3D: 330 x 330 x 256 81.9 / 91.5, but 302 x 278 x 256 67.6 / 64.9; odd
+    //     301 x 277 x 255 56.5 / 65.3 (1.13), but 301 x 277 x 259 74.9 / 71.0; past the
+    //     cache 528 x 528 x 400 396 / 418 (1.22), but 336 x 336 x 400 170 / 168 (1.35);
+    //     beside the frequency accumulators, both fields and those together, 301 x
+    //     277 x 259 413 / 424, 240 x 200 x 300 234 / 239 (1.46);
+    //   imaging: 300 x 300 x 180 89.5 / 97.1 (1.60), 592 x 592 x 161 345 / 362 (1.60),
+    //     but 640 x 300 x 140 195 / 184 (1.82), 592 x 592 x 150 341 / 336 (1.71).
+    const double cells = 1e-6 * g.nx * g.ny * g.nz;
+    const bool cached = cells * arrays < 90.0, odd = g.nz & 1;
+    double line;
+    if (fuse) line = 1.65;
+    else if (!taper || taper->b <= 0) line = !cached ? 1.5 : odd ? 1.7 : 1.2;
+    else if (taper->all == 3) line = !cached ? 1.45 : odd ? 1.6 : 1.13;
+    else line = arrays > 6 ? 1.55 : !cached ? 1.3 : odd ? 1.35 : 1.08;
     const int nyt = y_tiles(g);
     const March m = choose_march(nyt, g.nx - 8);
-    if ((double)m.steps >= line * (double)g.nx * g.ny * g.nz) return none;
+    if ((double)m.steps >= line * cells) return none;
     return SlabGrid{nyt, (g.nx - 8 + m.chunk - 1) / m.chunk, m.chunk};
 }
 

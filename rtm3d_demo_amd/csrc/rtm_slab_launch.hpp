@@ -31,8 +31,11 @@ constexpr int y_waves(int nzw) { return 12 / nzw; }
 
 // The step (radius 4, FP32) that the full-row kernel serves: no taper, taper3D
 // or the upper taper on the output, imaging without a taper or with the upper
-// taper on the output.  launch_slab takes the plan of the same step.
-slab::SlabGrid slab_plan(int radius, const Grid &g, const ImageFuse *fuse, const TaperFuse *taper);
+// taper on the output.  arrays: how many of the grid's size the loop touches from
+// one such step to the next (P, PP and V alone: 3).  launch_slab takes the plan
+// of the same step.
+slab::SlabGrid slab_plan(int radius, const Grid &g, const ImageFuse *fuse, const TaperFuse *taper,
+                         int arrays = 3);
 hipError_t launch_slab(const slab::SlabGrid &plan, const float *P, float *PP, const float *V,
                        const Coefs &cf, const Grid &g, const ImageFuse *fuse,
                        const TaperFuse *taper, int *flag, hipStream_t s);

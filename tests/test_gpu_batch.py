@@ -24,7 +24,7 @@ SHOTS = [
 ]
 # one grid that the FP32 full-row step serves (test_launch_limits.py checks it)
 # and two that it does not
-MIXED = [SHOTS[0], ((104, 500, 384), (52, 250, B + 2), (1, 2, 3, 3, 4, 7, 6)), SHOTS[1]]
+MIXED = [SHOTS[0], ((136, 503, 500), (68, 250, B + 2), (1, 2, 3, 3, 4, 7, 6)), SHOTS[1]]
 
 
 def _wave(rng, shape, fmt):

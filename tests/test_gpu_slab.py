@@ -4,7 +4,8 @@ on dense random states against the oracle's operators in the reference's
 order, bit for bit, at the edges of the kernel's range -- rows of two to four
 128-cell waves, odd and even, just past and just at a wave; last blocks of
 one row and of every row; odd and even borders.  test_launch_limits.py checks
-that every shape here is one that the kernel takes.
+that every shape here takes the kernel for the plain and the imaging step, and
+the tapered forms for each number of waves, odd and even.
 """
 import pytest
 
@@ -23,6 +24,12 @@ SHAPES = [
     ((104, 503, 500), 40),  # four waves; whole blocks
     ((104, 504, 509), 12),
     ((104, 500, 512), 9),
+    # grids past the Infinity Cache, where even rows take the tapered forms too
+    ((200, 603, 250), 13),
+    ((152, 592, 336), 40),
+    ((160, 585, 384), 15),  # last block of one row
+    ((136, 503, 500), 10),
+    ((130, 500, 512), 33),
 ]
 
 
@@ -45,12 +52,12 @@ def test_short_migration_window(gpu, oracle, shape, blen, n):
 
 
 # taper3D on the output with and without the older field's taper
-@pytest.mark.parametrize("shape,blen", [SHAPES[0], SHAPES[1], SHAPES[5], SHAPES[8]])
+@pytest.mark.parametrize("shape,blen", [SHAPES[1], SHAPES[5], SHAPES[10], SHAPES[13]])
 def test_frequency_window(gpu, oracle, shape, blen):
     windows.frequency(gpu, oracle, windows.setup(oracle, shape, blen, 5))
 
 
 # the upper taper on the output of the whole border
-@pytest.mark.parametrize("shape,blen", [SHAPES[0], SHAPES[1], SHAPES[4], SHAPES[7]])
+@pytest.mark.parametrize("shape,blen", [SHAPES[1], SHAPES[4], SHAPES[10], SHAPES[14]])
 def test_snapshot_window(gpu, oracle, shape, blen):
     windows.snapshots(gpu, oracle, windows.setup(oracle, shape, blen, 6))

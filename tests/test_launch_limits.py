@@ -48,7 +48,8 @@ int main(int argc, char **argv)
     if (!strcmp(argv[1], "full-row")) {  // R: the stencil radius, taps: the taper's form
         const ImageFuse fz{};
         const TaperFuse tf{p, b, 1, taps, 0};
-        printf("%d\n", slab_plan(R, g, arg(8) ? &fz : nullptr, taps ? &tf : nullptr).nyt);
+        printf("%d\n",
+               slab_plan(R, g, arg(8) ? &fz : nullptr, taps ? &tf : nullptr, arg(9)).nyt);
         return 0;
     }
     hipError_t e;
@@ -130,17 +131,43 @@ def test_parts_that_fit_by_themselves(program, args, refused):
     ((301, 277, 259), 21, 4, 0, 1, True),
     ((192, 192, 192), 24, 4, 0, 0, False),
     ((40, 44, 90), 12, 4, 0, 0, False),
+    # either side of the lines: the other kernels were faster on the second
+    ((302, 278, 256), 20, 4, 0, 0, True),
+    ((240, 200, 400), 20, 4, 0, 0, False),
+    ((400, 260, 161), 20, 4, 0, 0, True),
+    ((350, 350, 160), 20, 4, 0, 0, False),
+    ((448, 448, 300), 20, 4, 0, 0, True),
+    ((592, 592, 161), 20, 4, 0, 0, False),
+    ((330, 330, 256), 20, 4, 3, 0, True),
+    ((280, 280, 256), 20, 4, 3, 0, False),
+    ((330, 330, 256), 20, 4, 2, 0, True),
+    ((302, 278, 256), 20, 4, 2, 0, False),
+    ((528, 528, 400), 20, 4, 2, 0, True),
+    ((336, 336, 400), 20, 4, 2, 0, False),
+    ((300, 300, 180), 20, 4, 3, 1, True),
+    ((640, 300, 140), 20, 4, 3, 1, False),
 ])
 def test_full_row_steps(program, grid, b, radius, taper, image, served):
-    assert (_result(program, "full-row", *grid, b, radius, taper, image) > 0) == served
+    assert (_result(program, "full-row", *grid, b, radius, taper, image, 3) > 0) == served
+
+
+# a grid whose forward loop stays in the cache and whose backward loop does not
+@pytest.mark.parametrize("arrays, served", [(3, False), (6, True)])
+def test_full_row_steps_count_the_loops_arrays(program, arrays, served):
+    assert (_result(program, "full-row", 250, 250, 300, 20, 4, 0, 0, arrays) > 0) == served
 
 
 @pytest.mark.parametrize("taper, image", [(0, 0), (2, 0), (3, 0), (0, 1), (3, 1)])
 def test_windows_of_the_full_row_kernel_run_it(program, taper, image):
     """The grids of test_gpu_slab.py, and of the mixed batch, lie where those
     tests say."""
+    rows = set()
     for grid, b in test_gpu_slab.SHAPES:
-        assert _result(program, "full-row", *grid, b, 4, taper, image) > 0, grid
-    served = [_result(program, "full-row", *shot[0], test_gpu_batch.B, 4, taper, image) > 0
+        taken = _result(program, "full-row", *grid, b, 4, taper, image, 3) > 0
+        assert taken or (taper and not image), grid
+        if taken:
+            rows.add((-(-grid[2] // 128), grid[2] % 2))
+    assert rows == {(waves, odd) for waves in (2, 3, 4) for odd in (0, 1)}
+    served = [_result(program, "full-row", *shot[0], test_gpu_batch.B, 4, taper, image, 3) > 0
               for shot in test_gpu_batch.MIXED]
     assert served == [False, True, False]
