@@ -489,21 +489,26 @@ int rtmhip_get_tiling(int kernel_class, int *tz, int *by, int *ry, int *xchunk);
  * HBC upper tapers (taperUpper3D of both fields before each step,
  * RTMFiniteDifferencesKernel_HBC.cpp:160-165 and :311-316) in the single-shot
  * loops (rtmhip_forward_steps, rtmhip_backward_steps with fused = 1,
- * rtmhip_snap_*): mode 1 fuses them into the stencil (tapered on load);
- * mode 0 runs them as one in-place pass over both fields' upper slabs
- * followed by the untapered stencil; mode 4 applies the forward loops' tapers
- * to each step's output (the step stores the tapered value its successor
- * reads as P and tapers only the centre PP; used when the source lies at
- * z >= blen) and fuses the backward loops' on load.
+ * rtmhip_snap_*) and in batches: mode 1 fuses them into the stencil (tapered
+ * on load); mode 0 runs them as one in-place pass over both fields' upper
+ * slabs followed by the untapered stencil; mode 4 applies them to each step's
+ * output (the step stores the tapered value its successor reads as P and
+ * tapers only the centre PP) in the forward loops (stencil order 8, the source
+ * at z >= blen), in the snapshot loops' receiver steps, and for F32 in the
+ * receiver step with imaging where the full-row kernel runs it (no tile shape
+ * set, rows of 129 to 512 cells on grids large enough for it); the other steps
+ * taper on load.
  * Every-border tapers of rtmhip_model_steps (taper3D of both fields before
  * each step, RTMFiniteDifferencesKernel.cpp:180-181; stencil order 8): on
  * each step's output with modes 3 and 4 (used when the source and receivers
  * lie off the borders, else the separate pass runs), fused on load with
  * mode 2 (upper tapers as mode 1), one in-place pass with modes 0 and 1.
  * Mode -1 restores the default: mode 4 for F32; for F16 and BF16 as mode 4
- * where nze is even, with upper tapers in separate passes in the HBC backward
- * loop and where nze is odd.
- * Batches and fused = 2 always fuse the upper tapers on load.
+ * where nze is even and, in rtmhip_forward_steps, blen >= 8, with upper tapers
+ * in separate passes in the HBC backward loop and otherwise.
+ * Batches take the output form when every shot of the batch does and each
+ * step is one launch per shot, else (and with mode 0) they taper on load;
+ * fused = 2 always tapers on load.
  * rtmhip_get_taper_fusion returns the last mode set (-1 for the default). */
 int rtmhip_set_taper_fusion(int wave_format, int mode);
 int rtmhip_get_taper_fusion(int wave_format, int *fused);

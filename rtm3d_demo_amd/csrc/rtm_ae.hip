@@ -13,9 +13,10 @@
 //   L3  transposed L2, 32 -> 8, tanh           [64 rows x 32]   * [32 x 512]
 //   L4  transposed L1, 8 -> 1                  [4096 rows x 8]  * [8 x 8]
 // so one brick of 32768 FP16 values (64 KB) becomes 2048 FP16 codes (4 KB)
-// plus its scale.  The GEMMs run on the matrix cores (MFMA 16x16x32, FP16
-// operands, FP32 accumulation) for inference and for training (forward,
-// backward, split-K weight gradients).
+// plus its scale.  The products run on the matrix cores (FP16 operands, FP32
+// accumulation): inference as one launch per direction with every layer in
+// registers, a training step as one launch for the gradient (each block's
+// partial sums in a slab of its own) and one that adds the slabs and updates.
 #include "rtm_internal.hpp"
 
 #include <algorithm>

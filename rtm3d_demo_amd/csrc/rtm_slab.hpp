@@ -2,7 +2,8 @@
 // lane.  Included by the translation units that instantiate it (even and odd
 // row lengths).  Arithmetic, fusions and rounding are those of the kernels in
 // rtm_stencil.hip (rtm-3d/src/platform/host/RTMCPUPlatform.cpp:325-395,
-// :513-540, :566-657, :710-920), so results are bit-identical to them.
+// :513-540, :566-657, :710-920), so results are bit-identical to them but for
+// the sign of a zero after an underflow.
 //
 // What bounds it: the bytes that miss the XCD's L2.  A wave that marches its
 // own 4-row tile (k_stencil_wave2) re-reads its 8 halo rows from beyond L2,
@@ -19,17 +20,17 @@
 //   * the next plane is staged into LDS during this plane's arithmetic (its
 //     centre rows have been in the ring for R planes): one barrier per plane,
 //     with nothing to wait for behind it.
-// That is 17.0 bytes per cell (FETCH_SIZE + WRITE_SIZE).  Salt grid, 592 x 592
-// x 336, ms, against the best wave or row shape: plain 0.348 (0.417), upper
-// taper on the output 0.351 (0.431), taper3D on the output 0.365 (0.474),
-// imaging 0.595, with the upper taper 0.605 (0.714); 5.1 TB/s of algorithmic
+// That is 17.2 bytes per cell (FETCH_SIZE + WRITE_SIZE).  Salt grid, 592 x 592
+// x 336, ms, against the best wave or row shape: plain 0.355 (0.417), upper
+// taper on the output 0.353 (0.431), taper3D on the output 0.368 (0.474),
+// imaging with the upper taper 0.622 (0.714); 5.0 TB/s of algorithmic
 // bytes for the plain step.  With branches around the loads and stores (see
-// bounded_view) these were 0.373, 0.381, 0.404 and 0.605.  Halos loaded a
+// bounded_view) the first three were 0.373, 0.381 and 0.404.  Halos loaded a
 // plane ahead instead of with the lead: 18.8 bytes per cell, 4 % slower;
 // cacheable streams: plain 2 %, imaging 6 % slower.  The x ring's 60 registers
 // and the 20 of the waiting halo rows set 3 rows per wave (4 rows spill),
 // 12 waves per CU.  It is then bound by the 5 to 6 TB/s beyond L2 and nearly as
-// much by the VALU (57 % of its issue slots).
+// much by the VALU (55 % of its issue slots; imaging 37 %).
 #pragma once
 #include "rtm_internal.hpp"
 #include "rtm_slab_launch.hpp"
@@ -347,8 +348,8 @@ __global__ void __launch_bounds__(64 * NZW *NYW, 1)
                                             : (ry >= RY ? yn[R + ry - RY][a] : q[ctr][ry][a]);
                     const float vz = (io == R) ? p : w[io + a];
                     if (io == 0) {
-                        // 0 + v*c in one instruction: the product's rounding
-                        // is the only one, and -0 becomes +0 as in the sum
+                        // 0 + v*c in one instruction (the same number; only
+                        // a negative product that underflows gives -0 here)
                         ax = __builtin_fmaf(vx, cf.c[0][io], 0.f);
                         ay = __builtin_fmaf(vy, cf.c[1][io], 0.f);
                         az = __builtin_fmaf(vz, cf.c[2][io], 0.f);

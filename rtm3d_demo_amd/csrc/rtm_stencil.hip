@@ -946,7 +946,7 @@ __device__ __forceinline__ void wave_tile(const T *__restrict__ P, T *__restrict
                 const float vz = (io == R) ? p : t[io - R];
                 const float vx = q[(K + io) % NR][r];
                 if (io == 0) {
-                    // 0 + v*c: one rounding, and -0 becomes +0 as in the sum
+                    // 0 + v*c (a negative product that underflows: -0)
                     ax = __builtin_fmaf(vx, cf.c[0][io], 0.f);
                     ay = __builtin_fmaf(vy, cf.c[1][io], 0.f);
                     az = __builtin_fmaf(vz, cf.c[2][io], 0.f);
@@ -1338,7 +1338,7 @@ __device__ __forceinline__ void wave_tile2(const T *__restrict__ P, T *__restric
                     const float vz = (io == R) ? p : w[io + a];
                     const float vx = q[(K + io) % NR][r][a];
                     if (io == 0) {
-                        // 0 + v*c: one rounding, and -0 becomes +0 as in the sum
+                        // 0 + v*c (a negative product that underflows: -0)
                         ax = __builtin_fmaf(vx, cf.c[0][io], 0.f);
                         ay = __builtin_fmaf(vy, cf.c[1][io], 0.f);
                         az = __builtin_fmaf(vz, cf.c[2][io], 0.f);

@@ -473,11 +473,13 @@ def set_taper_fusion(fmt, mode):
     """mode 1: upper tapers fused into the stencil; 2: also the modeling
     loop's every-border tapers, applied as values are loaded; 3: those
     applied to each step's output instead (needs the source and receivers
-    off the borders, else the separate pass runs); 4: also the forward
-    loops' upper tapers applied to each step's output (backward loops fused
-    on load); 0: separate in-place passes; -1: the format's default (F32:
-    mode 4; 16-bit formats: as mode 4, but the HBC backward loop and odd
-    rows in separate passes)."""
+    off the borders, else the separate pass runs); 4: also the upper tapers
+    of the forward loops, of the snapshot receiver steps and (F32, where the
+    full-row kernel runs it) of the receiver step with imaging applied to each
+    step's output, the others on load; 0: separate in-place passes; -1: the
+    format's default (F32: mode 4; 16-bit formats: as mode 4, but the HBC
+    backward loop, odd rows and forward borders below 8 in separate
+    passes)."""
     check(load().rtmhip_set_taper_fusion(WAVE_FORMATS[fmt][0], mode))
 
 

@@ -19,7 +19,7 @@ Fields hold random values; counters do not depend on them.
 turns the counter_collection.csv files of a FETCH_SIZE pass and a WRITE_SIZE
 pass into per-kernel bytes per dispatch.  Each counter is scaled by what it
 reads for k_stack, whose true traffic is known (8 B read + 4 B written per
-cell), and the first kernel of each stencil class is printed as
+cell), and the most launched kernel of each stencil class is printed as
 "traffic_bytes_per_launch[class C, tile T]: N", the lines bench.py reads (0
 plain, 1 fused receiver, 2 tapered forward, 3 dual backward; T the class's
 tile shape TZxBYxRY, or "default").
@@ -31,7 +31,8 @@ the shapes.
 --wave-format f16 (or bf16) runs the 16-bit sequence instead: k_stack, then
 5 HBC forward steps, 7 fused backward steps (mode 1) and 5 + 5 snapshot-RTM
 steps (16-bit snapshots) with 16-bit wavefields and the library's defaults
-(separate upper-taper pass, two-z waves).  Its summary (--summarize with the
+(two-z waves; the upper taper on the forward steps' output, in a pass of its
+own before the receiver steps).  Its summary (--summarize with the
 same option) gives per-kernel bytes and the 16-bit algorithmic bytes per
 updated cell: 10 for a step (V stays FP32), 20 for the imaging step.
 """
@@ -99,7 +100,8 @@ def _short(name):
         if m:
             return "%s<%s>" % (m.group(1), ", ".join(_demangle_args(m.group(2))))
         return name
-    name = name.replace("rtmhip::(anonymous namespace)::", "").replace("void ", "")
+    for prefix in ("rtmhip::(anonymous namespace)::", "rtmhip::slab::", "void "):
+        name = name.replace(prefix, "")
     return name.split("(")[0]
 
 
@@ -131,7 +133,7 @@ def summarize(fetch_dir, write_dir, tilings=None, wave_format="f32"):
     print()
     print("| kernel | dispatches | read MB | write MB | total MB | B per updated cell |")
     print("|---|---|---|---|---|---|")
-    first = {}
+    most = {}
     for name in sorted(fetch, key=lambda k: -fetch[k][0]):
         if name not in write:
             continue
@@ -143,26 +145,28 @@ def summarize(fetch_dir, write_dir, tilings=None, wave_format="f32"):
         cls = None
         if short.startswith("k_stencil_dual"):
             cls = 3
-        elif short.startswith("k_stencil"):
-            tail = short.rsplit(",", 2)[-2:]  # the IMG and TAPER arguments
+        elif short.startswith(("k_stencil", "k_slab")):
+            # the IMG and TAPER arguments, k_slab's before the last
+            tail = short.split(",")[-3:-1] if short.startswith("k_slab") else \
+                short.split(",")[-2:]
             img, tap = (t.strip(" >") not in ("false", "0") for t in tail)
             cls = 1 if img else (2 if tap else 0)
-        if cls is not None and cls not in first:
-            first[cls] = (short, r + w)
+        if cls is not None and fetch[name][1] > most.get(cls, (0,))[0]:
+            most[cls] = (fetch[name][1], short, r + w)
     print()
     if wave_format != "f32":
         # 16-bit wavefields: P, PP read, PP written (2 B each), V (4 B); the
         # imaging step adds PS (2 B) and the FP32 image read and written
-        for cls in sorted(first):
-            short, t = first[cls]
+        for cls in sorted(most):
+            _, short, t = most[cls]
             bpc = 20.0 if cls == 1 else 10.0
             print("%s class %d (%s): algorithmic %.0f B per launch (%.0f B x %d cells), "
                   "traffic %.0f B (%.2f x)" % (wave_format, cls, short, bpc * interior, bpc,
                                                interior, t, t / (bpc * interior)))
         return
     algo = {0: 16.0, 1: 28.0, 2: 16.0, 3: 36.0}
-    for cls in sorted(first):
-        short, t = first[cls]
+    for cls in sorted(most):
+        _, short, t = most[cls]
         print("class %d (%s): algorithmic %.0f B per launch (%.0f B x %d updated cells)"
               % (cls, short, algo[cls] * interior, algo[cls], interior))
         tile = "%dx%dx%d" % tilings[cls] if cls in tilings else "default"
